@@ -1547,8 +1547,8 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
 #define ATLAS_EDGE_NODES 0u
 #endif
 #define ATLAS_EDGE_CNT_WORDS (ATLAS_BLOCK + ATLAS_BLOCK / 64u + 4u)
-// target j's count word: one pad word per 64, so the scanning wave's lanes (64 consecutive counts
-// each) read and write 64 different LDS banks at every step
+// target j's count word: one pad word per 64, so with 4096-neuron blocks the scanning wave's lanes
+// (64 consecutive counts each) read and write 64 different LDS banks at every step
 __device__ __forceinline__ u32 edge_at(u32 j) { return j + (j >> 6); }
 #define ATLAS_EDGE_BUCKET_MAX 64u   // events of one target and tick beyond which the tick is replayed
 
@@ -1598,18 +1598,19 @@ __device__ __forceinline__ void lds_wait_at_least(u32* counter, u32 target, bool
 }
 
 // One wave turns the block's ATLAS_BLOCK event counts into bucket starts (exclusive scan, in
-// place): 64 consecutive counts per lane, then a scan of the lanes' sums.  Returns the total;
-// `largest` receives the largest count.
+// place): ATLAS_BLOCK / 64 consecutive counts per lane, then a scan of the lanes' sums.  Returns the
+// total; `largest` receives the largest count.
 __device__ __forceinline__ u32 edge_scan(u32* cnt, u32& largest) {
-    static_assert(ATLAS_BLOCK % 64 == 0, "64 counts per lane");
+    static_assert(ATLAS_BLOCK % 64 == 0, "whole counts per lane");
     constexpr u32 PER = ATLAS_BLOCK / 64;
     const u32 lane = __lane_id();
-    u32* mine = cnt + lane * (PER + 1u);
+    const u32 mine = lane * PER;   // its first target
     u32 sum = 0, big = 0;
 #pragma unroll 16
     for (u32 i = 0; i < PER; ++i) {
-        sum += mine[i];
-        big = mine[i] > big ? mine[i] : big;
+        const u32 c = cnt[edge_at(mine + i)];
+        sum += c;
+        big = c > big ? c : big;
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -1627,8 +1628,8 @@ __device__ __forceinline__ u32 edge_scan(u32* cnt, u32& largest) {
     u32 run = x - sum;
 #pragma unroll 16
     for (u32 i = 0; i < PER; ++i) {
-        const u32 c = mine[i];
-        mine[i] = run;
+        const u32 c = cnt[edge_at(mine + i)];
+        cnt[edge_at(mine + i)] = run;
         run += c;
     }
     return total;

@@ -221,3 +221,22 @@ def test_weighted_full_size_split_loop_equals_per_tick(monkeypatch):
     assert len(result["populations"][0]["spike_ticks"]) > 10_000
     tick_dump, tick_events, _ = run(doc, "per-tick", monkeypatch, lift_recording_budget=True, verify_envelope=False)
     assert tick_dump == dump and tick_events == events
+
+
+@pytest.mark.parametrize("edge_weights,delay", [(False, 1), (False, 0), (True, 1)])
+@pytest.mark.parametrize("indegree", [200, 260, 1100])
+def test_segments_longer_than_a_slot_equal_oracle_and_per_tick(monkeypatch, indegree, edge_weights, delay):
+    """4,200 neurons in 17 blocks of 256: (source, block) segments of 12, 16 and 65 targets on average, so
+    lengths on both sides of a slot's inline targets (15, or 12 with a weight per synapse) and of a
+    wave's 64 lanes, which share a longer segment's edges.  The persistent launches (the split loop
+    at delay 1, by counters or edge buckets) and one launch per tick equal the oracle."""
+    print(f"case: long segments, in-degree {indegree}, weights {edge_weights}, delay {delay}", flush=True)
+    doc = models.cuba_network(4200, indegree=indegree, delay_ticks=delay, steps=400, weight_scale=11.6 / indegree,
+                              edge_weights=edge_weights)
+    expected = oracle.run(doc, lift_recording_budget=True)
+    assert expected.synaptic_events > 50_000
+    dump, events, _ = run(doc, "persistent", monkeypatch, lift_recording_budget=True,
+                          shape=engine.Shape(256, 256, 4, 10))
+    assert dump == expected.results and events == expected.events
+    tick_dump, tick_events, _ = run(doc, "per-tick", monkeypatch, lift_recording_budget=True)
+    assert tick_dump == dump and tick_events == events
