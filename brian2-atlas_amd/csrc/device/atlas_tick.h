@@ -701,7 +701,7 @@ __device__ void apply_counts(const u64* __restrict__ tab, i64 tick, double t, u3
 // Counting through the slot table (SLOTS groups): one 32-byte load per (fired source,
 // pathway) gives the count of the segment (word 0) and, for up to 15 targets, its
 // block-local targets (words 1..15), so counting needs no row-table round trip; a
-// longer segment's targets are read from the row table (count_long_slot).  Only valid
+// longer segment's targets are read from the row table (count_long_slots).  Only valid
 // slots are fetched (exec-masked loads, issued back to back).
 template <class Group>
 __device__ __forceinline__ void load_slots(const u64* __restrict__ tab, u32 blk, const u64* at, const bool* ok,
@@ -720,12 +720,36 @@ __device__ __forceinline__ void load_slots(const u64* __restrict__ tab, u32 blk,
     }
 }
 
-// The targets of a slot whose segment is longer than its 15 inline words (word 0 the count,
-// u32 word 1 the segment's first row), read from the pathway's row table and counted.
+// The edges of the segments longer than their slots' inline words (is_long: this lane's slot holds
+// such a segment, of n edges of pathway p from row0): each segment's edges are spread over the
+// wave's lanes, each(pathway, row) per edge, so a segment costs one memory round trip for its row
+// table instead of one per edge of a single lane.  A chip's tick waits for its slowest workgroup:
+// with one lane per segment, at in-degree 1000 and 4096-neuron blocks, the 1M-neuron network (7
+// such segments in a million slots, about one per tick over the chip) took 5.85 us per
+// tick against 5.21, the one of 300,000 neurons (13.5 edges per segment on average)
+// 14.7 against 9.7.  Every lane of the wave calls it.
+template <class Each>
+__device__ __forceinline__ void long_segments(bool is_long, u32 p, u32 n, u32 row0, const Each& each) {
+    u64 m = __ballot(is_long);
+    while (m) {
+        const u32 src = (u32)__builtin_ctzll(m);
+        m &= m - 1ull;
+        const u32 edges = __builtin_amdgcn_readlane(n, src);
+        const u32 first = __builtin_amdgcn_readlane(row0, src);
+        const u32 path = __builtin_amdgcn_readlane(p, src);
+        for (u32 r = __lane_id(); r < edges; r += 64) each(path, first + r);
+    }
+}
+
+// The targets of the slots whose segments are longer than their 15 inline words (word 0 the count,
+// u32 word 1 the segment's first row), read from the pathway's row table and counted; hist is the
+// first pathway's counters.
 template <class Group>
-__device__ __forceinline__ void count_long_slot(const u64* __restrict__ tab, u32 p, u32 n, u32 row0, u32 blk,
-                                                u32* hist) {
-    for (u32 r = 0; r < n; ++r) atomicAdd(&hist[Group::row_target(tab, p, row0 + r) - blk * ATLAS_BLOCK], 1u);
+__device__ __forceinline__ void count_long_slots(const u64* __restrict__ tab, bool is_long, u32 p, u32 n, u32 row0,
+                                                 u32 blk, u32* hist) {
+    long_segments(is_long, p, n, row0, [&](u32 path, u32 row) {
+        atomicAdd(&hist[path * ATLAS_BLOCK + Group::row_target(tab, path, row) - blk * ATLAS_BLOCK], 1u);
+    });
 }
 
 template <class Group>
@@ -750,7 +774,7 @@ __device__ __forceinline__ void count_slots(const u64* __restrict__ tab, u32 blk
             if (!__ballot(r < inline_n)) break;
             if (r < inline_n) atomicAdd(&hist[(w[(r + 1) / 2] >> (16u * ((r + 1) % 2))) & 0xFFFFu], 1u);
         }
-        if (__ballot(n > 15u) && n > 15u) count_long_slot<Group>(tab, p, n, w[1], blk, hist);
+        count_long_slots<Group>(tab, n > 15u, p < Group::NP ? p : 0u, n, w[1], blk, &s.hist[HB]);
     }
     // delivered-event counters: wavefront reduction, one LDS atomic per wave
 #pragma unroll
@@ -1360,7 +1384,7 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
                     if (r < inline_cnt) atomicAdd(&hist[(w[(r + 1) / 2] >> (16u * ((r + 1) % 2))) & 0xFFFFu], 1u);
                 }
                 // a segment longer than the slot's 15 inline targets: read from the row table
-                if (__ballot(cnt > 15u) && cnt > 15u) count_long_slot<Group>(tab, pq[q], cnt, w[1], blk, hist);
+                count_long_slots<Group>(tab, cnt > 15u, pq[q], cnt, w[1], blk, &s.hist[HB]);
             }
         };
         if constexpr (!SAME_TICK) {
@@ -2001,7 +2025,7 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
                                 if (!__ballot(r < inline_cnt)) break;
                                 if (r < inline_cnt) atomicAdd(&h[(w[(r + 1) / 2] >> (16u * ((r + 1) % 2))) & 0xFFFFu], 1u);
                             }
-                            if (__ballot(c > 15u) && c > 15u) count_long_slot<Group>(tab, pq, c, w[1], blk, h);
+                            count_long_slots<Group>(tab, c > 15u, pq, c, w[1], blk, hist);
                         });
 #pragma unroll
                     for (u32 p = 0; p < NP; ++p) lane_delivered[p] += per_path[p];
@@ -2032,9 +2056,9 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
                                 if (!__ballot(r < inline_cnt)) break;
                                 if (r < inline_cnt) atomicAdd(&cnt[edge_at((w[(r + 4) / 2] >> (16u * (r % 2))) & 0xFFFFu)], 1u);
                             }
-                            if (__ballot(c > 12u) && c > 12u)
-                                for (u32 r = 0; r < c; ++r)
-                                    atomicAdd(&cnt[edge_at(Group::row_target(tab, pq, w[1] + r) - blk * ATLAS_BLOCK)], 1u);
+                            long_segments(c > 12u, pq, c, w[1], [&](u32 p, u32 row) {
+                                atomicAdd(&cnt[edge_at(Group::row_target(tab, p, row) - blk * ATLAS_BLOCK)], 1u);
+                            });
                         });
 #pragma unroll
                     for (u32 p = 0; p < NP; ++p) lane_delivered[p] += per_path[p];
@@ -2076,9 +2100,9 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
                                 if (!__ballot(r < inline_cnt)) break;
                                 if (r < inline_cnt) place((w[(r + 4) / 2] >> (16u * (r % 2))) & 0xFFFFu, pp, w[1] + r);
                             }
-                            if (__ballot(c > 12u) && c > 12u)
-                                for (u32 r = 0; r < c; ++r)
-                                    place(Group::row_target(tab, pp, w[1] + r) - blk * ATLAS_BLOCK, pp, w[1] + r);
+                            long_segments(c > 12u, pp, c, w[1], [&](u32 p, u32 row) {
+                                place(Group::row_target(tab, p, row) - blk * ATLAS_BLOCK, p, row);
+                            });
                         });
                 }
                 __builtin_amdgcn_s_setprio(0);
