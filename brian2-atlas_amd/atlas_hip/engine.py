@@ -44,6 +44,7 @@ EDGE_KEY_BITS = 30          # edge id bits of an edge-keyed event (atlas_tick.h 
 LDS_BYTES = 160 * 1024      # LDS per CU (one workgroup of the split loop per CU)
 ATLAS_XLIST = 512           # fired sources one exchange wave of the split loop keeps (atlas_tick.h)
 EDGE_XLIST = 256            # the same with edge buckets (config 3 lists about 111 per wave and tick)
+RING_SLOTS = 64             # ring ticks a persistent launch keeps its counts of (atlas_tick.h ATLAS_RING_PREV)
 RESIDENT_BLOCKS = 512       # 512-wide workgroups resident at once: two per CU on 256 CUs
 CUS = 256             # compute units
 PATH_MAX_SOURCE_BLOCKS = 8192
@@ -2581,6 +2582,8 @@ def persistent_eligible(plan: Plan, groups: list, counting: list, split_loop: bo
     if not PERSISTENT_MIN_BLOCKS <= plan.total_blocks <= RESIDENT_BLOCKS * 512 // plan.shape.wg:
         return False
     if pop.count > 1 << 20:   # stamped ring words carry 20-bit neuron indices
+        return False
+    if pop.ring > RING_SLOTS:   # a delay of more than 31 ticks
         return False
     for k, group in enumerate(groups):
         delays = {d for path in group for d in path.dvals}

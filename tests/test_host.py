@@ -416,6 +416,15 @@ def test_persistent_eligibility():
     assert _generate(models.plastic_network(5000, steps=5, packed=False)).persistent is None
 
 
+@pytest.mark.parametrize("delay,persistent", [(31, True), (32, False), (50, False)])
+def test_long_delays_keep_one_launch_per_tick(delay, persistent):
+    """A persistent launch keeps the counts of 64 ring slots, 2 d + 2 ticks: delays of up to 31 ticks;
+    a longer one (here 3.2 and 5 ms) keeps one launch per tick, and its module compiles."""
+    plan = _generate(models.cuba_network(5000, indegree=20, delay_ticks=delay, steps=60))
+    assert (plan.persistent is not None) == persistent
+    assert len(rtc.compile_source(plan.source, engine.COMPILE_OPTIONS)) > 1000
+
+
 def test_weighted_network_runs_the_split_loop_through_edge_buckets():
     """An ordered group (a float32 weight per synapse, drawn from the edge id) of one delay >= 1 in
     4096-neuron blocks runs the split persistent loop through edge-keyed buckets: row slots (the
