@@ -642,6 +642,7 @@ class Plan:
     clocks: list = field(default_factory=list)       # (dt, start tick, steps) of each clock
     clock_buffer: int = -1
     edge_nodes: int = 0                              # events the split loop's edge buckets hold per workgroup and tick
+    min_blocks: int | None = None                    # fewest blocks of a persistent launch (PERSISTENT_MIN_BLOCKS)
 
     @property
     def multi_clock(self) -> bool:
@@ -2539,7 +2540,11 @@ def _edge_loop_candidate(plan: Plan) -> bool:
         return False
     groups = delivery_groups(plan)
     return (len(groups) == 1 and edge_group(plan, groups[0])
-            and PERSISTENT_MIN_BLOCKS <= plan.total_blocks)
+            and _min_blocks(plan) <= plan.total_blocks)
+
+
+def _min_blocks(plan: Plan) -> int:
+    return PERSISTENT_MIN_BLOCKS if plan.min_blocks is None else plan.min_blocks
 
 
 SLOT_TARGETS = 15   # targets held inline by one 32-byte slot (word 0 is the count)
@@ -2549,6 +2554,89 @@ SLOT_MAX_COUNT = 0xFFFF   # longer segments keep their first row in the slot, up
 def per_xcd(plan: "Plan") -> int:
     """Consecutive workgroup indices (blocks) per XCD: workgroup w runs on XCD w // per_xcd."""
     return (plan.total_blocks + XCDS - 1) // XCDS
+
+
+# Shapes of persistent launches, smallest block first, with the most blocks each takes: the split
+# loop reads at most 64 source blocks per exchange wave (one wave of 256 work-items, three of 512,
+# seven of 1024), and one workgroup runs per CU.  Measured on CUBA with a fixed in-degree of 1000,
+# delay 1, us per tick, the first shape that fits against the next two (and, before, the shape of
+# choose_shape): 20,000 neurons 3.4 / 3.4 / 4.7 (4.1), 100,000 3.3 / 6.9 / 7.4 (4.4), 200,000
+# 2.9 / 4.1 / 8.4 (4.5), 300,000 3.4 / 5.0 / 9.1 (9.1), 600,000 4.0 / 4.8 (4.8); with a weight per
+# synapse 100,000 9.9 / 15.0 / 16.3 (12.6, one launch per tick), 300,000 9.7 / 17.5 / 28.7 (28.7).
+# Fewer neurons and shorter slots per workgroup shorten both of its chains; more workgroups than
+# CUs make two of them share one.
+FITTED = ((Shape(256, 256, 4, 10), 64), (Shape(512, 512, 2, 10), 192), (Shape(1024, 1024, 1, 11), CUS),
+          (Shape(2048, 1024, 2, 11), CUS), (Shape(3072, 1024, 2, 11), CUS), (Shape(4096, 1024, 2, 11), CUS))
+
+
+# Operations of a neuron's tick (its update, threshold and run_regularly statements; OP_COST for the
+# long ones) above which the update bounds the tick and a network keeps its shape: the split loop
+# gives two or more neurons to each update work-item.  CUBA has 9; COBAHH (719) of 50,000 neurons,
+# delay 1, measured 13.1 us per tick in its FITTED shape against 9.0.
+HEAVY_OPS = 100
+OP_COST = {**dict.fromkeys(("exp", "expm1", "exprel", "log", "rand", "randn", "poisson", "binomial"), 40),
+           **dict.fromkeys(("div", "sqrt", "mod", "floordiv"), 10),
+           **dict.fromkeys(("load", "literal", "boolean", "integer", "f32_to_f64", "f64_to_f32"), 0)}
+
+
+def _update_ops(pop: PopulationPlan) -> int:
+    """Arithmetic operations of one neuron's tick, refractoriness and recording aside."""
+    def ops(value) -> int:
+        if isinstance(value, dict):
+            here = OP_COST.get(value["op"], 1) if "op" in value else 0
+            return here + sum(ops(v) for v in value.values())
+        return sum(ops(v) for v in value) if isinstance(value, list) else 0
+    codes = [code for code in (pop.update, pop.threshold) if code is not None] + [code for code, _ in pop.regular]
+    return sum(ops(code["vector"]) for code in codes)
+
+
+def fit_shape(plan: Plan) -> bool:
+    """Give a plan that can run persistent launches the shape they run fastest in (before
+    allocate()); whether the shape changed.  One population of at most 2^20 neurons whose single
+    delivery group persistent_eligible takes in some shape: with a delay >= 1 the first shape of
+    FITTED whose blocks it fits, at delay 0 (no split loop) or with a heavy update (HEAVY_OPS) the
+    shape it has, in both cases with no least number of blocks (a CUBA network of 500 neurons, 2
+    blocks: 3.2 us per tick persistent, 4.3 with one launch per tick)."""
+    if (plan.multi_clock or len(plan.populations) != 1 or plan.post_paths or plan.synapse_codes
+            or plan.populations[0].count > 1 << 20):
+        return False
+    groups = delivery_groups(plan)
+    if len(groups) != 1 or not _persistent_model(plan, groups[0]):
+        return False
+    pop, group = plan.populations[0], groups[0]
+    delay = group[0].dvals[0]
+    if not counting_group(group) and not (PERSISTENT_SPLIT and PERSISTENT_EDGES and edge_group(plan, group)):
+        return False
+    # the ring of a persistent launch (2 d + 2 ticks, one more with the split launches of delay 0)
+    ring = max(pop.ring, 2 * delay + 2 + (1 if plan.split else 0))
+    if ring > RING_SLOTS:
+        return False
+    shape = plan.shape
+    if delay >= 1 and PERSISTENT_SPLIT and not SPLIT_XWAVES and _update_ops(pop) <= HEAVY_OPS:
+        shape = next(shape for shape, most in FITTED if -(-pop.count // shape.block) <= most)
+    plan.min_blocks = 1
+    pop.ring = ring
+    changed = shape != plan.shape
+    plan.shape = shape
+    pop.blocks = plan.total_blocks = -(-pop.count // shape.block)
+    return changed
+
+
+def _persistent_model(plan: Plan, group: list[PathwayPlan]) -> bool:
+    """What persistent_eligible asks of the population and its delivery group whatever the shape."""
+    pop = plan.populations[0]
+    if pop.poisson_inputs or pop.generator is not None or pop.event_monitors or pop.custom_events:
+        return False
+    if any(where == "end" for _, where in pop.regular):   # run on the states in memory after the reset
+        return False
+    if pop.monitor_record and pop.monitor_vars:
+        return False
+    if not (pop.reset is None or _reset_fusable(plan, pop)):
+        return False
+    delays = {d for path in group for d in path.dvals}
+    if len(delays) != 1 or (min(delays) < 1) != plan.split:
+        return False
+    return not any(path.pending is not None or "\0not_refractory" in _touched_post(path)[0] for path in group)
 
 
 def persistent_eligible(plan: Plan, groups: list, counting: list, split_loop: bool = False) -> bool:
@@ -2571,27 +2659,18 @@ def persistent_eligible(plan: Plan, groups: list, counting: list, split_loop: bo
     # counted events applied in registers: after the update (delay >= 1), or, with delay 0, after
     # the tick's own exchange (the same Fused programs)
     edges = pop.fused_edges and split_loop
-    if not (pop.fused_split if plan.split else (pop.fused_counts or edges)) or not (pop.reset is None or pop.reset_fused):
+    if not (pop.fused_split if plan.split else (pop.fused_counts or edges)) or not _persistent_model(plan, groups[0]):
         return False
-    if pop.poisson_inputs or pop.generator is not None or pop.event_monitors or pop.custom_events:
-        return False
-    if any(where == "end" for _, where in pop.regular):   # run on the states in memory after the reset
-        return False
-    if pop.monitor_record and pop.monitor_vars:
-        return False
-    if not PERSISTENT_MIN_BLOCKS <= plan.total_blocks <= RESIDENT_BLOCKS * 512 // plan.shape.wg:
+    if not _min_blocks(plan) <= plan.total_blocks <= RESIDENT_BLOCKS * 512 // plan.shape.wg:
         return False
     if pop.count > 1 << 20:   # stamped ring words carry 20-bit neuron indices
         return False
     if pop.ring > RING_SLOTS:   # a delay of more than 31 ticks
         return False
     for k, group in enumerate(groups):
-        delays = {d for path in group for d in path.dvals}
-        if not (counting[k] or edges) or len(delays) != 1 or (min(delays) < 1) != plan.split or group[0].pending_ticks:
+        if not (counting[k] or edges) or group[0].pending_ticks:
             return False
         if not all("slot" in path.buffers and path.index not in plan.slot_fallback for path in group):
-            return False
-        if any(path.pending is not None for path in group):
             return False
     return True
 

@@ -74,6 +74,15 @@ class HipExecutor:
         started = time.perf_counter()
         self.plan = engine.lower(model, verify_envelope=verify_envelope, shape=shape)
         self.document = self.plan.document
+        # persistent launches (one cooperative launch for many ticks, states in registers) where the
+        # plan allows them; ATLAS_HIP_PERSISTENT=0 keeps one launch per tick, =plain issues them as
+        # ordinary launches once the kernel's occupancy shows the grid fits (for kernel tracers
+        # that cannot follow cooperative launches)
+        mode = os.environ.get("ATLAS_HIP_PERSISTENT", "1")
+        self.persistent = mode != "0"
+        self.plain_launches = mode == "plain"
+        if self.persistent and shape is None:
+            engine.fit_shape(self.plan)
         engine.allocate(self.plan)
         engine.generate(self.plan, native.device_header_text())
         self.sim = native.Sim(device)
@@ -91,13 +100,6 @@ class HipExecutor:
         if self._build_slots():
             engine.generate(self.plan, native.device_header_text())
         lowered = time.perf_counter()
-        # persistent launches (one cooperative launch for many ticks, states in registers) where the
-        # plan allows them; ATLAS_HIP_PERSISTENT=0 keeps one launch per tick, =plain issues them as
-        # ordinary launches once the kernel's occupancy shows the grid fits (for kernel tracers
-        # that cannot follow cooperative launches)
-        mode = os.environ.get("ATLAS_HIP_PERSISTENT", "1")
-        self.persistent = mode != "0"
-        self.plain_launches = mode == "plain"
         self._compile()
         self.compile_seconds = time.perf_counter() - lowered
         self.setup_seconds = lowered - started

@@ -240,3 +240,19 @@ def test_segments_longer_than_a_slot_equal_oracle_and_per_tick(monkeypatch, inde
     assert dump == expected.results and events == expected.events
     tick_dump, tick_events, _ = run(doc, "per-tick", monkeypatch, lift_recording_budget=True)
     assert tick_dump == dump and tick_events == events
+
+
+@pytest.mark.parametrize("n,edge_weights", [(300, False), (300, True), (16_384, False), (16_385, True), (98_305, False),
+                                            (98_305, True), (262_145, True), (524_289, False)])
+def test_fitted_shapes_equal_the_oracle(monkeypatch, n, edge_weights):
+    """Networks on both sides of the sizes where the executor's launch shape changes (2 blocks of 256;
+    64 of 256; 33 of 512; 97 of 1024; 129 of 2048; 171 of 3072, ragged last blocks), with counted
+    events and with a float32 weight per synapse: persistent, equal to the oracle."""
+    print(f"case: fitted shape, {n} neurons, weights {edge_weights}", flush=True)
+    doc = models.cuba_network(n, indegree=30, delay_ticks=1, steps=150, weight_scale=11.6 / 30,
+                              edge_weights=edge_weights)
+    expected = oracle.run(doc, lift_recording_budget=True)
+    assert expected.spike_count > n // 20
+    dump, events, result = run(doc, "persistent", monkeypatch, lift_recording_budget=True)
+    assert dump == expected.results and events == expected.events
+    assert result["hip_runtime"]["launches"] == 1

@@ -796,3 +796,33 @@ def test_refractory_table_equals_the_recompute_search(dt, period, start):
         expected = engine.initial_until(np.array([tick * dt]), tick + 1, dt, period)[0]
         assert table[k] == expected, (tick, table[k], expected)
     assert engine.refractory_table(0, engine.UNTIL_TABLE_TICKS + 1, dt, dt, period) is None
+
+
+@pytest.mark.parametrize("n,block", [(300, 256), (16_384, 256), (16_385, 512), (98_304, 512), (98_305, 1024),
+                                     (262_144, 1024), (262_145, 2048), (524_289, 3072), (786_433, 4096)])
+def test_fit_shape_takes_the_smallest_block_the_network_fits(n, block):
+    """fit_shape gives a persistent plan the first of FITTED it fits, and leaves alone what does not run
+    the split loop: delay 0 (the shape kept, no least number of blocks), a heavy update, a delay past
+    the ring, two populations."""
+    plan = engine.lower(models.cuba_network(n, indegree=2, delay_ticks=1, steps=5), verify_envelope=False)
+    engine.fit_shape(plan)
+    assert plan.shape.block == block and plan.total_blocks == plan.populations[0].blocks == -(-n // block)
+    assert plan.populations[0].ring == 4
+
+
+def test_fit_shape_keeps_other_plans():
+    for doc, min_blocks in ((models.cuba_network(600, p=0.02, steps=5), 1),
+                            (models.cobahh_network(600, steps=5, delay_ticks=1), 1),
+                            (models.cuba_network(600, p=0.02, steps=5, delay_ticks=40), None),
+                            (models.poisson_network(100, 200, indegree=10, steps=5), None),
+                            (models.plastic_network(500, indegree=20, steps=5), None)):
+        plan = engine.lower(doc, verify_envelope=False)
+        shape, ring = plan.shape, plan.populations[0].ring
+        assert not engine.fit_shape(plan)
+        assert plan.shape == shape and plan.min_blocks == min_blocks
+        assert plan.populations[0].ring == (ring if min_blocks is None else 3 if plan.split else 4)
+    small = engine.lower(models.cuba_network(600, p=0.02, steps=5))
+    engine.fit_shape(small)
+    engine.allocate(small)
+    engine.generate(small, native.device_header_text())
+    assert small.persistent is not None and small.total_blocks == 3
