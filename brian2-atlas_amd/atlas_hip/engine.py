@@ -642,7 +642,7 @@ class Plan:
     clocks: list = field(default_factory=list)       # (dt, start tick, steps) of each clock
     clock_buffer: int = -1
     edge_nodes: int = 0                              # events the split loop's edge buckets hold per workgroup and tick
-    min_blocks: int | None = None                    # fewest blocks of a persistent launch (PERSISTENT_MIN_BLOCKS)
+    fitted: bool = False                             # fit_shape chose the shape of its persistent launches
 
     @property
     def multi_clock(self) -> bool:
@@ -2075,6 +2075,8 @@ def _population_code(plan: Plan, pop: PopulationPlan) -> str:
     L.append("    }")
     # ---- State / load / step / store (update + threshold [+ fused reset])
     L.append(f"    static constexpr bool RESET_FUSED = {'true' if pop.reset_fused else 'false'};")
+    late = pop.reset is not None and not pop.reset_fused   # the reset follows the tick's deliveries
+    L.append(f"    static constexpr bool RESET_LATE = {'true' if late else 'false'};")
     L.append("    struct State {")
     for name, dtype, _ in pop.states:
         L.append(f"        {CTYPE[dtype]} st_{name};")
@@ -2235,7 +2237,8 @@ def _population_code(plan: Plan, pop: PopulationPlan) -> str:
     # per-tick kernel stages the states an ordered group writes in LDS instead)
     L.append("    __device__ static void store_mem(const u64* __restrict__ tab, u32 i, const State& st) {")
     L.append("        (void)tab; (void)i; (void)st;")
-    for name in sorted(written | set(pop.lds_states) | pop.fused_writes):
+    reset_writes = set(pop.reset["effects"]["writes"]) if late else set()
+    for name in sorted(written | set(pop.lds_states) | pop.fused_writes | reset_writes):
         dtype = next(s_[1] for s_ in pop.states if s_[0] == name)
         L.append(f"        __builtin_nontemporal_store(st.st_{name}, atlas::buf<{CTYPE[dtype]}>(tab, {b['state:' + name]}) + i);")
     if pop.generator is not None:
@@ -2317,6 +2320,22 @@ def _population_code(plan: Plan, pop: PopulationPlan) -> str:
             dtype = next(s[1] for s in pop.states if s[0] == name)
             L.append(f"        atlas::buf<{CTYPE[dtype]}>(tab, {b['state:' + name]})[i] = "
                      f"{commit_expr(dtype, prog.symbols[name][0])};")
+    L.append("    }")
+    # the same on the states in registers (the split loop's resets that follow the deliveries)
+    L.append("    __device__ static void reset_state(const u64* __restrict__ tab, u32 i, State& st, double t, i64 tick, "
+             "u32& fault) {")
+    L.append("        (void)tab; (void)i; (void)st; (void)tick; (void)t; (void)fault;")
+    if late:
+        if pop.refractory is not None:
+            L.append("        const bool nr = tick >= (i64)st.until;")
+        env = _scalar_env(pop, pop.reset)
+        inputs = _with_scalars(_population_inputs(pop, state_in), env, pop.reset)
+        prog = DeviceProgram(inputs, L, "zs", rng=(plan.rng_seed, "i"))
+        prog.scalar_statements(env)
+        prog.statements(pop.reset["vector"])
+        for name in pop.reset["effects"]["writes"]:
+            dtype = next(s[1] for s in pop.states if s[0] == name)
+            L.append(f"        st.st_{name} = {commit_expr(dtype, prog.symbols[name][0])};")
     L.append("    }")
     _custom_phase_code(plan, pop, L)
     _event_ring_code(pop, L)
@@ -2544,7 +2563,7 @@ def _edge_loop_candidate(plan: Plan) -> bool:
 
 
 def _min_blocks(plan: Plan) -> int:
-    return PERSISTENT_MIN_BLOCKS if plan.min_blocks is None else plan.min_blocks
+    return 1 if plan.fitted else PERSISTENT_MIN_BLOCKS
 
 
 SLOT_TARGETS = 15   # targets held inline by one 32-byte slot (word 0 is the count)
@@ -2556,17 +2575,62 @@ def per_xcd(plan: "Plan") -> int:
     return (plan.total_blocks + XCDS - 1) // XCDS
 
 
-# Shapes of persistent launches, smallest block first, with the most blocks each takes: the split
-# loop reads at most 64 source blocks per exchange wave (one wave of 256 work-items, three of 512,
-# seven of 1024), and one workgroup runs per CU.  Measured on CUBA with a fixed in-degree of 1000,
-# delay 1, us per tick, the first shape that fits against the next two (and, before, the shape of
-# choose_shape): 20,000 neurons 3.4 / 3.4 / 4.7 (4.1), 100,000 3.3 / 6.9 / 7.4 (4.4), 200,000
-# 2.9 / 4.1 / 8.4 (4.5), 300,000 3.4 / 5.0 / 9.1 (9.1), 600,000 4.0 / 4.8 (4.8); with a weight per
-# synapse 100,000 9.9 / 15.0 / 16.3 (12.6, one launch per tick), 300,000 9.7 / 17.5 / 28.7 (28.7).
-# Fewer neurons and shorter slots per workgroup shorten both of its chains; more workgroups than
-# CUs make two of them share one.
-FITTED = ((Shape(256, 256, 4, 10), 64), (Shape(512, 512, 2, 10), 192), (Shape(1024, 1024, 1, 11), CUS),
-          (Shape(2048, 1024, 2, 11), CUS), (Shape(3072, 1024, 2, 11), CUS), (Shape(4096, 1024, 2, 11), CUS))
+# Shapes of the split loop, smallest block first.  It reads at most 64 source blocks per exchange
+# wave (one wave of 256 work-items, three of 512, seven of 1024), and one workgroup runs per CU.
+# Measured on CUBA with a fixed in-degree of 1000, delay 1, us per tick, the first shape that fits
+# against the next two (and, before, the shape of choose_shape): 20,000 neurons 3.4 / 3.4 / 4.7 (4.1),
+# 100,000 3.3 / 6.9 / 7.4 (4.4), 200,000 2.9 / 4.1 / 8.4 (4.5), 300,000 3.4 / 5.0 / 9.1 (9.1), 600,000
+# 4.0 / 4.8 (4.8); with a weight per synapse 100,000 9.9 / 15.0 / 16.3 (12.6, one launch per tick),
+# 300,000 9.7 / 17.5 / 28.7 (28.7).  Fewer neurons and shorter slots per workgroup shorten both of its
+# chains; more workgroups than CUs make two of them share one.
+FITTED = (Shape(256, 256, 4, 10), Shape(512, 512, 2, 10), Shape(1024, 1024, 1, 11), Shape(2048, 1024, 2, 11),
+          Shape(3072, 1024, 2, 11), Shape(4096, 1024, 2, 11))
+
+
+def _fits_split(plan: Plan, groups: list, shape: Shape) -> bool:
+    """Whether the split loop takes the plan in this shape: two halves of waves, every workgroup on a
+    CU of its own, at most 64 source blocks per exchange wave (the first one only publishes), one fired
+    mask per lane of that wave."""
+    xwaves = SPLIT_XWAVES or shape.wg // 128
+    blocks = [-(-pop.count // shape.block) for pop in plan.populations]
+    return (1 <= xwaves < shape.wg // 64 and sum(blocks) <= CUS
+            and all(blocks[g[0].source] <= 64 * max(1, xwaves - 1) for g in groups)
+            and -(-shape.block // (shape.wg - 64 * xwaves)) * (shape.wg // 64 - xwaves) <= 64)
+
+
+def _split_lag(groups: list) -> int:
+    """The largest delay, at least 1: how many ticks ago a block waits for its readers' records; the
+    ring holds twice as many ticks and two more."""
+    return max([1] + [max(path.dvals) for group in groups for path in group])
+
+
+def _split_model(plan: Plan, groups: list) -> bool:
+    """Whether the split loop (atlas_tick.h persistent_run_split) runs the plan's ticks, whatever the
+    shape: nothing reads or writes states in memory during a tick, and every delivery is a counting
+    group of one delay applied to the states in registers (or one population's only group is an
+    ordered one that edge buckets take), under updates light enough for its few update waves."""
+    if not PERSISTENT_SPLIT or plan.multi_clock or plan.post_paths or plan.synapse_codes or not groups:
+        return False
+    # a population driving itself without delay has one chain, update to apply, and more of its waves
+    # on each part of it in persistent_run, from a few blocks on (us per tick, split loop against
+    # persistent_run: CUBA of 500 neurons 2.8 / 3.2, 4000 3.9 / 3.5, 8000 4.1 / 3.7)
+    if plan.split and len(plan.populations) == 1 and plan.populations[0].count > 1024:
+        return False
+    for pop in plan.populations:
+        if not _registers_only(pop) or pop.count > 1 << 20 or _update_ops(pop) > HEAVY_OPS:
+            return False
+        mine = [g for g in groups if g[0].target == pop.index]
+        # with a delay-0 pathway anywhere, resets that follow the deliveries keep one launch per tick
+        if plan.split and mine and pop.reset is not None and not _reset_fusable(plan, pop):
+            return False
+    edges = (len(plan.populations) == len(groups) == 1 and PERSISTENT_EDGES and edge_group(plan, groups[0])
+             and (plan.populations[0].reset is None or _reset_fusable(plan, plan.populations[0])))
+    for group in groups:
+        if len({d for path in group for d in path.dvals}) != 1 or not (counting_group(group) or edges):
+            return False
+        if any(path.pending is not None or "\0not_refractory" in _touched_post(path)[0] for path in group):
+            return False
+    return 2 * _split_lag(groups) + 2 <= RING_SLOTS
 
 
 # Operations of a neuron's tick (its update, threshold and run_regularly statements; OP_COST for the
@@ -2592,46 +2656,51 @@ def _update_ops(pop: PopulationPlan) -> int:
 
 def fit_shape(plan: Plan) -> bool:
     """Give a plan that can run persistent launches the shape they run fastest in (before
-    allocate()); whether the shape changed.  One population of at most 2^20 neurons whose single
-    delivery group persistent_eligible takes in some shape: with a delay >= 1 the first shape of
-    FITTED whose blocks it fits, at delay 0 (no split loop) or with a heavy update (HEAVY_OPS) the
-    shape it has, in both cases with no least number of blocks (a CUBA network of 500 neurons, 2
-    blocks: 3.2 us per tick persistent, 4.3 with one launch per tick)."""
-    if (plan.multi_clock or len(plan.populations) != 1 or plan.post_paths or plan.synapse_codes
-            or plan.populations[0].count > 1 << 20):
-        return False
+    allocate()); whether the shape changed.  A plan the split loop runs takes the first shape of
+    FITTED it fits; one that only persistent_run takes (a heavy update) keeps its own.  Neither has a
+    least number of blocks (a CUBA network of 500 neurons, 2 blocks: 3.2 us per tick persistent, 4.3
+    with one launch per tick)."""
     groups = delivery_groups(plan)
-    if len(groups) != 1 or not _persistent_model(plan, groups[0]):
+    shape, before = plan.shape, plan.shape
+    if _split_model(plan, groups):
+        shape = next((shape for shape in FITTED if _fits_split(plan, groups, shape)), None)
+        if shape is None:
+            return False
+        # every population's ring: 2 d + 2 ticks of the longest lag between two of their blocks
+        ring = 2 * _split_lag(groups) + 2
+    elif (len(plan.populations) == len(groups) == 1 and not plan.multi_clock and not plan.post_paths
+          and not plan.synapse_codes and plan.populations[0].count <= 1 << 20 and counting_group(groups[0])
+          and _persistent_model(plan, groups[0])):
+        # the ring of a persistent launch (2 d + 2 ticks, one more with the split launches of delay 0)
+        ring = 2 * groups[0][0].dvals[0] + 2 + (1 if plan.split else 0)
+        if ring > RING_SLOTS:
+            return False
+    else:
         return False
-    pop, group = plan.populations[0], groups[0]
-    delay = group[0].dvals[0]
-    if not counting_group(group) and not (PERSISTENT_SPLIT and PERSISTENT_EDGES and edge_group(plan, group)):
-        return False
-    # the ring of a persistent launch (2 d + 2 ticks, one more with the split launches of delay 0)
-    ring = max(pop.ring, 2 * delay + 2 + (1 if plan.split else 0))
-    if ring > RING_SLOTS:
-        return False
-    shape = plan.shape
-    if delay >= 1 and PERSISTENT_SPLIT and not SPLIT_XWAVES and _update_ops(pop) <= HEAVY_OPS:
-        shape = next(shape for shape, most in FITTED if -(-pop.count // shape.block) <= most)
-    plan.min_blocks = 1
-    pop.ring = ring
-    changed = shape != plan.shape
+    plan.fitted = True
     plan.shape = shape
-    pop.blocks = plan.total_blocks = -(-pop.count // shape.block)
-    return changed
+    plan.total_blocks = 0
+    for pop in plan.populations:
+        pop.ring = max(pop.ring, ring)
+        pop.blocks = -(-pop.count // shape.block)
+        pop.first_block = plan.total_blocks
+        plan.total_blocks += pop.blocks
+    return shape != before
+
+
+def _registers_only(pop: PopulationPlan) -> bool:
+    """Whether nothing but the update, its events and the deliveries touches the population's states
+    during a tick."""
+    return not (pop.poisson_inputs or pop.generator is not None or pop.event_monitors or pop.custom_events
+                # run on the states in memory after the reset
+                or any(where == "end" for _, where in pop.regular)
+                or (pop.monitor_record and pop.monitor_vars))
 
 
 def _persistent_model(plan: Plan, group: list[PathwayPlan]) -> bool:
     """What persistent_eligible asks of the population and its delivery group whatever the shape."""
     pop = plan.populations[0]
-    if pop.poisson_inputs or pop.generator is not None or pop.event_monitors or pop.custom_events:
-        return False
-    if any(where == "end" for _, where in pop.regular):   # run on the states in memory after the reset
-        return False
-    if pop.monitor_record and pop.monitor_vars:
-        return False
-    if not (pop.reset is None or _reset_fusable(plan, pop)):
+    if not _registers_only(pop) or not (pop.reset is None or _reset_fusable(plan, pop)):
         return False
     delays = {d for path in group for d in path.dvals}
     if len(delays) != 1 or (min(delays) < 1) != plan.split:
@@ -4147,21 +4216,36 @@ def generate(plan: Plan, header_text: str) -> None:
             lines.append("    }")
         return lines
 
+    def readers_of(pop: PopulationPlan) -> list[int]:
+        # populations that read this one's ring and that it does not read
+        read = {g[0].source for g in groups if g[0].target == pop.index}
+        return sorted({g[0].target for g in groups if g[0].source == pop.index} - read - {pop.index})
+
     def persistent_body() -> list[str]:
         # one cooperative launch runs `ticks` ticks: the block's states stay in registers, the
         # spike ring is exchanged device-coherently and a grid barrier separates the ticks
-        pop = plan.populations[0]
         px = padded // XCDS
+        if split_loop:
+            # exchange and update waves side by side (atlas_tick.h persistent_run_split)
+            lines = ["    __shared__ atlas::LdsSplit s;",
+                     f"    const u32 wg = (blockIdx.x % {XCDS}u) * {px}u + blockIdx.x / {XCDS}u;",
+                     f"    if (wg >= {total}u) return;"]
+            for pop in plan.populations:
+                into = [k for k, g in enumerate(groups) if g[0].target == pop.index]
+                readers = readers_of(pop)
+                lines.append(f"    if (wg - {pop.first_block}u < {pop.blocks}u) {{")
+                lines.append(f"        atlas::persistent_run_split<Pop{pop.index}, "
+                             f"atlas::GroupList<{', '.join(f'Group{k}' for k in into)}>, "
+                             f"atlas::ReaderList<{', '.join(f'Reader{q}' for q in readers)}>, "
+                             f"{f'Fused{pop.index}' if into else 'atlas::NoFused'}>(tab, tick0, ticks, "
+                             f"wg - {pop.first_block}u, wg, {total}u, {plan.start_tick}LL, {hexlit(plan.dt)}, s);")
+                lines.append("        return;")
+                lines.append("    }")
+            return lines
+        pop = plan.populations[0]
         n = pop.index
         mine = [k for k, g in enumerate(groups) if g[0].target == pop.index]
         assert len(mine) == 1
-        if split_loop:
-            # delay >= 1: exchange and update waves side by side (atlas_tick.h persistent_run_split)
-            return ["    __shared__ atlas::LdsSplit s;",
-                    f"    const u32 wg = (blockIdx.x % {XCDS}u) * {px}u + blockIdx.x / {XCDS}u;",
-                    f"    if (wg >= {total}u) return;",
-                    f"    atlas::persistent_run_split<Pop{n}, Group{mine[0]}, Fused{n}>(tab, tick0, ticks, wg, {total}u, "
-                    f"{plan.start_tick}LL, {hexlit(plan.dt)}, s);"]
         return ["    __shared__ atlas::Lds s;",
                 f"    const u32 wg = (blockIdx.x % {XCDS}u) * {px}u + blockIdx.x / {XCDS}u;",
                 f"    if (wg >= {total}u) return;",
@@ -4191,16 +4275,24 @@ def generate(plan: Plan, header_text: str) -> None:
         parts.extend(lines)
         parts.append("}")
     plan.persistent = None
-    # the split loop needs a delay of at least one tick, two halves of waves and at most 64 source
-    # blocks per exchange wave (the first exchange wave only publishes)
+    # the split loop: a fitted plan that it takes, or one population's only group of a delay >= 1
     xwaves = SPLIT_XWAVES or WG // 128
-    # and one fired mask per lane of the publishing wave: (rounds per update work-item) x (update waves)
-    split_loop = (PERSISTENT_SPLIT and not plan.split and 1 <= xwaves < WG // 64
-                  and plan.total_blocks <= 64 * max(1, xwaves - 1)
-                  and -(-BLOCK // (WG - 64 * xwaves)) * (WG // 64 - xwaves) <= 64)
+    wide = (plan.fitted and _split_model(plan, groups) and _fits_split(plan, groups, plan.shape)
+            and all(pop.fused_counts or pop.fused_split or pop.fused_edges for pop in plan.populations
+                    if any(g[0].target == pop.index for g in groups))
+            and all("slot" in path.buffers and path.index not in plan.slot_fallback for g in groups for path in g))
+    split_loop = wide or (PERSISTENT_SPLIT and not plan.split and len(groups) == 1 and _fits_split(plan, groups, plan.shape))
     if split_loop:
+        pathways_into = [sum(len(g) for g in groups if g[0].target == pop.index) for pop in plan.populations]
         parts.insert(parts.index(header_text), f"#define ATLAS_XWAVES {xwaves}u")
-    eligible = persistent_eligible(plan, groups, counting, split_loop)
+        parts.insert(parts.index(header_text), f"#define ATLAS_SUM_NP {max(1, *pathways_into)}u")
+    eligible = wide or persistent_eligible(plan, groups, counting, split_loop)
+    if eligible and split_loop:
+        lag = _split_lag(groups)
+        for q in sorted({q for pop in plan.populations for q in readers_of(pop)}):
+            reader = plan.populations[q]
+            parts.append(f"struct Reader{q} {{ static constexpr u32 NB = {reader.blocks}u, R = {reader.ring}u, LAG = {lag}u;\n"
+                         f"    static constexpr int SMALL = {reader.buffers['spk_small']}; }};")
     if eligible and split_loop and plan.populations[0].fused_edges:
         # the edge buckets take the LDS the split loop's other arrays leave (LdsSplit), by tick
         # parity: a count array of BLOCK + 4 words, a key (4 bytes) and a value (8 bytes) per event;

@@ -1517,20 +1517,23 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
 }
 
 // ---------------------------------------------------------------- split persistent tick loop
-// For a delay d >= 1 the counts of tick t need only the spikes of tick t - d, and the update of
-// tick t + 1 only the counts of tick t applied.  The split loop runs these two chains side by side
-// in one workgroup: its first half of waves (the exchange waves) reads the records of tick t - d
+// The split loop runs the two chains of a tick side by side in one workgroup: its first half of waves
+// (the exchange waves) reads the records of tick t - d of every group of pathways into the population
 // and counts the events of tick t, while its second half (the update waves, which keep the block's
-// states in registers) applies the counts of tick t - 1, runs the update of tick t and publishes
-// its spikes.  One workgroup barrier per tick hands the counts over; the LDS counters are
-// double-buffered by tick parity.
+// states in registers) applies the counts of tick t - 1, runs the resets that follow them, then the
+// update of tick t, and publishes its spikes.  For d >= 1 the counts of tick t need only the spikes of
+// tick t - d, and the update of tick t + 1 only the counts of tick t applied.  For d = 0 the exchange
+// waves wait for the spikes of the same tick instead.  One workgroup barrier per tick hands the counts
+// over; the LDS counters are double-buffered by tick parity.
 //
 // There is no grid barrier: each exchange wave polls the stamped records of tick t - d of its own
-// share of the source blocks until they carry that tick's stamp.  A block publishes tick t only
-// after its exchange waves have read every block's records of tick t - 1 - d (their counts come
-// before its update), so a block that publishes tick e + R has seen every block publish tick
-// e + R - 1 - d, and every block has read tick e before publishing tick e + R - 1 - d when
-// R >= 2 d + 2: a ring of 2 d + 2 ticks is never overwritten while read.  Each publication waits
+// share of the source blocks until they carry that tick's stamp.  A population that is read but does
+// not read its readers' spikes waits for their records of LAG ticks ago all the same (Readers), so
+// that every block is bound to every block that reads its ring.  A block P publishes tick e + R after its
+// exchange waves have seen a reader Q publish tick e + R - 1 - L (L the delay of P's group from Q,
+// or LAG); Q has then read P's tick e + R - 2 - L - d.  With L, d <= D (the largest delay, at least 1)
+// and R >= 2 D + 2, a slot is never overwritten before it is read (one population driving itself at
+// delay d needs 2 d + 2 slots, 2 at delay 0).  Each publication waits
 // for the stores of the previous one first (vmcnt(0); they are long complete), so a reader that
 // has seen a block's tick e - 1 sees its words of tick e as tick e - R left them or newer: the
 // stamp argument of the ring holds as with the barrier.
@@ -1544,7 +1547,10 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
 //
 // Measured on config 3 (1M neurons, 245 workgroups of 1024 work-items): 7.8 us per tick for the
 // single-chain loop, 6.6 split into halves, 6.0 with the update waves at higher priority and the
-// bound checks of full blocks dropped, 5.8 with the masks published by the first exchange wave.
+// bound checks of full blocks dropped, 5.8 with the masks published by the first exchange wave, 5.2
+// with long segments shared by the wave.  Against one launch per tick, us per tick: 20,011 neurons with
+// voltage-jump synapses of two delays 3.5 (8.7), 100,000 of them 4.6 (11.0), 2000 Poisson inputs
+// into 4000 neurons 2.2 (5.8), 8000 into 20,000 at delay 0 2.1 (5.8): the chains' round trips remain.
 #ifndef ATLAS_XLIST
 #define ATLAS_XLIST 512u               // fired sources one exchange wave keeps in LDS per tick
 #endif
@@ -1570,6 +1576,9 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
 #ifndef ATLAS_EDGE_NODES
 #define ATLAS_EDGE_NODES 0u
 #endif
+#ifndef ATLAS_SUM_NP
+#define ATLAS_SUM_NP ATLAS_MAX_NP   // most pathways into one population
+#endif
 #define ATLAS_EDGE_CNT_WORDS (ATLAS_BLOCK + ATLAS_BLOCK / 64u + 4u)
 // target j's count word: one pad word per 64, so with 4096-neuron blocks the scanning wave's lanes
 // (64 consecutive counts each) read and write 64 different LDS banks at every step
@@ -1584,7 +1593,7 @@ struct LdsSplit {
     u32 x_scan;                                // edge buckets: the last tick (+ 1) whose counts are scanned
     u32 x_bad[2];                              // edge buckets: the tick (by parity) did not fit (replayed)
     u64 pub_masks[64];                         // the tick's fired masks, (round, update wave) order
-    u32 wave_sums[2 * ATLAS_WAVES * ATLAS_MAX_NP];
+    u32 wave_sums[2 * ATLAS_WAVES * ATLAS_SUM_NP];
     alignas(16) u32 hist[ATLAS_SPLIT_HIST];    // counters of tick t at (t & 1) * ATLAS_HIST, or edge buckets
     u32 xlist[ATLAS_XWAVES][ATLAS_XLIST];      // each exchange wave's fired list
     u32 xstart[ATLAS_XWAVES][64];              // each exchange wave's block starts in its list
@@ -1673,29 +1682,43 @@ struct BoolTag {
     static constexpr bool value = B;
 };
 
-template <class Pop, class Group, class Fused, u32 UR, u32 UL, bool FULL = false>
+template <class Pop, class Fused, u32 NP, u32 UR, u32 UL, bool FULL = false>
 __device__ __forceinline__ void apply_split(const u64* __restrict__ tab, u32 base, u32 n, u32 ul,
                                             typename Pop::State* st, LdsSplit& s, i64 tick, double dt_clock,
                                             u32& fault) {
-    constexpr u32 NP = Group::NP;
-    __builtin_assume(ul < UL);
-    const u32* h = &s.hist[(u32)(tick & 1) * ATLAS_HIST + Group::HIST_BASE];
-    u32 cn[UR][NP];
+    if constexpr (NP > 0) {
+        __builtin_assume(ul < UL);
+        const u32* h = &s.hist[(u32)(tick & 1) * ATLAS_HIST];
+        u32 cn[UR][NP];
 #pragma unroll
-    for (u32 r = 0; r < UR; ++r) {
-        const u32 j = r * UL + ul;
+        for (u32 r = 0; r < UR; ++r) {
+            const u32 j = r * UL + ul;
 #pragma unroll
-        for (u32 p = 0; p < NP; ++p) cn[r][p] = (FULL ? j < ATLAS_BLOCK : j < n) ? h[p * ATLAS_BLOCK + j] : 0u;
-    }
-    const double t = (double)tick * dt_clock;
-#pragma unroll
-    for (u32 r = 0; r < UR; ++r) {
-        const u32 j = r * UL + ul;
-        if (FULL ? j < ATLAS_BLOCK : j < n) {
-            Fused::apply_n(tab, base + j, st[r], cn[r], t, tick, fault);
-#pragma unroll
-            for (u32 p = 0; p < NP; ++p) s.hist[(u32)(tick & 1) * ATLAS_HIST + Group::HIST_BASE + p * ATLAS_BLOCK + j] = 0;
+            for (u32 p = 0; p < NP; ++p) cn[r][p] = (FULL ? j < ATLAS_BLOCK : j < n) ? h[p * ATLAS_BLOCK + j] : 0u;
         }
+        const double t = (double)tick * dt_clock;
+#pragma unroll
+        for (u32 r = 0; r < UR; ++r) {
+            const u32 j = r * UL + ul;
+            if (FULL ? j < ATLAS_BLOCK : j < n) {
+                Fused::apply_n(tab, base + j, st[r], cn[r], t, tick, fault);
+#pragma unroll
+                for (u32 p = 0; p < NP; ++p) s.hist[(u32)(tick & 1) * ATLAS_HIST + p * ATLAS_BLOCK + j] = 0;
+            }
+        }
+    }
+}
+
+// The resets of the neurons that fired at `tick` (fired: this work-item's, a bit per round), after
+// its deliveries, where the reset does not commute with them.
+template <class Pop, u32 UR, u32 UL>
+__device__ __forceinline__ void reset_split(const u64* __restrict__ tab, u32 base, u32 ul, typename Pop::State* st,
+                                            u32 fired, i64 tick, double dt_clock, u32& fault) {
+    if constexpr (Pop::RESET_LATE) {
+        const double t = (double)tick * dt_clock;
+#pragma unroll
+        for (u32 r = 0; r < UR; ++r)
+            if (fired >> r & 1u) Pop::reset_state(tab, base + r * UL + ul, st[r], t, tick, fault);
     }
 }
 
@@ -1861,30 +1884,40 @@ __device__ __forceinline__ void publish_split(const u64* __restrict__ tab, i64 t
     }
 }
 
-template <class Pop, class Group, class Fused>
-__device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab, i64 tick0, i64 ticks, u32 blk, u32 nwg,
-                                     i64 start_tick, double dt_clock, LdsSplit& s) {
-    static_assert(Group::NG == 1 && (Group::COUNT ? Group::SLOTS : Group::EDGE_SLOTS),
-                  "one delay group through slot tables");
-    constexpr bool EDGE = !Group::COUNT;             // ordered: edge-keyed buckets instead of counters
-    constexpr u32 HB = Group::HIST_BASE;
-    constexpr u32 NP = Group::NP;
-    constexpr u32 ITEMS = Group::DISJOINT ? 1u : NP;
+// The delivery groups into a population (in schedule order), and the populations its spikes reach.
+template <class... G>
+struct GroupList {
+    static constexpr u32 NP = (0u + ... + G::NP);                       // pathways, the groups' in order
+    static constexpr bool EDGE = (false || ... || !G::COUNT);           // one ordered group (edge buckets)
+    static constexpr bool SLOTS = (true && ... && (G::NG == 1 && (G::COUNT ? G::SLOTS : G::EDGE_SLOTS)));
+    template <class F>
+    __device__ static __forceinline__ void each(const F& f) { (f(G{}), ...); }
+};
+template <class... P>
+struct ReaderList {
+    template <class F>
+    __device__ static __forceinline__ void each(const F& f) { (f(P{}), ...); }
+};
+
+template <class Pop, class Groups, class Readers, class Fused>
+__device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab, i64 tick0, i64 ticks, u32 blk, u32 wg,
+                                     u32 nwg, i64 start_tick, double dt_clock, LdsSplit& s) {
+    static_assert(Groups::SLOTS, "groups of one delay through slot tables");
+    constexpr bool EDGE = Groups::EDGE;              // ordered: edge-keyed buckets instead of counters
+    constexpr u32 NP = Groups::NP;
+    constexpr u32 NPA = NP > 0 ? NP : 1;
     constexpr u32 XW = ATLAS_XWAVES;                 // exchange waves
     constexpr u32 UL = ATLAS_WG - 64 * XW;           // update work-items
     constexpr u32 UR = (ATLAS_BLOCK + UL - 1) / UL;  // neurons per update work-item (the last round may be partial)
     constexpr u32 XQ = XW > 1 ? 1u : 0u;             // the first exchange wave only publishes
     constexpr u32 XE = XW - XQ;                      // exchange waves that read records
-    constexpr u32 RPW = (Group::SRC_NB + XE - 1) / XE;   // source blocks per exchange wave
     constexpr u32 SP = 2;                            // slot loads in flight per exchange lane
     static_assert(XW >= 1 && XW < ATLAS_WAVES, "exchange and update waves");
-    static_assert(RPW <= 64, "one record per exchange lane");
-    static_assert(Group::gval_max >= 1, "the counts of a tick need earlier ticks' spikes only");
-    static_assert(Pop::R == Group::SRC_R && Pop::R >= 2 * Group::gval_max + 2 && Pop::R < 4095u &&
-                  Pop::R <= ATLAS_RING_PREV, "ring of 2 d + 2 ticks");
+    static_assert(Pop::R < 4095u && Pop::R <= ATLAS_RING_PREV, "ring slots whose counts are kept");
     static_assert(Pop::N <= ATLAS_RING_VALUE + 1u, "neuron indices fit a stamped word");
-    static_assert(EDGE || (HB + NP * ATLAS_BLOCK <= ATLAS_HIST && ATLAS_SPLIT_HIST >= 2 * ATLAS_HIST),
+    static_assert(EDGE || (NP * ATLAS_BLOCK <= ATLAS_HIST && ATLAS_SPLIT_HIST >= 2 * ATLAS_HIST),
                   "one tick's counters fit a buffer");
+    static_assert(UR <= 32, "a fired bit per round");
     static_assert(!EDGE || (ATLAS_EDGE_NODES > 0 && ATLAS_EDGE_NODES % 2 == 0 &&
                             2 * ATLAS_EDGE_CNT_WORDS + 6 * ATLAS_EDGE_NODES <= ATLAS_SPLIT_HIST && NP <= 4),
                   "edge buckets fit their buffer");
@@ -1894,8 +1927,8 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
     const u32 wave = threadIdx.x >> 6;
     const bool xwave = wave < XW;
     const u32 ul = threadIdx.x - 64 * XW;            // update work-item index (update waves)
-    const u32 delay = Group::gval(0);
     bool gave_up = false;
+    u32 fired_before = 0;   // this work-item's neurons that fired in the previous tick, for their resets
     typename Pop::State st[UR];
     if (!xwave) {
 #pragma unroll
@@ -1913,22 +1946,45 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
         s.x_scan = 0;
         s.x_bad[0] = s.x_bad[1] = 0;
     }
-    u64 lane_delivered[NP];
+    u64 lane_delivered[NPA];
 #pragma unroll
-    for (u32 p = 0; p < NP; ++p) lane_delivered[p] = 0;
+    for (u32 p = 0; p < NPA; ++p) lane_delivered[p] = 0;
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the state loads, before the loop
     __syncthreads();
     for (i64 k = 0; k < ticks; ++k) {
         const i64 tick = tick0 + k;
         u32 fault = 0;
         if (xwave) {
-            // the counts of tick `tick`: the spikes of tick - d, into the counters of tick & 1
+            const u32 xe = wave - XQ;   // this wave's share of the source blocks
+            // the blocks that read this population's ring and that it does not read: their records of
+            // LAG ticks ago are waited for, so that no block runs more than the ring ahead of them
+            Readers::each([&](auto reader) {
+                using Reader = decltype(reader);
+                const i64 seen = tick - (i64)Reader::LAG;
+                if (wave >= XQ && seen >= start_tick)
+                    for (u32 b = xe * 64 + lane; b < Reader::NB; b += XE * 64) {
+                        uint4 rc[ATLAS_REC_WORDS / 4];
+                        ring_wait_record(buf<const u32>(tab, Reader::SMALL) +
+                                         ((u64)(u32)(seen % Reader::R) * Reader::NB + b) * ATLAS_REC_WORDS,
+                                         ring_stamp(seen), rc, gave_up, fault);
+                    }
+            });
+            // the counts of tick `tick`: each group's spikes of tick - d, into the counters of tick & 1
+            Groups::each([&](auto group) {
+            using Group = decltype(group);
+            constexpr u32 HB = Group::HIST_BASE;
+            constexpr u32 GP = HB / ATLAS_BLOCK;                 // its first pathway among the groups'
+            constexpr u32 ITEMS = Group::DISJOINT ? 1u : Group::NP;
+            constexpr u32 RPW = (Group::SRC_NB + XE - 1) / XE;   // source blocks per exchange wave
+            static_assert(RPW <= 64, "one record per exchange lane");
+            static_assert(!EDGE || Group::gval_max >= 1, "edge buckets are placed ahead of the update");
+            static_assert(Group::SRC_R >= 2 * Group::gval_max + 2, "ring of 2 d + 2 ticks");
+            const u32 delay = Group::gval(0);
             const i64 emitted = tick - (i64)delay;
             const bool active = emitted >= start_tick;
-            const u32 xe = wave - XQ;   // this wave's share of the source blocks
             const u32 eslot = active ? (u32)(emitted % Group::SRC_R) : 0u;
             const u32 stamp = ring_stamp(emitted);
-            const u32 valid = Group::SRC_NB - xe * RPW < RPW ? Group::SRC_NB - xe * RPW : RPW;
+            const u32 valid = xe * RPW < Group::SRC_NB ? (Group::SRC_NB - xe * RPW < RPW ? Group::SRC_NB - xe * RPW : RPW) : 0u;
             // the wave's fired list: one record per lane, a wave scan of the counts, the ids in the
             // wave's LDS list (ids past a record's marked, read from the ring below); its length
             auto read_list = [&]() -> u32 {
@@ -2009,15 +2065,15 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
                     __builtin_amdgcn_s_setprio(ATLAS_XPRIO);
                     const u32 total = read_list();
                     u32* hist = &s.hist[(u32)(tick & 1) * ATLAS_HIST + HB];
-                    u32 per_path[NP];
+                    u32 per_path[Group::NP];
 #pragma unroll
-                    for (u32 p = 0; p < NP; ++p) per_path[p] = 0;
+                    for (u32 p = 0; p < Group::NP; ++p) per_path[p] = 0;
                     for (u32 c0 = 0; c0 < total * ITEMS; c0 += 64 * SP)
                         slot_pass(c0, total, [&](u32 pq, const u32* w) {
-                            const bool ok = pq < NP;
+                            const bool ok = pq < Group::NP;
                             const u32 c = ok ? (w[0] & 0xFFFFu) : 0u;
 #pragma unroll
-                            for (u32 p = 0; p < NP; ++p) per_path[p] += pq == p ? c : 0u;
+                            for (u32 p = 0; p < Group::NP; ++p) per_path[p] += pq == p ? c : 0u;
                             const u32 inline_cnt = c <= 15u ? c : 0u;
                             u32* h = &hist[(ok ? pq : 0u) * ATLAS_BLOCK];
 #pragma unroll
@@ -2028,7 +2084,7 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
                             count_long_slots<Group>(tab, c > 15u, pq, c, w[1], blk, hist);
                         });
 #pragma unroll
-                    for (u32 p = 0; p < NP; ++p) lane_delivered[p] += per_path[p];
+                    for (u32 p = 0; p < Group::NP; ++p) lane_delivered[(EDGE ? 0u : GP) + p] += per_path[p];
                     __builtin_amdgcn_s_setprio(0);
                 }
             } else if (wave >= XQ) {
@@ -2041,15 +2097,15 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
                 u32 total = 0;
                 if (active) {
                     total = read_list();
-                    u32 per_path[NP];
+                    u32 per_path[Group::NP];
 #pragma unroll
-                    for (u32 p = 0; p < NP; ++p) per_path[p] = 0;
+                    for (u32 p = 0; p < Group::NP; ++p) per_path[p] = 0;
                     for (u32 c0 = 0; c0 < total * ITEMS; c0 += 64 * SP)
                         slot_pass(c0, total, [&](u32 pq, const u32* w) {
-                            const bool ok = pq < NP;
+                            const bool ok = pq < Group::NP;
                             const u32 c = ok ? (w[0] & 0xFFFFu) : 0u;
 #pragma unroll
-                            for (u32 p = 0; p < NP; ++p) per_path[p] += pq == p ? c : 0u;
+                            for (u32 p = 0; p < Group::NP; ++p) per_path[p] += pq == p ? c : 0u;
                             const u32 inline_cnt = c <= 12u ? c : 0u;
 #pragma unroll
                             for (u32 r = 0; r < 12; ++r) {
@@ -2061,7 +2117,7 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
                             });
                         });
 #pragma unroll
-                    for (u32 p = 0; p < NP; ++p) lane_delivered[p] += per_path[p];
+                    for (u32 p = 0; p < Group::NP; ++p) lane_delivered[(EDGE ? 0u : GP) + p] += per_path[p];
                 }
                 // every exchange wave has counted: the first scans
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -2091,7 +2147,7 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
                     };
                     for (u32 c0 = 0; c0 < total * ITEMS; c0 += 64 * SP)
                         slot_pass(c0, total, [&](u32 pq, const u32* w) {
-                            const bool ok = pq < NP;
+                            const bool ok = pq < Group::NP;
                             const u32 c = ok ? (w[0] & 0xFFFFu) : 0u;
                             const u32 pp = ok ? pq : 0u;
                             const u32 inline_cnt = c <= 12u ? c : 0u;
@@ -2107,6 +2163,7 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
                 }
                 __builtin_amdgcn_s_setprio(0);
             }
+            });
             if (wave == 0) publish_split<Pop, UR, ATLAS_WAVES - XW, UL>(tab, tick, blk, base, n, s, gave_up, fault);
         } else {
           // full blocks (all but possibly the last) bound their neurons by the block size, a
@@ -2125,17 +2182,21 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
                 if (lane == 0) atomicAdd(&s.apply_done, 1u);
             } else {
-                if (k > 0) apply_split<Pop, Group, Fused, UR, UL, FULL>(tab, base, n, ul, st, s, tick - 1, dt_clock, fault);
+                if (k > 0) apply_split<Pop, Fused, NP, UR, UL, FULL>(tab, base, n, ul, st, s, tick - 1, dt_clock, fault);
             }
+            if (k > 0) reset_split<Pop, UR, UL>(tab, base, ul, st, fired_before, tick - 1, dt_clock, fault);
             // the update of tick
             u64 masks[UR];
+            u32 fired_now = 0;
 #pragma unroll
             for (u32 r = 0; r < UR; ++r) {
                 const u32 j = r * UL + ul;
                 bool fired = false;
                 if (FULL ? j < ATLAS_BLOCK : j < n) fired = Pop::step(tab, base + j, t, tick, st[r], fault, until_next);
                 masks[r] = __ballot(fired);
+                if constexpr (Pop::RESET_LATE) fired_now |= (fired ? 1u : 0u) << r;
             }
+            fired_before = fired_now;
             // the fired masks to LDS, then the arrival the publishing wave waits for
             u32 uw = wave - XW;
             asm volatile("" : "+v"(uw));   // the masks' addresses formed here, not kept live across ticks
@@ -2170,8 +2231,9 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
         if constexpr (EDGE) {
             if (ticks > 0) apply_split_edges<Pop, Fused, UR, UL>(tab, base, n, ul, st, s, last, dt_clock, fault);
         } else {
-            if (ticks > 0) apply_split<Pop, Group, Fused, UR, UL>(tab, base, n, ul, st, s, last, dt_clock, fault);
+            if (ticks > 0) apply_split<Pop, Fused, NP, UR, UL>(tab, base, n, ul, st, s, last, dt_clock, fault);
         }
+        if (ticks > 0) reset_split<Pop, UR, UL>(tab, base, ul, st, fired_before, last, dt_clock, fault);
         report(tab, Pop::FAULT, fault);
 #pragma unroll
         for (u32 r = 0; r < UR; ++r) {
@@ -2179,23 +2241,30 @@ __device__ __forceinline__ void persistent_run_split(const u64* __restrict__ tab
             if (j < n) Pop::store_mem(tab, base + j, st[r]);
         }
     }
+    if constexpr (NP > 0) {
 #pragma unroll
-    for (u32 p = 0; p < NP; ++p) {
-        u64 v = lane_delivered[p];
+        for (u32 p = 0; p < NP; ++p) {
+            u64 v = lane_delivered[p];
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-        if (lane == 0) {
-            s.wave_sums[2 * (wave * NP + p)] = (u32)v;
-            s.wave_sums[2 * (wave * NP + p) + 1] = (u32)(v >> 32);
+            for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+            if (lane == 0) {
+                s.wave_sums[2 * (wave * NP + p)] = (u32)v;
+                s.wave_sums[2 * (wave * NP + p) + 1] = (u32)(v >> 32);
+            }
         }
+        lds_barrier();
+        Groups::each([&](auto group) {
+            using Group = decltype(group);
+            constexpr u32 GP = EDGE ? 0u : Group::HIST_BASE / ATLAS_BLOCK;
+            if (threadIdx.x >= Group::NP) return;
+            u64 delivered = 0;
+            for (u32 w = 0; w < XW; ++w) {
+                const u32 at = 2 * (w * NP + GP + threadIdx.x);
+                delivered += (u64)s.wave_sums[at] | (u64)s.wave_sums[at + 1] << 32;
+            }
+            if (delivered) buf<u64>(tab, Group::DELIVERED)[(u64)Group::path_index(threadIdx.x) * nwg + wg] += delivered;
+        });
     }
-    lds_barrier();
-    u64 delivered = 0;
-    if (threadIdx.x < NP)
-        for (u32 w = 0; w < XW; ++w)
-            delivered += (u64)s.wave_sums[2 * (w * NP + threadIdx.x)] | (u64)s.wave_sums[2 * (w * NP + threadIdx.x) + 1] << 32;
-    if (threadIdx.x < NP && delivered)
-        buf<u64>(tab, Group::DELIVERED)[(u64)Group::path_index(threadIdx.x) * nwg + blk] += delivered;
 }
 
 // ---------------------------------------------------------------- pushed counts

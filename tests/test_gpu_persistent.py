@@ -256,3 +256,27 @@ def test_fitted_shapes_equal_the_oracle(monkeypatch, n, edge_weights):
     dump, events, result = run(doc, "persistent", monkeypatch, lift_recording_budget=True)
     assert dump == expected.results and events == expected.events
     assert result["hip_runtime"]["launches"] == 1
+
+
+@pytest.mark.parametrize("doc", [
+    models.delta_lif_network(300, indegree=20, steps=600),                       # 2 blocks, delays 2 and 1, late reset
+    models.delta_lif_network(16_500, indegree=60, steps=300),                    # 33 blocks of 512
+    models.delta_lif_network(4000, indegree=50, steps=400, delays=(1, 12), dtype="f64"),
+    models.poisson_network(700, 1300, indegree=40, steps=800, delay_ticks=0),
+    models.poisson_network(17_000, 300, indegree=300, steps=300, delay_ticks=1),  # 34 + 1 blocks of 512
+    models.poisson_network(300, 17_000, indegree=30, steps=300, delay_ticks=5),   # 1 + 34 blocks of 512
+    models.cuba_network(1024, p=0.05, steps=600)], ids=lambda doc: "")
+def test_split_loop_of_several_groups_and_populations_equals_the_oracle(monkeypatch, doc):
+    """The split loop over several counting groups of different delays, resets after the deliveries, a
+    population that reads no spikes but waits for its readers, and delay 0: equal to the oracle in one
+    launch and in launches of 37 ticks."""
+    sizes = [pop["count"] for pop in doc["definition"]["populations"]]
+    print(f"case: split loop, populations {sizes}", flush=True)
+    expected = oracle.run(doc, lift_recording_budget=True)
+    assert expected.spike_count > 100
+    dump, events, result = run(doc, "persistent", monkeypatch, lift_recording_budget=True)
+    assert dump == expected.results and events == expected.events
+    assert result["hip_runtime"]["launches"] == 1
+    monkeypatch.setattr(engine, "PERSISTENT_TICKS", 37)
+    dump, events, _ = run(doc, "persistent", monkeypatch, lift_recording_budget=True)
+    assert dump == expected.results and events == expected.events

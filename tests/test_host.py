@@ -811,18 +811,34 @@ def test_fit_shape_takes_the_smallest_block_the_network_fits(n, block):
 
 
 def test_fit_shape_keeps_other_plans():
-    for doc, min_blocks in ((models.cuba_network(600, p=0.02, steps=5), 1),
-                            (models.cobahh_network(600, steps=5, delay_ticks=1), 1),
-                            (models.cuba_network(600, p=0.02, steps=5, delay_ticks=40), None),
-                            (models.poisson_network(100, 200, indegree=10, steps=5), None),
-                            (models.plastic_network(500, indegree=20, steps=5), None)):
+    for doc, fitted in ((models.cobahh_network(600, steps=5), True), (models.cuba_network(1100, p=0.02, steps=5), True), (models.cobahh_network(600, steps=5, delay_ticks=1), True),
+                        (models.cuba_network(600, p=0.02, steps=5, delay_ticks=40), False),
+                        (models.generator_network(50, 200, spikes=100, indegree=10, steps=20), False),
+                        (models.plastic_network(500, indegree=20, steps=5), False)):
         plan = engine.lower(doc, verify_envelope=False)
         shape, ring = plan.shape, plan.populations[0].ring
         assert not engine.fit_shape(plan)
-        assert plan.shape == shape and plan.min_blocks == min_blocks
-        assert plan.populations[0].ring == (ring if min_blocks is None else 3 if plan.split else 4)
-    small = engine.lower(models.cuba_network(600, p=0.02, steps=5))
-    engine.fit_shape(small)
-    engine.allocate(small)
-    engine.generate(small, native.device_header_text())
-    assert small.persistent is not None and small.total_blocks == 3
+        assert plan.shape == shape and plan.fitted == fitted
+        assert plan.populations[0].ring == (ring if not fitted else 3 if plan.split else 4)
+
+
+@pytest.mark.parametrize("doc,rings,readers", [
+    (models.cuba_network(600, p=0.02, steps=5), [4], []),                                # delay 0: lag 1
+    (models.delta_lif_network(3000, indegree=40, steps=5), [6], []),                     # delays 2 and 1, late reset
+    (models.poisson_network(300, 700, indegree=10, steps=5), [4, 4], ["Reader1"]),       # two populations
+    (models.poisson_network(300, 700, indegree=10, steps=5, delay_ticks=0), [4, 4], ["Reader1"]),
+    (models.poisson_network(300, 700, indegree=10, steps=5, delay_ticks=5), [12, 12], ["Reader1"])])
+def test_fitted_plans_of_several_groups_run_the_split_loop(doc, rings, readers):
+    """The split loop takes several counting groups of one delay each (0 included), resets that follow
+    the deliveries and several populations; a population that is read but does not read back waits for
+    its readers.  Every ring holds 2 max(d, 1) + 2 ticks, and the module compiles."""
+    plan = engine.lower(doc, verify_envelope=False)
+    engine.fit_shape(plan)
+    engine.allocate(plan)
+    engine.generate(plan, native.device_header_text())
+    assert plan.fitted and plan.persistent is not None
+    assert [pop.ring for pop in plan.populations] == rings
+    run = plan.source[plan.source.index("atlas_run(const u64*"):]
+    assert run.count("persistent_run_split<") == len(plan.populations)
+    assert [name for name in ("Reader0", "Reader1") if name in run] == readers
+    assert len(rtc.compile_source(plan.source, engine.COMPILE_OPTIONS)) > 1000
