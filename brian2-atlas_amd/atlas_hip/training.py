@@ -321,13 +321,19 @@ class NativeLIFTrainer:
         loss = 0.0
         for value in out["losses"]:
             loss += float(value)
-        return dict(schema="b2-lif-training-result-v1", state=copy.deepcopy(self.state), loss=loss / batch,
+        return dict(schema="b2-lif-training-result-v1", state=self._state_copy(), loss=loss / batch,
                     backend="hip", numeric_profile=NUMERIC_PROFILE, gradients=gradients,
                     initial_gradients=out["initial_grad"].astype(np.float64),
                     final_membrane=out["membrane"].astype(np.float64), spikes=out["spikes"].astype(np.float64),
                     logits=out["logits"].astype(np.float64), losses=out["losses"].astype(np.float64),
                     gradient_scope="tbptt-detach-boundaries" if (plan["tbptt_window"] or time) < time
                     else "full-bptt")
+
+    def _state_copy(self) -> dict:
+        """The state's own lists copied (their elements are floats; a deep copy visits each of them,
+        4.4 ms of a gradients() call of [64, 128, 32, 10])."""
+        return {key: [list(bank) for bank in value] if isinstance(value, list) else value
+                for key, value in self.state.items()}
 
     def _optimizer(self, gradients) -> None:
         """Adam / SGD in f64 (training.rs:924-979)."""
