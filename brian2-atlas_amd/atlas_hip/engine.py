@@ -1805,6 +1805,11 @@ def allocate(plan: Plan) -> None:
                 records[name] = values[path.order] if path.order is not None else values
             b["syn"] = plan.add(f"path{path.index}.synapses", max(4, records.nbytes),
                                 records.view(np.uint8) if records.nbytes else None)
+            if path.order is not None:
+                # the edge of each record, for the results' edge order
+                edges = path.order.astype(np.uint32)
+                b["syn_order"] = plan.add(f"path{path.index}.edge_of_row", max(4, edges.nbytes),
+                                          edges if edges.size else None)
     for path in plan.pathways:
         owner = path.state_owner
         if owner is not None:

@@ -147,7 +147,7 @@ class HipExecutor:
         # tables built once, and queue records (only read below their counters)
         static = (".param.", ".row_target", ".segment", ".slots", ".monitor_entries", ".monitor_offsets",
                   ".queue_records", ".queue_scratch", ".generator_offsets", ".generator_ticks", ".records",
-                  ".pending", ".refractory_table", "clock_table")
+                  ".pending", ".refractory_table", "clock_table", ".edge_of_row")
         return not any(part in name for part in static)
 
     def _build_topologies(self) -> None:
@@ -293,72 +293,92 @@ class HipExecutor:
 
     def _collect(self, steps: int) -> dict:
         plan = self.plan
+        # every small array of the results in one read: requests first, then the arrays by key
+        requests = {}
+
+        def ask(key, buffer: int, dtype, count: int, offset: int = 0) -> None:
+            requests[key] = (buffer, dtype, count, offset)
+
+        for pop in plan.populations:
+            b, p = pop.buffers, pop.index
+            # with several clocks each population has advanced its own clock's ticks
+            end_tick = plan.end_tick(pop, steps)
+            ran = end_tick > pop.start_tick
+            rows = max(0, end_tick - pop.window_start)
+            for name, dtype, _ in pop.states:
+                ask((p, "state", name), b[f"state:{name}"], NUMPY[dtype], pop.count)
+            if pop.has_spike_event and ran:
+                slot = (end_tick - 1) % pop.ring
+                ask((p, "cnt"), b["spk_cnt"], np.uint32, pop.blocks, slot * pop.blocks * 4)
+                ask((p, "ids"), b["spk_ids"], np.uint32, pop.count, slot * pop.count * 4)
+            if "mon_entries" in b:
+                for name in pop.monitor_vars:
+                    ask((p, "trace", name), b[f"sample:{name}"], NUMPY[engine._var_dtype(pop, name)],
+                        rows * len(pop.monitor_record))
+            if pop.refractory is not None:
+                ask((p, "lastspike"), b["lastspike"], np.float64, pop.count)
+                if ran:
+                    ask((p, "until"), b["until"], np.int32, pop.count)
+        if plan.pathways:
+            ask("delivered", plan.delivered_buffer, np.uint64, plan.buffers[plan.delivered_buffer].nbytes // 8)
+        got = dict(zip(requests, self.sim.read_many(list(requests.values()))))
         populations = []
         for pop in plan.populations:
-            b = pop.buffers
-            # with several clocks each population has advanced its own clock's ticks
+            b, p = pop.buffers, pop.index
             end_tick = plan.end_tick(pop, steps)
             last_tick = end_tick - 1
             ran = end_tick > pop.start_tick
-            states = {name: self.sim.read(b[f"state:{name}"], NUMPY[dtype], pop.count)
-                      for name, dtype, _ in pop.states}
+            states = {name: got[p, "state", name] for name, _, _ in pop.states}
             rows = max(0, end_tick - pop.window_start)
             if pop.has_spike_event and rows:
-                pairs = self.sim.extract_spikes(b["rec"], rows, b["rec_words"], pop.count)
-                ticks_ = pairs[:, 0] + pop.window_start
-                idx = pairs[:, 1]
+                ticks_, idx, fired = self.sim.spikes(b["rec"], rows, b["rec_words"], pop.count, pop.window_start)
             else:
                 ticks_ = np.zeros(0, np.int64)
                 idx = np.zeros(0, np.int64)
+                fired = np.zeros(pop.count, np.int64)
             if not self.lift_recording_budget and len(ticks_) > RECORDING_BUDGET:
                 raise RuntimeError("event stream recording budget exceeded")
             if pop.spike_monitor:
                 spike_ticks, indices = ticks_, idx
-                counts = np.bincount(idx, minlength=pop.count).astype(np.int64)
+                counts = fired
             else:
                 spike_ticks = indices = np.zeros(0, np.int64)
                 counts = np.zeros(pop.count, np.int64)
             last_spikes = np.zeros(0, np.int64)
-            if pop.has_spike_event and ran:
-                slot = last_tick % pop.ring
-                n_by_block = self.sim.read(b["spk_cnt"], np.uint32, pop.blocks, offset=slot * pop.blocks * 4)
-                ids = self.sim.read(b["spk_ids"], np.uint32, pop.count, offset=slot * pop.count * 4)
+            if (p, "cnt") in got:
+                n_by_block, ids = got[p, "cnt"], got[p, "ids"]
                 if self.launch_mode == "persistent":
                     ids &= RING_VALUE   # persistent launches stamp ring words with their tick
                 last_spikes = np.concatenate(
                     [ids[k * plan.shape.block:k * plan.shape.block + int(n)] for k, n in enumerate(n_by_block)]
                 ).astype(np.int64) if pop.blocks else last_spikes
             trace = {}
-            if "mon_entries" in b:
-                for name in pop.monitor_vars:
-                    dtype = engine._var_dtype(pop, name)
-                    trace[name] = self.sim.read(b[f"sample:{name}"], NUMPY[dtype],
-                                                rows * len(pop.monitor_record)).reshape(rows, len(pop.monitor_record))
-            else:
-                for name in pop.monitor_vars:
+            for name in pop.monitor_vars:
+                if "mon_entries" in b:
+                    trace[name] = got[p, "trace", name].reshape(rows, len(pop.monitor_record))
+                else:
                     trace[name] = np.zeros((rows, len(pop.monitor_record)), NUMPY[engine._var_dtype(pop, name)])
             refractory = None
             if pop.refractory is not None:
                 if ran:
-                    until = self.sim.read(b["until"], np.int32, pop.count)
-                    available = until.astype(np.int64) <= last_tick
+                    available = got[p, "until"] <= last_tick
                 else:
                     available = pop.refractory[2].astype(bool)
-                refractory = {"lastspike": self.sim.read(b["lastspike"], np.float64, pop.count),
-                              "not_refractory": available}
+                refractory = {"lastspike": got[p, "lastspike"], "not_refractory": available}
             streams = {"spike": {"ticks": ticks_, "indices": idx}} if pop.has_spike_event else {}
             for k, (event, _, _) in enumerate(pop.custom_events):
                 # a custom event's stream: its bitmap rows over the recording window, like the spikes
-                pairs = (self.sim.extract_spikes(b[f"evrec:{k}"], rows, b["rec_words"], pop.count) if rows
-                         else np.zeros((0, 2), np.int64))
-                if not self.lift_recording_budget and len(pairs) > RECORDING_BUDGET:
+                event_ticks, event_idx, _ = (
+                    self.sim.spikes(b[f"evrec:{k}"], rows, b["rec_words"], pop.count, pop.window_start) if rows
+                    else (np.zeros(0, np.int64), np.zeros(0, np.int64), None))
+                if not self.lift_recording_budget and len(event_ticks) > RECORDING_BUDGET:
                     raise RuntimeError("event stream recording budget exceeded")
-                streams[event] = {"ticks": pairs[:, 0] + pop.window_start, "indices": pairs[:, 1]}
+                streams[event] = {"ticks": event_ticks, "indices": event_idx}
             populations.append({"states": states, "trace": trace, "spike_ticks": spike_ticks, "indices": indices,
                                 "counts": counts, "last_spikes": last_spikes, "refractory": refractory,
                                 "event_streams": streams,
                                 "event_monitors": self._event_monitors(pop)})
-        delivered = self.sim.read(plan.delivered_buffer, np.uint64).reshape(-1, plan.total_blocks) \
+        delivered = got["delivered"].reshape(-1, plan.total_blocks) \
             if plan.pathways else np.zeros((0, max(1, plan.total_blocks)), np.uint64)
         synapses = [{"states": {}, "events": 0, "edges": plan.synapse_edges[s]} for s in range(plan.synapse_count)]
         for post in plan.post_paths:
@@ -368,19 +388,11 @@ class HipExecutor:
             entry["events"] += int(delivered[path.index].sum())
             if path.state_owner is not None:   # its states are the owner pathway's records
                 continue
-            records = None
-            if path.syn_states and path.edge_count:
-                records = self.sim.read(path.buffers["syn"], np.uint8, path.edge_count * path.syn_stride) \
-                    .view(engine.syn_record_dtype(path))
             for name, dtype, _ in path.syn_states:
-                rows_values = np.ascontiguousarray(records[name]) if records is not None \
-                    else np.zeros(0, NUMPY[dtype])
-                if path.order is not None:
-                    edge_values = np.empty_like(rows_values)
-                    edge_values[path.order] = rows_values
-                else:
-                    edge_values = rows_values
-                entry["states"][name] = edge_values
+                # edge order, field by field, from the records in row order
+                entry["states"][name] = self.sim.read_field(
+                    path.buffers["syn"], path.syn_stride, path.syn_fields[name][0], NUMPY[dtype], path.edge_count,
+                    path.buffers.get("syn_order")) if path.edge_count else np.zeros(0, NUMPY[dtype])
         return {"populations": populations, "synapses": synapses}
 
     def _event_monitors(self, pop) -> dict:

@@ -67,10 +67,16 @@ class SlotTable(ctypes.Structure):
                 ("xcds", ctypes.c_uint64), ("row_slots", ctypes.c_uint32)]
 
 
+class Read(ctypes.Structure):
+    _fields_ = [("buffer", ctypes.c_uint32), ("offset", ctypes.c_uint64), ("host", ctypes.c_void_p),
+                ("bytes", ctypes.c_uint64)]
+
+
 EXPORTS = ["atlas_sim_create", "atlas_sim_destroy", "atlas_sim_alloc", "atlas_sim_upload", "atlas_sim_read",
            "atlas_sim_zero", "atlas_sim_copy", "atlas_sim_compile", "atlas_sim_set_schedule", "atlas_sim_run",
            "atlas_sim_fixed_indegree", "atlas_sim_build_slots", "atlas_sim_extract_spikes", "atlas_sim_set_profiling",
            "atlas_sim_kernel_time", "atlas_sim_set_epilogue", "atlas_sim_device_name", "atlas_sim_set_persistent",
+           "atlas_sim_spikes_count", "atlas_sim_spikes_read", "atlas_sim_read_many", "atlas_sim_read_field",
            "atlas_prepare_fixed_indegree", "atlas_prepare_fixed_total", "atlas_prepare_initializer"]
 
 _lib = None
@@ -101,6 +107,10 @@ def library() -> ctypes.CDLL:
     lib.atlas_sim_fixed_indegree.argtypes = [vp, ctypes.POINTER(FixedIndegree), *e]
     lib.atlas_sim_build_slots.argtypes = [vp, ctypes.POINTER(SlotTable), ctypes.POINTER(u32), *e]
     lib.atlas_sim_extract_spikes.argtypes = [vp, u32, u64, u64, u64, vp, u64, ctypes.POINTER(u64), *e]
+    lib.atlas_sim_spikes_count.argtypes = [vp, u32, u64, u64, ctypes.POINTER(u64), *e]
+    lib.atlas_sim_spikes_read.argtypes = [vp, u32, u64, u64, u64, i64, vp, vp, vp, u64, *e]
+    lib.atlas_sim_read_many.argtypes = [vp, ctypes.POINTER(Read), u32, *e]
+    lib.atlas_sim_read_field.argtypes = [vp, u32, u64, u64, u32, i64, u64, vp, *e]
     lib.atlas_sim_set_profiling.argtypes = [vp, ctypes.c_int, *e]
     lib.atlas_sim_kernel_time.argtypes = [vp, u32, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(u64), *e]
     lib.atlas_sim_device_name.argtypes = [vp, ctypes.c_char_p, ctypes.c_size_t, *e]
@@ -280,6 +290,32 @@ class Sim:
             self._call("atlas_sim_extract_spikes", buffer, rows, words, neurons,
                        pairs.ctypes.data_as(ctypes.c_void_p), count.value, ctypes.byref(count))
         return pairs
+
+    def read_many(self, requests: list) -> list[np.ndarray]:
+        """Arrays of (buffer, dtype, count, offset) requests, read together."""
+        out = [np.empty(count, dtype) for _, dtype, count, _ in requests]
+        reads = (Read * len(requests))(*[Read(buffer, offset, array.ctypes.data, array.nbytes)
+                                         for (buffer, _, _, offset), array in zip(requests, out)])
+        self._call("atlas_sim_read_many", reads, len(requests))
+        return out
+
+    def read_field(self, records: int, stride: int, offset: int, dtype, count: int, order: int | None) -> np.ndarray:
+        """One field of `count` records, at the positions the u32 buffer `order` gives (None: in place)."""
+        out = np.empty(count, dtype)
+        if count:
+            self._call("atlas_sim_read_field", records, stride, offset, out.itemsize, -1 if order is None else order,
+                       count, out.ctypes.data)
+        return out
+
+    def spikes(self, buffer: int, rows: int, words: int, neurons: int, first_tick: int):
+        """(ticks, neurons, spikes per neuron) of a recording bitmap whose first row is `first_tick`."""
+        total = ctypes.c_uint64()
+        self._call("atlas_sim_spikes_count", buffer, rows, words, ctypes.byref(total))
+        ticks, indices = np.empty(total.value, np.int64), np.empty(total.value, np.int64)
+        counts = np.empty(neurons, np.int64)
+        self._call("atlas_sim_spikes_read", buffer, rows, words, neurons, first_tick, ticks.ctypes.data,
+                   indices.ctypes.data, counts.ctypes.data, total.value)
+        return ticks, indices, counts
 
     def set_profiling(self, enabled: bool) -> None:
         self._call("atlas_sim_set_profiling", 1 if enabled else 0)

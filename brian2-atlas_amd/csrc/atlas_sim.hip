@@ -40,6 +40,12 @@ struct AtlasSim {
     uint32_t persistent_barrier = 0;   // buffer zeroed before each persistent launch
     bool persistent_plain = false;     // ordinary launches (residency checked by occupancy) instead of cooperative
     bool profiling = false;
+    // device workspace and pinned staging of the result reads, grown as needed, freed with the handle
+    void* work = nullptr;
+    u64 work_bytes = 0;
+    unsigned char* staging = nullptr;
+    u64 spikes_total = 0, spikes_rows = 0;   // atlas_sim_spikes_count's, for atlas_sim_spikes_read
+    uint32_t spikes_buffer = 0;
     std::vector<double> kernel_ms;
     std::vector<u64> kernel_launches;
 };
@@ -267,53 +273,140 @@ __global__ void slot_kernel(const u32* __restrict__ segment, const u32* __restri
 }
 
 // --------------------------------------------------------- spike decoding
-__global__ void bitmap_row_counts(const u32* __restrict__ bits, u64 rows, u64 words,
-                                  u32* __restrict__ counts) {
-    __shared__ u32 partial[256];
-    const u64 row = blockIdx.x;
-    if (row >= rows) return;
-    u32 c = 0;
-    for (u64 w = threadIdx.x; w < words; w += 256) c += __popc(bits[row * words + w]);
-    partial[threadIdx.x] = c;
-    __syncthreads();
-    for (u32 s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) partial[threadIdx.x] += partial[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) counts[row] = partial[0];
+// One workgroup of 256 per recorded tick throughout: a row of the bitmap is read coalesced, and
+// spikes are sparse (config 3: 775 in 31,250 words a tick), so the rows' scans bound it.
+__device__ __forceinline__ u32 wave_sum(u32 v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
 }
 
-__global__ void bitmap_row_pairs(const u32* __restrict__ bits, u64 rows, u64 words, u64 neurons,
-                                 const u64* __restrict__ row_start, long long* __restrict__ pairs) {
-    __shared__ u32 scan[257];
+__global__ void __launch_bounds__(256) bitmap_row_counts(const u32* __restrict__ bits, u64 rows, u64 words,
+                                                         u32* __restrict__ counts) {
+    __shared__ u32 partial[4];
     const u64 row = blockIdx.x;
-    if (row >= rows) return;
-    u64 base = row_start[row];
-    for (u64 w0 = 0; w0 < words; w0 += 256) {
-        const u64 w = w0 + threadIdx.x;
-        const u32 word = w < words ? bits[row * words + w] : 0u;
-        scan[threadIdx.x + 1] = __popc(word);
-        if (threadIdx.x == 0) scan[0] = 0;
-        __syncthreads();
-        if (threadIdx.x == 0)
-            for (u32 k = 1; k <= 256; ++k) scan[k] += scan[k - 1];
-        __syncthreads();
-        u64 out = base + scan[threadIdx.x];
-        u32 bitsleft = word;
-        while (bitsleft) {
-            const u32 b = __ffs(bitsleft) - 1;
-            bitsleft &= bitsleft - 1;
-            const u64 neuron = w * 32 + b;
-            if (neuron < neurons) {
-                pairs[2 * out] = (long long)row;
-                pairs[2 * out + 1] = (long long)neuron;
-            }
-            ++out;
+    u32 c = 0;
+    for (u64 w = threadIdx.x; w < words; w += 256) c += __popc(bits[row * words + w]);
+    c = wave_sum(c);
+    if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) counts[row] = partial[0] + partial[1] + partial[2] + partial[3];
+}
+
+// starts[r] = the spikes of the rows before r; starts[rows] = all of them.  One workgroup.
+__global__ void __launch_bounds__(1024) row_starts(const u32* __restrict__ counts, u64 rows, u64* __restrict__ starts) {
+    __shared__ u64 sums[16];
+    const u32 lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    u64 base = 0;
+    for (u64 r0 = 0; r0 < rows; r0 += 1024) {
+        const u64 r = r0 + threadIdx.x;
+        const u64 mine = r < rows ? counts[r] : 0u;
+        u64 x = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const u64 y = __shfl_up(x, off, 64);
+            if (lane >= (u32)off) x += y;
         }
-        base += scan[256];
+        if (lane == 63) sums[wave] = x;
+        __syncthreads();
+        u64 before = base, total = 0;
+        for (u32 w = 0; w < 16; ++w) {
+            if (w < wave) before += sums[w];
+            total += sums[w];
+        }
+        if (r < rows) starts[r] = before + x - mine;
+        base += total;
         __syncthreads();
     }
+    if (threadIdx.x == 0) starts[rows] = base;
 }
+
+// The spikes of each row, neurons ascending, from position starts[row]: to_spike(position, row, neuron).
+template <class ToSpike>
+__device__ __forceinline__ void row_spikes(const u32* __restrict__ bits, u64 words, u64 neurons,
+                                           const u64* __restrict__ starts, const ToSpike& to_spike) {
+    __shared__ u32 sums[2][4];
+    const u32 lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const u64 row = blockIdx.x;
+    u64 base = starts[row];
+    u32 odd = 0;
+    for (u64 w0 = 0; w0 < words; w0 += 256, odd ^= 1u) {
+        const u64 w = w0 + threadIdx.x;
+        u32 word = w < words ? bits[row * words + w] : 0u;
+        const u32 mine = __popc(word);
+        u32 x = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const u32 y = __shfl_up(x, off, 64);
+            if (lane >= (u32)off) x += y;
+        }
+        if (lane == 63) sums[odd][wave] = x;
+        __syncthreads();   // the sums of the other parity are read a tile later, past the next barrier
+        u64 out = base + x - mine;
+        for (u32 k = 0; k < 4; ++k) {
+            if (k < wave) out += sums[odd][k];
+            base += sums[odd][k];
+        }
+        while (word) {
+            const u64 neuron = w * 32 + (__ffs(word) - 1);
+            word &= word - 1;
+            if (neuron < neurons) to_spike(out, row, neuron);
+            ++out;
+        }
+    }
+}
+
+__global__ void __launch_bounds__(256) bitmap_row_pairs(const u32* __restrict__ bits, u64 words, u64 neurons,
+                                                        const u64* __restrict__ starts, long long* __restrict__ pairs) {
+    row_spikes(bits, words, neurons, starts, [&](u64 at, u64 row, u64 neuron) {
+        pairs[2 * at] = (long long)row;
+        pairs[2 * at + 1] = (long long)neuron;
+    });
+}
+
+// The same into one array per column, rows counted from first_tick, with the spikes per neuron (into
+// zeroed counts): the arrays the caller returns, where pairs cost it two strided copies and a
+// histogram on the host (all of a run's results, 1.5M spikes of 1M neurons: 8.8 -> 4.1 ms, of which
+// the copies to pageable memory are most; 100 spikes of 500 neurons 0.32 -> 0.18).
+__global__ void __launch_bounds__(256) bitmap_row_columns(const u32* __restrict__ bits, u64 words, u64 neurons,
+                                                          const u64* __restrict__ starts, long long first_tick,
+                                                          long long* __restrict__ ticks, long long* __restrict__ indices,
+                                                          u64* __restrict__ counts) {
+    row_spikes(bits, words, neurons, starts, [&](u64 at, u64 row, u64 neuron) {
+        ticks[at] = first_tick + (long long)row;
+        indices[at] = (long long)neuron;
+        atomicAdd(&counts[neuron], 1ull);
+    });
+}
+
+// out[order[row]] (or out[row]) = the T at byte `offset` of record `row`: scattered 4- and 8-byte stores,
+// against a permutation on the host after copying whole records (1.3M plastic synapses of 32
+// bytes, four fields: 20 -> 2.3 ms with the rest of the results).
+template <class T>
+__global__ void gather_field(const unsigned char* __restrict__ records, u64 stride, u64 offset,
+                             const u32* __restrict__ order, u64 count, T* __restrict__ out) {
+    for (u64 r = (u64)blockIdx.x * blockDim.x + threadIdx.x; r < count; r += (u64)gridDim.x * blockDim.x)
+        out[order ? order[r] : r] = *reinterpret_cast<const T*>(records + r * stride + offset);
+}
+
+// The handle's device workspace of at least `bytes` (its contents are lost when it grows).
+int workspace(AtlasSim* sim, u64 bytes, char* err, size_t cap) {
+    if (bytes <= sim->work_bytes) return ATLAS_OK;
+    if (sim->work) {
+        HIP_TRY(hipStreamSynchronize(sim->stream), ATLAS_E_KERNEL);
+        HIP_TRY(hipFree(sim->work), ATLAS_E_ALLOC);
+        sim->work = nullptr;
+        sim->work_bytes = 0;
+    }
+    const u64 grown = bytes + bytes / 4;
+    HIP_TRY(hipMalloc(&sim->work, grown), ATLAS_E_ALLOC);
+    sim->work_bytes = grown;
+    return ATLAS_OK;
+}
+
+constexpr u64 STAGING_BYTES = 1ull << 20;   // pinned; small reads share one wait through it
+
+u64 aligned(u64 bytes) { return (bytes + 255) / 256 * 256; }
 
 int upload_table(AtlasSim* sim, char* err, size_t cap) {
     if (!sim->table_dirty) return ATLAS_OK;
@@ -369,6 +462,8 @@ void atlas_sim_destroy(AtlasSim* sim) {
     for (void* p : sim->buffers)
         if (p) (void)hipFree(p);
     if (sim->table) (void)hipFree(sim->table);
+    if (sim->work) (void)hipFree(sim->work);
+    if (sim->staging) (void)hipHostFree(sim->staging);
     (void)hipStreamDestroy(sim->stream);
     delete sim;
 }
@@ -794,6 +889,24 @@ int atlas_sim_build_slots(AtlasSim* sim, const AtlasSlotTable* spec, uint32_t* m
     return ATLAS_OK;
 }
 
+namespace {
+// The spikes of each of the bitmap's rows counted and scanned into the row starts at the workspace's
+// beginning; *total receives all of them.
+int count_rows(AtlasSim* sim, const u32* bits, u64 rows, u64 words, uint64_t* total, char* err, size_t cap) {
+    const u64 starts_bytes = aligned((rows + 1) * 8);
+    if (int rc = workspace(sim, starts_bytes + aligned(rows * 4), err, cap)) return rc;
+    unsigned char* work = static_cast<unsigned char*>(sim->work);
+    u32* counts = reinterpret_cast<u32*>(work + starts_bytes);
+    u64* starts = reinterpret_cast<u64*>(work);
+    hipLaunchKernelGGL(bitmap_row_counts, dim3((u32)rows), dim3(256), 0, sim->stream, bits, rows, words, counts);
+    hipLaunchKernelGGL(row_starts, dim3(1), dim3(1024), 0, sim->stream, counts, rows, starts);
+    HIP_TRY(hipGetLastError(), ATLAS_E_KERNEL);
+    HIP_TRY(hipMemcpyAsync(total, starts + rows, 8, hipMemcpyDeviceToHost, sim->stream), ATLAS_E_READBACK);
+    HIP_TRY(hipStreamSynchronize(sim->stream), ATLAS_E_KERNEL);
+    return ATLAS_OK;
+}
+}  // namespace
+
 int atlas_sim_extract_spikes(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t rows, uint64_t words,
                              uint64_t neurons, int64_t* pairs_host, uint64_t capacity, uint64_t* count,
                              char* err, size_t cap) {
@@ -801,42 +914,149 @@ int atlas_sim_extract_spikes(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t row
         return fail(err, cap, ATLAS_E_HOST, "invalid spike bitmap arguments");
     HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
     *count = 0;
+    sim->spikes_total = sim->spikes_rows = 0;   // the workspace is this call's
     if (!rows) return ATLAS_OK;
     const u32* bits = static_cast<const u32*>(sim->buffers[bitmap_buffer]);
-    u32* counts = nullptr;
-    u64* starts = nullptr;
-    long long* pairs = nullptr;
-    HIP_TRY(hipMalloc(&counts, rows * 4), ATLAS_E_ALLOC);
-    hipLaunchKernelGGL(bitmap_row_counts, dim3((u32)rows), dim3(256), 0, sim->stream, bits, rows, words, counts);
-    std::vector<u32> host_counts(rows);
-    hipError_t e = hipStreamSynchronize(sim->stream);
-    if (e == hipSuccess) e = hipMemcpy(host_counts.data(), counts, rows * 4, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) {
-        (void)hipFree(counts);
-        return fail(err, cap, ATLAS_E_KERNEL, "spike counts: %s", hipGetErrorString(e));
-    }
-    std::vector<u64> host_starts(rows);
-    u64 total = 0;
-    for (u64 r = 0; r < rows; ++r) {
-        host_starts[r] = total;
-        total += host_counts[r];
-    }
-    *count = total;
+    if (int rc = count_rows(sim, bits, rows, words, count, err, cap)) return rc;
+    const u64 total = *count;
     if (total && pairs_host && capacity >= total) {
-        e = hipMalloc(&starts, rows * 8);
-        if (e == hipSuccess) e = hipMalloc(&pairs, total * 16);
-        if (e == hipSuccess) e = hipMemcpy(starts, host_starts.data(), rows * 8, hipMemcpyHostToDevice);
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(bitmap_row_pairs, dim3((u32)rows), dim3(256), 0, sim->stream, bits, rows, words,
-                               neurons, starts, pairs);
-            e = hipStreamSynchronize(sim->stream);
+        // the row starts stay below the pairs
+        const u64 starts_bytes = aligned((rows + 1) * 8), counts_bytes = aligned(rows * 4);
+        if (starts_bytes + counts_bytes + total * 16 > sim->work_bytes) {
+            if (int rc = workspace(sim, starts_bytes + counts_bytes + total * 16, err, cap)) return rc;
+            if (int rc = count_rows(sim, bits, rows, words, count, err, cap)) return rc;
         }
-        if (e == hipSuccess) e = hipMemcpy(pairs_host, pairs, total * 16, hipMemcpyDeviceToHost);
+        unsigned char* work = static_cast<unsigned char*>(sim->work);
+        long long* pairs = reinterpret_cast<long long*>(work + starts_bytes + counts_bytes);
+        hipLaunchKernelGGL(bitmap_row_pairs, dim3((u32)rows), dim3(256), 0, sim->stream, bits, words, neurons,
+                           reinterpret_cast<const u64*>(work), pairs);
+        HIP_TRY(hipGetLastError(), ATLAS_E_KERNEL);
+        HIP_TRY(hipStreamSynchronize(sim->stream), ATLAS_E_KERNEL);
+        HIP_TRY(hipMemcpy(pairs_host, pairs, total * 16, hipMemcpyDeviceToHost), ATLAS_E_READBACK);
     }
-    (void)hipFree(counts);
-    if (starts) (void)hipFree(starts);
-    if (pairs) (void)hipFree(pairs);
-    if (e != hipSuccess) return fail(err, cap, ATLAS_E_KERNEL, "spike pairs: %s", hipGetErrorString(e));
+    return ATLAS_OK;
+}
+
+int atlas_sim_spikes_count(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t rows, uint64_t words, uint64_t* count,
+                           char* err, size_t cap) {
+    if (!sim || bitmap_buffer >= sim->buffers.size() || sim->sizes[bitmap_buffer] < rows * words * 4 || !count ||
+        rows > 0x7FFFFFFFull)
+        return fail(err, cap, ATLAS_E_HOST, "invalid spike bitmap arguments");
+    HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
+    *count = 0;
+    sim->spikes_buffer = bitmap_buffer;
+    sim->spikes_rows = rows;
+    sim->spikes_total = 0;
+    if (!rows) return ATLAS_OK;
+    if (int rc = count_rows(sim, static_cast<const u32*>(sim->buffers[bitmap_buffer]), rows, words, count, err, cap))
+        return rc;
+    sim->spikes_total = *count;
+    return ATLAS_OK;
+}
+
+int atlas_sim_spikes_read(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t rows, uint64_t words, uint64_t neurons,
+                          int64_t first_tick, int64_t* ticks, int64_t* indices, int64_t* counts, uint64_t total,
+                          char* err, size_t cap) {
+    if (!sim || !counts || (total && (!ticks || !indices)) || bitmap_buffer != sim->spikes_buffer ||
+        rows != sim->spikes_rows || total != sim->spikes_total || bitmap_buffer >= sim->buffers.size() ||
+        sim->sizes[bitmap_buffer] < rows * words * 4)
+        return fail(err, cap, ATLAS_E_HOST, "the spikes of this bitmap have not been counted");
+    HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
+    if (!total) {
+        memset(counts, 0, neurons * 8);
+        return ATLAS_OK;
+    }
+    const u32* bits = static_cast<const u32*>(sim->buffers[bitmap_buffer]);
+    const u64 at_ticks = aligned((rows + 1) * 8) + aligned(rows * 4), at_indices = at_ticks + aligned(total * 8);
+    const u64 at_counts = at_indices + aligned(total * 8), bytes = at_counts + neurons * 8;
+    if (bytes > sim->work_bytes) {
+        uint64_t again = 0;
+        if (int rc = workspace(sim, bytes, err, cap)) return rc;
+        if (int rc = count_rows(sim, bits, rows, words, &again, err, cap)) return rc;
+        if (again != total) return fail(err, cap, ATLAS_E_HOST, "the spike bitmap changed between count and read");
+    }
+    unsigned char* work = static_cast<unsigned char*>(sim->work);
+    if (int rc = zero_range(sim, work + at_counts, neurons * 8, err, cap)) return rc;
+    hipLaunchKernelGGL(bitmap_row_columns, dim3((u32)rows), dim3(256), 0, sim->stream, bits, words, neurons,
+                       reinterpret_cast<const u64*>(work), (long long)first_tick,
+                       reinterpret_cast<long long*>(work + at_ticks), reinterpret_cast<long long*>(work + at_indices),
+                       reinterpret_cast<u64*>(work + at_counts));
+    HIP_TRY(hipGetLastError(), ATLAS_E_KERNEL);
+    HIP_TRY(hipMemcpyAsync(ticks, work + at_ticks, total * 8, hipMemcpyDeviceToHost, sim->stream), ATLAS_E_READBACK);
+    HIP_TRY(hipMemcpyAsync(indices, work + at_indices, total * 8, hipMemcpyDeviceToHost, sim->stream), ATLAS_E_READBACK);
+    HIP_TRY(hipMemcpyAsync(counts, work + at_counts, neurons * 8, hipMemcpyDeviceToHost, sim->stream), ATLAS_E_READBACK);
+    HIP_TRY(hipStreamSynchronize(sim->stream), ATLAS_E_KERNEL);
+    return ATLAS_OK;
+}
+
+int atlas_sim_read_many(AtlasSim* sim, const AtlasRead* reads, uint32_t count, char* err, size_t cap) {
+    if (!sim || (count && !reads)) return fail(err, cap, ATLAS_E_HOST, "null argument");
+    for (uint32_t k = 0; k < count; ++k)
+        if (reads[k].buffer >= sim->buffers.size() || reads[k].offset + reads[k].bytes > sim->sizes[reads[k].buffer] ||
+            (reads[k].bytes && !reads[k].host))
+            return fail(err, cap, ATLAS_E_HOST, "read outside buffer %u", reads[k].buffer);
+    HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
+    if (!sim->staging) {
+        void* p = nullptr;
+        HIP_TRY(hipHostMalloc(&p, STAGING_BYTES, hipHostMallocDefault), ATLAS_E_ALLOC);
+        sim->staging = static_cast<unsigned char*>(p);
+    }
+    // reads that fit the staging go there together; one wait, then to the caller's memory.  A larger
+    // one goes straight to it.
+    u64 used = 0;
+    uint32_t first = 0;
+    auto flush = [&](uint32_t end) -> int {
+        HIP_TRY(hipStreamSynchronize(sim->stream), ATLAS_E_KERNEL);
+        u64 at = 0;
+        for (uint32_t k = first; k < end; ++k) {
+            if (reads[k].bytes > STAGING_BYTES / 4) continue;
+            memcpy(reads[k].host, sim->staging + at, reads[k].bytes);
+            at += aligned(reads[k].bytes);
+        }
+        used = 0;
+        first = end;
+        return ATLAS_OK;
+    };
+    for (uint32_t k = 0; k < count; ++k) {
+        const AtlasRead& r = reads[k];
+        if (!r.bytes) continue;
+        const char* from = static_cast<char*>(sim->buffers[r.buffer]) + r.offset;
+        if (r.bytes > STAGING_BYTES / 4) {
+            HIP_TRY(hipMemcpyAsync(r.host, from, r.bytes, hipMemcpyDeviceToHost, sim->stream), ATLAS_E_READBACK);
+            continue;
+        }
+        if (used + aligned(r.bytes) > STAGING_BYTES)
+            if (int rc = flush(k)) return rc;
+        HIP_TRY(hipMemcpyAsync(sim->staging + used, from, r.bytes, hipMemcpyDeviceToHost, sim->stream), ATLAS_E_READBACK);
+        used += aligned(r.bytes);
+    }
+    return flush(count);
+}
+
+int atlas_sim_read_field(AtlasSim* sim, uint32_t records, uint64_t stride, uint64_t offset, uint32_t itemsize,
+                         int64_t order, uint64_t count, void* host, char* err, size_t cap) {
+    if (!sim || records >= sim->buffers.size() || (itemsize != 1 && itemsize != 4 && itemsize != 8) ||
+        offset + itemsize > stride || offset % itemsize || stride % itemsize || sim->sizes[records] < count * stride ||
+        order >= (int64_t)sim->buffers.size() || (order >= 0 && sim->sizes[order] < count * 4) || (count && !host))
+        return fail(err, cap, ATLAS_E_HOST, "invalid record field");
+    if (!count) return ATLAS_OK;
+    HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
+    if (int rc = workspace(sim, count * itemsize, err, cap)) return rc;
+    const unsigned char* from = static_cast<const unsigned char*>(sim->buffers[records]);
+    const u32* rows = order >= 0 ? static_cast<const u32*>(sim->buffers[order]) : nullptr;
+    const dim3 grid((u32)std::min<u64>((count + 255) / 256, 65536)), block(256);
+    if (itemsize == 8)
+        hipLaunchKernelGGL(gather_field<u64>, grid, block, 0, sim->stream, from, stride, offset, rows, count,
+                           static_cast<u64*>(sim->work));
+    else if (itemsize == 4)
+        hipLaunchKernelGGL(gather_field<u32>, grid, block, 0, sim->stream, from, stride, offset, rows, count,
+                           static_cast<u32*>(sim->work));
+    else
+        hipLaunchKernelGGL(gather_field<unsigned char>, grid, block, 0, sim->stream, from, stride, offset, rows, count,
+                           static_cast<unsigned char*>(sim->work));
+    HIP_TRY(hipGetLastError(), ATLAS_E_KERNEL);
+    HIP_TRY(hipMemcpyAsync(host, sim->work, count * itemsize, hipMemcpyDeviceToHost, sim->stream), ATLAS_E_READBACK);
+    HIP_TRY(hipStreamSynchronize(sim->stream), ATLAS_E_KERNEL);
     return ATLAS_OK;
 }
 

@@ -167,6 +167,30 @@ int atlas_sim_extract_spikes(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t row
                              uint64_t neurons, int64_t* pairs_host, uint64_t capacity,
                              uint64_t* count, char* err, size_t cap);
 
+/* The same as one array per column, in two calls: the spikes counted (into *count), then read by the
+ * next call on the handle, of the same bitmap and `total`: ticks (row + first_tick) and neurons of
+ * every spike, and the spikes of each of the `neurons` neurons. */
+int atlas_sim_spikes_count(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t rows, uint64_t words, uint64_t* count,
+                           char* err, size_t cap);
+int atlas_sim_spikes_read(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t rows, uint64_t words, uint64_t neurons,
+                          int64_t first_tick, int64_t* ticks, int64_t* indices, int64_t* counts, uint64_t total,
+                          char* err, size_t cap);
+
+/* `count` reads as atlas_sim_read's, the small ones with one wait for all of them. */
+typedef struct AtlasRead {
+    uint32_t buffer;
+    uint64_t offset;
+    void* host;
+    uint64_t bytes;
+} AtlasRead;
+int atlas_sim_read_many(AtlasSim* sim, const AtlasRead* reads, uint32_t count, char* err, size_t cap);
+
+/* One field of the first `count` records of a buffer (itemsize 1, 4 or 8 bytes at byte `offset` of every
+ * `stride`) as a contiguous array: element order[r] is record r's, with `order` a buffer of u32 that is a
+ * permutation of the records (negative: element r is record r's). */
+int atlas_sim_read_field(AtlasSim* sim, uint32_t records, uint64_t stride, uint64_t offset, uint32_t itemsize,
+                         int64_t order, uint64_t count, void* host, char* err, size_t cap);
+
 /* Procedural projections materialised on the host (no device, no handle), as the reference
  * prepares them for its GPU engines (brian2_rust/gpu_initialization.py prepare_model,
  * "rust-host-f64-v0"): the engine lowers them as explicit topologies.  Outputs are caller-owned.

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import nets
-from atlas_hip import engine, models
+from atlas_hip import engine, models, native
 from atlas_hip.executor import HipExecutor
 from atlas_hip.results import read_results, write_events, write_results
 from oracle import oracle
@@ -992,3 +992,59 @@ def test_run_regularly_cuba_matches_oracle(end, delay, monkeypatch):
     assert_same_dump(ex.document, dump, expected.results)
     assert events == expected.events
     assert expected.spike_count > 1000
+
+
+@pytest.mark.parametrize("rows,words,neurons,density", [(1, 1, 1, 1.0), (3, 2, 33, 0.5), (1025, 8, 256, 0.02),
+                                                        (7, 257, 8200, 0.3), (2048, 16, 500, 0.0), (1023, 300, 9600, 0.01)])
+def test_spike_bitmap_decoding(rows, words, neurons, density):
+    """The recording bitmap as (tick, neuron) columns with the spikes per neuron, and as pairs, at the
+    edges of the kernels' tiles (256 words, 1024 rows): equal to NumPy's decoding."""
+    print(f"case: bitmap {rows} x {words} words, {neurons} neurons, density {density}", flush=True)
+    rng = np.random.default_rng(rows + words)
+    fired = rng.random((rows, neurons)) < density
+    bits = np.zeros((rows, words * 32), bool)
+    bits[:, :neurons] = fired
+    packed = np.packbits(bits, axis=1, bitorder="little").view(np.uint32)
+    sim = native.Sim(0)
+    try:
+        buffer = sim.alloc(packed.nbytes, packed)
+        want = np.argwhere(fired)
+        for _ in range(2):   # the workspace grown, then reused
+            ticks, indices, counts = sim.spikes(buffer, rows, words, neurons, 17)
+            assert np.array_equal(ticks, want[:, 0] + 17) and np.array_equal(indices, want[:, 1])
+            assert np.array_equal(counts, fired.sum(axis=0))
+            assert np.array_equal(sim.extract_spikes(buffer, rows, words, neurons), want)
+        with pytest.raises(native.NativeError):   # another total than counted
+            sim._call("atlas_sim_spikes_read", buffer, rows, words, neurons, 0, None, None, counts.ctypes.data, 1)
+    finally:
+        sim.close()
+
+
+def test_read_many_and_fields():
+    """Several reads with one wait (past the staging's size, empty ones among them) and a record field at
+    permuted positions, against the arrays they were uploaded from."""
+    rng = np.random.default_rng(3)
+    arrays = [rng.integers(0, 255, n).astype(np.uint8) for n in (5, 300_000, 1, 250_000, 262_144, 262_145, 200_000, 260_000, 77)]
+    records = np.zeros(1000, np.dtype([("t", "f8"), ("w", "f4"), ("b", "u1"), ("pad", "u1", 3)]))
+    records["t"], records["w"], records["b"] = rng.random(1000), rng.random(1000), rng.integers(0, 2, 1000)
+    order = rng.permutation(1000).astype(np.uint32)
+    sim = native.Sim(0)
+    try:
+        ids = [sim.alloc(a.nbytes, a) for a in arrays]
+        got = sim.read_many([(k, np.uint8, a.size, 0) for k, a in zip(ids, arrays)] + [(ids[0], np.uint8, 0, 0),
+                                                                                    (ids[8], np.uint8, 70, 7)])
+        assert all(np.array_equal(g, a) for g, a in zip(got, arrays)) and np.array_equal(got[-1], arrays[8][7:])
+        assert sim.read_many([]) == []
+        rec, perm = sim.alloc(records.nbytes, records), sim.alloc(order.nbytes, order)
+        for name in ("t", "w", "b"):
+            offset = records.dtype.fields[name][1]
+            assert np.array_equal(sim.read_field(rec, 16, offset, records[name].dtype, 1000, None), records[name])
+            want = np.empty_like(records[name])
+            want[order] = records[name]
+            assert np.array_equal(sim.read_field(rec, 16, offset, records[name].dtype, 1000, perm), want)
+        with pytest.raises(native.NativeError):
+            sim.read_many([(ids[0], np.uint8, 6, 0)])
+        with pytest.raises(native.NativeError):
+            sim.read_field(rec, 16, 12, np.float64, 1000, None)
+    finally:
+        sim.close()
