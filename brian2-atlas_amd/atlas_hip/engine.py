@@ -4275,10 +4275,13 @@ def generate(plan: Plan, header_text: str) -> None:
         kernels = [("atlas_tick", multi_body())]
     else:
         kernels = [("atlas_tick", body(True, True))]
+    # a persistent plan compiles its run kernel alone (RUN_ONLY) until it falls back to these
+    parts.append("#ifndef ATLAS_RUN_ONLY")
     for name, lines in kernels:
         parts.append(f'extern "C" __global__ void __launch_bounds__({WG}) {name}(const u64* __restrict__ tab, i64 tick) {{')
         parts.extend(lines)
         parts.append("}")
+    parts.append("#endif")
     plan.persistent = None
     # the split loop: a fitted plan that it takes, or one population's only group of a delay >= 1
     xwaves = SPLIT_XWAVES or WG // 128
@@ -4339,5 +4342,6 @@ def generate(plan: Plan, header_text: str) -> None:
         plan.launches.append((1, padded, WG, 0))
 
 
+RUN_ONLY = "-DATLAS_RUN_ONLY"   # compile option: the persistent launch's kernel alone
 COMPILE_OPTIONS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off", "-fno-fast-math",
                    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

@@ -103,7 +103,7 @@ class HipExecutor:
         self._compile()
         self.compile_seconds = time.perf_counter() - lowered
         self.setup_seconds = lowered - started
-        self.compilation_report = dict(requested=compile_reuse, kernels_compiled=len(self.plan.kernels),
+        self.compilation_report = dict(requested=compile_reuse, kernels_compiled=len(self.kernels),
                                        kernels_reused=0, source_bytes=len(self.plan.source),
                                        compiler_options=list(engine.COMPILE_OPTIONS))
         self.device_name = self.sim.device_name()
@@ -111,19 +111,36 @@ class HipExecutor:
         self._fresh = True
 
     def _compile(self) -> None:
-        """Compile the plan's module and set its launches: the per-tick schedule and epilogue, and
-        the persistent launch when the plan has one and persistent launches are enabled."""
-        self.sim.compile(self.plan.source, self.plan.kernels, engine.COMPILE_OPTIONS)
-        self.sim.set_schedule(self.plan.launches)
-        self.sim.set_epilogue(self.plan.epilogue)
-        try:
-            self.sim.set_persistent(self.plan.persistent if self.persistent else None, self.plan.barrier_buffer,
-                                    engine.PERSISTENT_TICKS, plain=self.plain_launches)
-        except native.NativeError as error:
-            if error.code != native.COOPERATIVE:
-                raise
-            self.persistent = False   # the grid cannot be resident at once: one launch per tick
-            self.sim.set_persistent(None)
+        """Compile what the plan's runs launch: the persistent launch's kernel where the plan has one and
+        persistent launches are enabled (the per-tick kernels, half or more of the compilation, only
+        when a run falls back to them), else the per-tick kernels with their schedule and epilogue."""
+        if self.persistent and self.plan.persistent is not None:
+            _, grid, items, lds = self.plan.persistent
+            self.kernels = ["atlas_run"]
+            self.sim.compile(self.plan.source, self.kernels, engine.COMPILE_OPTIONS + [engine.RUN_ONLY])
+            self.sim.set_schedule([])
+            self.sim.set_epilogue([])
+            try:
+                self.sim.set_persistent((0, grid, items, lds), self.plan.barrier_buffer, engine.PERSISTENT_TICKS,
+                                        plain=self.plain_launches)
+                return
+            except native.NativeError as error:
+                if error.code != native.COOPERATIVE:
+                    raise
+                self.persistent = False   # the grid cannot be resident at once: one launch per tick
+        self.kernels = [name for name in self.plan.kernels if name != "atlas_run"]
+        self.sim.compile(self.plan.source, self.kernels, engine.COMPILE_OPTIONS)
+        # the launches name plan.kernels
+        at = {k: self.kernels.index(name) for k, name in enumerate(self.plan.kernels) if name in self.kernels}
+        self.sim.set_schedule([(at[k], *shape) for k, *shape in self.plan.launches])
+        self.sim.set_epilogue([(at[k], *shape) for k, *shape in self.plan.epilogue])
+        self.sim.set_persistent(None)
+
+    def _fall_back(self) -> None:
+        """One launch per tick for the rest of the executor's life, from the initial snapshot."""
+        self.persistent = False
+        self._compile()
+        self.reset()
 
     @property
     def launch_mode(self) -> str:
@@ -137,9 +154,7 @@ class HipExecutor:
         except native.NativeError as error:
             if error.code != native.COOPERATIVE:
                 raise
-        self.persistent = False
-        self.sim.set_persistent(None)
-        self.reset()
+        self._fall_back()
         return self.sim.run(self.plan.start_tick, steps)
 
     @staticmethod
@@ -241,16 +256,16 @@ class HipExecutor:
             # a tick listed more events into one block than its LDS holds (events were dropped):
             # replay with one launch per tick, whose ordered delivery stages events in windows,
             # for the rest of the executor's life
-            self.persistent = False
-            self.sim.set_persistent(None)
-            self.reset()
+            self._fall_back()
             stats = self._run_ticks(steps)
             fault = self.sim.read(plan.fault_buffer, np.uint32, 4)
         if fault[0] & RING_STALL:
             raise RuntimeError("a persistent launch's wait for the spike ring timed out; its results are invalid")
         command_seconds = time.perf_counter() - command_started
         self.last_stats = stats
-        self.kernel_times = {name: self.sim.kernel_time(k) for k, name in enumerate(plan.kernels)} if profile else {}
+        # (milliseconds, launches) of every kernel of the plan, none for those that are not compiled
+        self.kernel_times = {name: self.sim.kernel_time(self.kernels.index(name)) if name in self.kernels else (0.0, 0)
+                             for name in plan.kernels} if profile else {}
         if fault[0]:
             reasons = []
             if fault[0] & 1:
