@@ -643,6 +643,8 @@ class Plan:
     clock_buffer: int = -1
     edge_nodes: int = 0                              # events the split loop's edge buckets hold per workgroup and tick
     fitted: bool = False                             # fit_shape chose the shape of its persistent launches
+    # the update as slices, one per replica of a block's neurons: [(statements, states), ...] (update_slices)
+    slices: list | None = None
 
     @property
     def multi_clock(self) -> bool:
@@ -2110,11 +2112,6 @@ def _population_code(plan: Plan, pop: PopulationPlan) -> str:
     else:
         L.append("    __device__ static int until_next(const u64* __restrict__ tab, i64 tick) "
                  "{ (void)tab; (void)tick; return 0; }")
-    L.append("    __device__ static bool step(const u64* __restrict__ tab, u32 i, double t, i64 tick, State& st, "
-             "u32& fault, int until_next) {")
-    L.append("        (void)tick; (void)fault; (void)t; (void)until_next;")
-    if pop.refractory is not None:
-        L.append("        bool nr = tick >= (i64)st.until;")
     state_in = lambda n, dt: f"(double)st.st_{n}"  # noqa: E731
     written = set()
 
@@ -2132,20 +2129,6 @@ def _population_code(plan: Plan, pop: PopulationPlan) -> str:
                 dtype = next(s_[1] for s_ in pop.states if s_[0] == name)
                 L.append(f"        st.st_{name} = {commit_expr(dtype, prog.symbols[name][0])};")
                 written.add(name)
-
-    regular_in_step("pre", "ra")
-    if pop.update is not None:
-        env = _scalar_env(pop, pop.update)
-        inputs = _with_scalars(_population_inputs(pop, state_in), env, pop.update)
-        prog = DeviceProgram(inputs, L, "u", rng=(plan.rng_seed, "i"))
-        prog.scalar_statements(env)
-        prog.statements(pop.update["vector"])
-        for name in pop.update["effects"]["writes"]:
-            require(name in {s_[0] for s_ in pop.states}, f"update writes {name!r}")
-            dtype = next(s_[1] for s_ in pop.states if s_[0] == name)
-            L.append(f"        st.st_{name} = {commit_expr(dtype, prog.symbols[name][0])};")
-            written.add(name)
-    regular_in_step("mid", "rb")
 
     def monitor_record(k: int, variables: list, value_of, indent: str) -> None:
         # EventMonitor k: one record (tick, neuron, the monitored values as f64) appended
@@ -2167,62 +2150,118 @@ def _population_code(plan: Plan, pop: PopulationPlan) -> str:
             return hexlit(pop.scalar_params[name][1])
         return f"atlas::buf<const double>(tab, {b['param:' + name]})[i]"
 
-    # custom events: each condition on the updated states (before any reset), its flag for the
-    # resets slot, and the EventMonitors recording it at the threshold
-    for k, (event, threshold_code, _) in enumerate(pop.custom_events):
-        prog = DeviceProgram(_population_inputs(pop, state_in), L, f"ce{k}_", rng=(plan.rng_seed, "i"))
-        prog.statements(threshold_code["vector"])
-        L.append(f"        const bool event{k} = {prog.symbols['_cond'][0]} != 0.0;")
-        L.append(f"        atlas::buf<byte_t>(tab, {b[f'evt:{k}']})[i] = event{k} ? (byte_t)1 : (byte_t)0;")
-        mons = [(m, variables) for m, (_, variables, ev, when) in enumerate(pop.event_monitors)
-                if ev == event and when == "thresholds"]
-        if mons:
-            L.append(f"        if (event{k}) {{")
-            for m, variables in mons:
-                monitor_record(m, variables, register_value, "            ")
-            L.append("        }")
-    fired = "false"
-    if pop.generator is not None:
-        # the neuron fires when its next scheduled tick is this one (ticks lie inside the run)
-        L.append("        const bool fired = st.next == (u32)tick;")
-        L.append("        if (fired) ++st.cursor;")
-        fired = "fired"
-    if pop.threshold is not None:
-        prog = DeviceProgram(_population_inputs(pop, state_in), L, "h", rng=(plan.rng_seed, "i"))
-        prog.statements(pop.threshold["vector"])
-        cond = prog.symbols["_cond"][0]
-        gate = " && nr" if pop.refractory is not None else ""
-        L.append(f"        const bool fired = ({cond} != 0.0){gate};")
-        fired = "fired"
-        L.append("        if (fired) {")
-        for k, (_, variables, event, when) in enumerate(pop.event_monitors):
-            # EventMonitor: the neuron's monitored values at the threshold, before the reset
-            if event == "spike" and when == "thresholds":
-                monitor_record(k, variables, register_value, "            ")
+    def update_in_step(statements: list, names: list, prefix: str, indent: str = "        ") -> None:
+        env = _scalar_env(pop, pop.update)
+        inputs = _with_scalars(_population_inputs(pop, state_in), env, pop.update)
+        prog = DeviceProgram(inputs, L, prefix, indent=indent, rng=(plan.rng_seed, "i"))
+        prog.scalar_statements(env)
+        prog.statements(statements)
+        for name in names:
+            require(name in {s_[0] for s_ in pop.states}, f"update writes {name!r}")
+            dtype = next(s_[1] for s_ in pop.states if s_[0] == name)
+            L.append(f"{indent}st.st_{name} = {commit_expr(dtype, prog.symbols[name][0])};")
+            written.add(name)
+
+    slices = plan.slices if pop.index == 0 else None
+    if slices:
+        # the update split over the block's replicas (atlas_tick.h ATLAS_REPL): each computes its slice's
+        # states into LDS, then every replica takes all of them from there
+        offsets = _exchange_offsets(plan)
+        L.append("    __device__ static void update_slice(const u64* __restrict__ tab, u32 i, u32 j, double t, i64 tick, "
+                 "State& st, u32& fault, u32 slice, byte_t* exch) {")
+        L.append("        (void)tab; (void)tick; (void)fault; (void)t; (void)i;")
         if pop.refractory is not None:
-            period = pop.refractory[0]
-            L.append(f"            __builtin_nontemporal_store(t, atlas::buf<double>(tab, {b['lastspike']}) + i);")
-            if "until_table" in b:
-                L.append("            st.until = until_next;")
-            else:
-                L.append(f"            st.until = (int)atlas::refractory_until(tick, t, {hexlit(pop.dt)}, "
-                         f"{hexlit(pop.dt)}, {period}ull, fault);")
-            L.append(f"            __builtin_nontemporal_store(st.until, atlas::buf<int>(tab, {b['until']}) + i);")
-            L.append("            nr = false;")
-        if pop.reset is not None and pop.reset_fused:
-            env = _scalar_env(pop, pop.reset)
-            inputs = _with_scalars(_population_inputs(pop, state_in), env, pop.reset)
-            prog = DeviceProgram(inputs, L, "z", indent="            ", rng=(plan.rng_seed, "i"))
-            prog.scalar_statements(env)
-            prog.statements(pop.reset["vector"])
-            for name in pop.reset["effects"]["writes"]:
-                require(name in {s_[0] for s_ in pop.states}, f"reset writes {name!r}")
+            L.append("        const bool nr = tick >= (i64)st.until;")
+        for k, (statements, names) in enumerate(slices):
+            L.append(f"        if (slice == {k}u) {{")
+            update_in_step(statements, names, f"us{k}_", "            ")
+            for name in names:
                 dtype = next(s_[1] for s_ in pop.states if s_[0] == name)
-                L.append(f"            st.st_{name} = {commit_expr(dtype, prog.symbols[name][0])};")
-                written.add(name)
-        L.append("        }")
-    L.append(f"        return {fired};")
-    L.append("    }")
+                L.append(f"            reinterpret_cast<{CTYPE[dtype]}*>(exch + {offsets[name]})[j] = st.st_{name};")
+            L.append("        }")
+        L.append("    }")
+
+    def step_body(update: bool) -> None:
+        L.append("        (void)tick; (void)fault; (void)t; (void)until_next;")
+        if pop.refractory is not None:
+            L.append("        bool nr = tick >= (i64)st.until;")
+        regular_in_step("pre", "ra")
+        if pop.update is not None and update:
+            update_in_step(pop.update["vector"], pop.update["effects"]["writes"], "u")
+        elif not update:
+            for name, offset in offsets.items():
+                dtype = next(s_[1] for s_ in pop.states if s_[0] == name)
+                L.append(f"        st.st_{name} = reinterpret_cast<const {CTYPE[dtype]}*>(exch + {offset})[j];")
+        regular_in_step("mid", "rb")
+        events_in_step()
+
+    def events_in_step() -> None:
+        """The custom events and the threshold on the updated states, with the fused reset."""
+
+        # custom events: each condition on the updated states (before any reset), its flag for the
+        # resets slot, and the EventMonitors recording it at the threshold
+        for k, (event, threshold_code, _) in enumerate(pop.custom_events):
+            prog = DeviceProgram(_population_inputs(pop, state_in), L, f"ce{k}_", rng=(plan.rng_seed, "i"))
+            prog.statements(threshold_code["vector"])
+            L.append(f"        const bool event{k} = {prog.symbols['_cond'][0]} != 0.0;")
+            L.append(f"        atlas::buf<byte_t>(tab, {b[f'evt:{k}']})[i] = event{k} ? (byte_t)1 : (byte_t)0;")
+            mons = [(m, variables) for m, (_, variables, ev, when) in enumerate(pop.event_monitors)
+                    if ev == event and when == "thresholds"]
+            if mons:
+                L.append(f"        if (event{k}) {{")
+                for m, variables in mons:
+                    monitor_record(m, variables, register_value, "            ")
+                L.append("        }")
+        fired = "false"
+        if pop.generator is not None:
+            # the neuron fires when its next scheduled tick is this one (ticks lie inside the run)
+            L.append("        const bool fired = st.next == (u32)tick;")
+            L.append("        if (fired) ++st.cursor;")
+            fired = "fired"
+        if pop.threshold is not None:
+            prog = DeviceProgram(_population_inputs(pop, state_in), L, "h", rng=(plan.rng_seed, "i"))
+            prog.statements(pop.threshold["vector"])
+            cond = prog.symbols["_cond"][0]
+            gate = " && nr" if pop.refractory is not None else ""
+            L.append(f"        const bool fired = ({cond} != 0.0){gate};")
+            fired = "fired"
+            L.append("        if (fired) {")
+            for k, (_, variables, event, when) in enumerate(pop.event_monitors):
+                # EventMonitor: the neuron's monitored values at the threshold, before the reset
+                if event == "spike" and when == "thresholds":
+                    monitor_record(k, variables, register_value, "            ")
+            if pop.refractory is not None:
+                period = pop.refractory[0]
+                L.append(f"            __builtin_nontemporal_store(t, atlas::buf<double>(tab, {b['lastspike']}) + i);")
+                if "until_table" in b:
+                    L.append("            st.until = until_next;")
+                else:
+                    L.append(f"            st.until = (int)atlas::refractory_until(tick, t, {hexlit(pop.dt)}, "
+                             f"{hexlit(pop.dt)}, {period}ull, fault);")
+                L.append(f"            __builtin_nontemporal_store(st.until, atlas::buf<int>(tab, {b['until']}) + i);")
+                L.append("            nr = false;")
+            if pop.reset is not None and pop.reset_fused:
+                env = _scalar_env(pop, pop.reset)
+                inputs = _with_scalars(_population_inputs(pop, state_in), env, pop.reset)
+                prog = DeviceProgram(inputs, L, "z", indent="            ", rng=(plan.rng_seed, "i"))
+                prog.scalar_statements(env)
+                prog.statements(pop.reset["vector"])
+                for name in pop.reset["effects"]["writes"]:
+                    require(name in {s_[0] for s_ in pop.states}, f"reset writes {name!r}")
+                    dtype = next(s_[1] for s_ in pop.states if s_[0] == name)
+                    L.append(f"            st.st_{name} = {commit_expr(dtype, prog.symbols[name][0])};")
+                    written.add(name)
+            L.append("        }")
+        L.append(f"        return {fired};")
+        L.append("    }")
+
+    L.append("    __device__ static bool step(const u64* __restrict__ tab, u32 i, double t, i64 tick, State& st, "
+             "u32& fault, int until_next) {")
+    step_body(True)
+    if slices:
+        L.append("    __device__ static bool finish_slices(const u64* __restrict__ tab, u32 i, u32 j, double t, i64 tick, "
+                 "State& st, u32& fault, int until_next, const byte_t* exch) {")
+        step_body(False)
     L.append("    __device__ static void store(const u64* __restrict__ tab, u32 i, u32 j, const State& st, "
              "byte_t* post) {")
     L.append("        (void)tab; (void)i; (void)j; (void)st; (void)post;")
@@ -2648,15 +2687,68 @@ OP_COST = {**dict.fromkeys(("exp", "expm1", "exprel", "log", "rand", "randn", "p
            **dict.fromkeys(("load", "literal", "boolean", "integer", "f32_to_f64", "f64_to_f32"), 0)}
 
 
+def _value_ops(value) -> int:
+    """Arithmetic operations of a statement or expression."""
+    if isinstance(value, dict):
+        here = OP_COST.get(value["op"], 1) if "op" in value else 0
+        return here + sum(_value_ops(v) for v in value.values())
+    return sum(_value_ops(v) for v in value) if isinstance(value, list) else 0
+
+
 def _update_ops(pop: PopulationPlan) -> int:
     """Arithmetic operations of one neuron's tick, refractoriness and recording aside."""
-    def ops(value) -> int:
-        if isinstance(value, dict):
-            here = OP_COST.get(value["op"], 1) if "op" in value else 0
-            return here + sum(ops(v) for v in value.values())
-        return sum(ops(v) for v in value) if isinstance(value, list) else 0
     codes = [code for code in (pop.update, pop.threshold) if code is not None] + [code for code, _ in pop.regular]
-    return sum(ops(code["vector"]) for code in codes)
+    return sum(_value_ops(code["vector"]) for code in codes)
+
+
+SLICES = 4            # replicas of a block's neurons that share a heavy update
+SLICED_BLOCK = 64     # neurons per block then: one wave per replica
+
+
+def update_slices(pop: PopulationPlan) -> list | None:
+    """The update's statements split into SLICES parts that run side by side, each with the states it
+    writes: a part holds the statements its states need, in order, and every statement is in one part
+    at least (their finiteness checks).  None where the heaviest part is more than half of the update or
+    run_regularly code runs beside it."""
+    if pop.update is None or any(where != "end" for _, where in pop.regular):
+        return None
+    statements = pop.update["vector"]
+    cost = [_value_ops(statement) for statement in statements]
+
+    def needed(names) -> set:
+        live, keep = set(names), set()
+        for k in range(len(statements) - 1, -1, -1):
+            if statements[k]["target"] in live:
+                keep.add(k)
+                if statements[k].get("condition") is None:
+                    live.discard(statements[k]["target"])
+                live |= _statement_reads(statements[k])
+        return keep
+
+    weigh = lambda keep: sum(cost[k] for k in keep)  # noqa: E731
+    parts = [[set(), []] for _ in range(SLICES)]
+    for name in sorted(pop.update["effects"]["writes"], key=lambda n: -weigh(needed([n]))):
+        part = min(parts, key=lambda p: weigh(p[0] | needed([name])))
+        part[0] |= needed([name])
+        part[1].append(name)
+    rest = set(range(len(statements))) - set().union(*(p[0] for p in parts))
+    if rest:   # read by no state: checked all the same, with what they read
+        parts[-1][0] |= needed([statements[k]["target"] for k in rest]) | rest
+    if 2 * max(weigh(p[0]) for p in parts) > sum(cost) or not all(names for _, names in parts):
+        return None
+    return [([statements[k] for k in sorted(keep)], names) for keep, names in parts]
+
+
+def _exchange_offsets(plan: Plan) -> dict:
+    """Byte offset of each sliced state's values in the block's LDS exchange, widest states first."""
+    pop = plan.populations[0]
+    sizes = {name: np.dtype(NUMPY[dtype]).itemsize for name, dtype, _ in pop.states}
+    names = sorted((name for _, names in plan.slices or [] for name in names), key=lambda name: -sizes[name])
+    return {name: plan.shape.block * sum(sizes[before] for before in names[:k]) for k, name in enumerate(names)}
+
+
+def _exchange_bytes(plan: Plan) -> int:
+    return plan.shape.block * 8 * len(_exchange_offsets(plan))
 
 
 def fit_shape(plan: Plan) -> bool:
@@ -2680,6 +2772,12 @@ def fit_shape(plan: Plan) -> bool:
         ring = 2 * groups[0][0].dvals[0] + 2 + (1 if plan.split else 0)
         if ring > RING_SLOTS:
             return False
+        # a heavy update is shared by several replicas of smaller blocks, one workgroup per CU
+        pop = plan.populations[0]
+        if _update_ops(pop) > HEAVY_OPS and -(-pop.count // SLICED_BLOCK) <= CUS:
+            plan.slices = update_slices(pop)
+            if plan.slices:
+                shape = Shape(SLICED_BLOCK, SLICED_BLOCK, 4, 10)
     else:
         return False
     plan.fitted = True
@@ -3921,7 +4019,12 @@ def generate(plan: Plan, header_text: str) -> None:
         hist = max(hist, offset)
     syn_bytes = max([_split_bytes(plan, g) or _prefetch_bytes(plan, g) for k, g in enumerate(groups)
                      if not counting[k]] + [0])
-    parts = [f"#define ATLAS_BLOCK {BLOCK}", f"#define ATLAS_WG {WG}", f"#define ATLAS_HIST {hist}",
+    # a persistent launch with a sliced update runs SLICES work-items per neuron
+    run_wg = WG * (SLICES if plan.slices else 1)
+    parts = [f"#define ATLAS_BLOCK {BLOCK}",
+             f"#ifdef ATLAS_RUN_ONLY\n#define ATLAS_WG {run_wg}\n#define ATLAS_REPL {run_wg // WG}\n#else\n"
+             f"#define ATLAS_WG {WG}\n#endif" if plan.slices else f"#define ATLAS_WG {WG}",
+             f"#define ATLAS_EXCH_BYTES {_exchange_bytes(plan)}", f"#define ATLAS_HIST {hist}",
              f"#define ATLAS_SYN_BYTES {syn_bytes}", f"#define ATLAS_TSTART {BLOCK + 1 if any(queued) else 1}",
              f"#define ATLAS_CAP_BITS {CAP_BITS}", f"#define ATLAS_MAX_NB {max_nb}", f"#define ATLAS_MAX_GNB {max_gnb}",
              f"#define ATLAS_MAX_NP {max_np}", f"#define ATLAS_SPT {SPT}", f"#define ATLAS_POST_BYTES {post_bytes}",
@@ -4318,12 +4421,12 @@ def generate(plan: Plan, header_text: str) -> None:
         # every workgroup must be resident at once: the waves per SIMD the grid needs (two 512-wide
         # workgroups per CU for 489 blocks of 2048: 4, at most 128 VGPRs; one 1024-wide for 245 of 4096:
         # 4; one 256-wide for configs 1 and 2: 1, so config 2's HH update keeps its values in registers)
-        waves = max(1, -(-plan.total_blocks // CUS) * (WG // 64) // 4)
-        parts.append(f'extern "C" __global__ void __launch_bounds__({WG}) __attribute__((amdgpu_waves_per_eu({waves}))) '
+        waves = max(1, -(-plan.total_blocks // CUS) * (run_wg // 64) // 4)
+        parts.append(f'extern "C" __global__ void __launch_bounds__(ATLAS_WG) __attribute__((amdgpu_waves_per_eu({waves}))) '
                      "atlas_run(const u64* __restrict__ tab, i64 tick0, i64 ticks) {")
         parts.extend(persistent_body())
         parts.append("}")
-        plan.persistent = (len(kernels), padded, WG, 0)
+        plan.persistent = (len(kernels), padded, run_wg, 0)
         kernels.append(("atlas_run", []))
     # synapse state updates and summed variables, each its own launch before the tick kernel,
     # in schedule order

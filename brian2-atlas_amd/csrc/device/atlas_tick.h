@@ -54,8 +54,16 @@ typedef long long i64;
 typedef unsigned short u16;
 typedef unsigned char byte_t;
 
+// Work-items per neuron of a persistent launch (persistent_run): the replicas of a heavy update
+#ifndef ATLAS_REPL
+#define ATLAS_REPL 1
+#endif
+#ifndef ATLAS_EXCH_BYTES
+#define ATLAS_EXCH_BYTES 0
+#endif
+
 #define ATLAS_WAVES (ATLAS_WG / 64)
-#define ATLAS_ROUNDS (ATLAS_BLOCK / ATLAS_WG)
+#define ATLAS_ROUNDS (ATLAS_BLOCK * ATLAS_REPL / ATLAS_WG)
 #define ATLAS_CAP (1u << ATLAS_CAP_BITS)
 #define ATLAS_PASS (ATLAS_WG * ATLAS_SPT)
 #define ATLAS_BATCH 8   // independent edges per work-item whose memory operations are issued together
@@ -117,6 +125,7 @@ struct Lds {
     u64 ev_sort[ATLAS_TSTART > 1 ? ATLAS_CAP : 1];   // bucketed sort keys of queued events
     alignas(16) byte_t post[ATLAS_POST_BYTES > 0 ? ATLAS_POST_BYTES : 16];
     alignas(16) byte_t syn[ATLAS_SYN_BYTES > 0 ? ATLAS_SYN_BYTES : 16];   // staged per-edge values
+    alignas(16) byte_t exch[ATLAS_EXCH_BYTES > 0 ? ATLAS_EXCH_BYTES : 16];   // sliced updates' states
 };
 
 // Workgroup barrier ordering LDS only.  Inside the tick every thread touches global
@@ -583,7 +592,7 @@ __device__ void flush(const u64* __restrict__ tab, i64 tick, double t, u32 blk, 
     }
     for (u32 k = threadIdx.x; k < nbuf; k += ATLAS_WG) atomicAdd(&s.hist[s.ev_tgt[k]], 1u);
     lds_barrier();
-    constexpr u32 PER = ATLAS_BLOCK / ATLAS_WG;
+    constexpr u32 PER = ATLAS_ROUNDS;
     u32 local = 0;
 #pragma unroll
     for (u32 q = 0; q < PER; ++q) local += s.hist[threadIdx.x * PER + q];
@@ -677,7 +686,7 @@ __device__ void flush(const u64* __restrict__ tab, i64 tick, double t, u32 blk, 
 // times.  On exit the counters are zero.
 template <class Group>
 __device__ void apply_counts(const u64* __restrict__ tab, i64 tick, double t, u32 blk, Lds& s) {
-    constexpr u32 PER = ATLAS_BLOCK / ATLAS_WG;
+    constexpr u32 PER = ATLAS_ROUNDS;
     constexpr u32 HB = Group::HIST_BASE;
     u32 fault = 0;
 #pragma unroll
@@ -1191,6 +1200,13 @@ __device__ void deliver(const u64* __restrict__ tab, i64 tick, double t, u32 blk
 //   5. each work-item applies its neurons' counts (Fused::apply) in registers and clears them.
 // Equal to one launch per tick bit for bit: the same programs in the same order per neuron.
 //
+// A heavy update (Hodgkin-Huxley: a dozen exponentials) is one long dependent float64 chain at one wave
+// per SIMD, and small networks leave most CUs idle.  With ATLAS_REPL replicas, blocks of 64 neurons run
+// on four waves that all hold the block's states: each computes one slice of the update (the statements
+// some of the states need), the states meet in LDS, and the threshold, the counting and the apply go on
+// in every replica alike.  COBAHH of 4000 neurons: 9.0 -> 5.8 us per tick at delay 0, 12.3 -> 4.9 at
+// delay 1 (where the split loop gave each update work-item two neurons).
+//
 // With delay 0 the deliveries of tick t need every block's spikes of tick t, so the tick runs
 // U_t, the publication and arrival, then the barrier of tick t, the records, the list, the slot
 // loads, the counting and the apply.  A workgroup that has passed the barrier of tick t
@@ -1209,7 +1225,8 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
     // fired sources per work-item per pass: 1024 per pass (775 fire per tick in config 3; one
     // slot per work-item of a 1024-wide workgroup measured 0.3 us per tick faster than two)
     constexpr u32 SLOTS_PER = ATLAS_WG >= 1024 ? 1 : 2;
-    constexpr u32 LIST = ATLAS_BLOCK;     // fired sources kept in LDS (s.cursor)
+    constexpr u32 LIST = ATLAS_REPL > 1 ? ATLAS_CAP : ATLAS_BLOCK;   // fired sources kept in LDS
+    u32* fired_list = ATLAS_REPL > 1 ? s.ev_row : s.cursor;
     constexpr u32 PERB = (Group::SRC_NB + ATLAS_WG - 1) / ATLAS_WG;   // source blocks per work-item
     constexpr u32 PASS = SLOTS_PER * ATLAS_WG;
     constexpr u32 BAR_SLOTS = 2 * Group::gval_max + 2;   // more than the 2 d barriers a wait and an arrival span
@@ -1219,17 +1236,24 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
     static_assert(Pop::R == Group::SRC_R && Pop::R >= 2 * Group::gval_max + 2 && Pop::R < 4095u &&
                   Pop::R <= ATLAS_RING_PREV, "ring of 2 d + 2 ticks");
     static_assert(Pop::N <= ATLAS_RING_VALUE + 1u, "neuron indices fit a stamped word");
+    // the neurons' work-items: ATLAS_REPL replicas of LANES, each holding the states of every neuron of
+    // the block; the first publishes and stores them
+    constexpr u32 LANES = ATLAS_WG / ATLAS_REPL;
+    constexpr u32 PW = ATLAS_WAVES / ATLAS_REPL;   // waves of a replica
+    static_assert(LANES % 64 == 0 && (ATLAS_REPL == 1 || ATLAS_ROUNDS == 1), "whole waves per replica");
     const u32 base = blk * ATLAS_BLOCK;
     const u32 n = (Pop::N - base < ATLAS_BLOCK) ? Pop::N - base : ATLAS_BLOCK;
     const u32 lane = __lane_id();
     const u32 wave = threadIdx.x >> 6;
+    const u32 replica = ATLAS_REPL > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / LANES) : 0u;
+    const u32 neuron_lane = ATLAS_REPL > 1 ? threadIdx.x % LANES : threadIdx.x;
     const u32 delay = Group::gval(0);
     u32* bar = buf<u32>(tab, bar_buf);
     bool gave_up = false;
     typename Pop::State st[ATLAS_ROUNDS];
 #pragma unroll
     for (u32 r = 0; r < ATLAS_ROUNDS; ++r) {
-        const u32 j = r * ATLAS_WG + threadIdx.x;
+        const u32 j = r * LANES + neuron_lane;
         if (j < n) Pop::load(tab, base + j, st[r]);
     }
     for (u32 j = threadIdx.x; j < NP * ATLAS_BLOCK; j += ATLAS_WG) s.hist[HB + j] = 0;
@@ -1307,7 +1331,7 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
 #pragma unroll
                     for (u32 k = 0; k < ATLAS_REC_IDS; ++k)
                         if (r == k) id = record_word(rc[q], k + 1) & ATLAS_RING_VALUE;
-                    s.cursor[e] = id;
+                    fired_list[e] = id;
                 }
                 start += count;
             }
@@ -1331,7 +1355,7 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
                 const u32 e = x / ITEMS;
                 u32 id = 0xFFFFFFFFu;
                 if (e < fired_total) {
-                    if (e < LIST) id = s.cursor[e];
+                    if (e < LIST) id = fired_list[e];
                     if (e >= LIST || id == ATLAS_LIST_FETCH) {
                         // an id past a record's seventh, or past the LDS list (a synchronous burst):
                         // the source block is the last whose start is at or before e (binary
@@ -1394,13 +1418,24 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
         }
         // 1. U_t, under the first pass's slot loads
         u64 masks[ATLAS_ROUNDS];
+        if constexpr (ATLAS_REPL > 1) {
+            // each replica its slice of the update, the states then taken from LDS
+            if (neuron_lane < n)
+                Pop::update_slice(tab, base + neuron_lane, neuron_lane, t, tick, st[0], fault, replica, s.exch);
+            lds_barrier();
+        }
 #pragma unroll
         for (u32 r = 0; r < ATLAS_ROUNDS; ++r) {
-            const u32 j = r * ATLAS_WG + threadIdx.x;
+            const u32 j = r * LANES + neuron_lane;
             bool fired = false;
-            if (j < n) fired = Pop::step(tab, base + j, t, tick, st[r], fault, until_next);
+            if (j < n) {
+                if constexpr (ATLAS_REPL > 1)
+                    fired = Pop::finish_slices(tab, base + j, j, t, tick, st[r], fault, until_next, s.exch);
+                else
+                    fired = Pop::step(tab, base + j, t, tick, st[r], fault, until_next);
+            }
             masks[r] = __ballot(fired);
-            if (lane == 0) s.round_counts[r * ATLAS_WAVES + wave] = (u32)__popcll(masks[r]);
+            if (lane == 0 && replica == 0) s.round_counts[r * PW + wave] = (u32)__popcll(masks[r]);
         }
         lds_barrier();
         // the slot loads are waited for here, before the publication's stores: a store counts in
@@ -1417,8 +1452,8 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
             // each wave's position in the tick's ascending list, per round: the exclusive prefix of
             // the (round, wave) spike counts in round-major order, one count per lane and a wave scan
             // (a loop over the waves' counts per round measured 0.35 us per tick slower with 16 waves)
-            static_assert(ATLAS_ROUNDS * ATLAS_WAVES <= 64, "one (round, wave) count per lane");
-            const u32 c_ = lane < ATLAS_ROUNDS * ATLAS_WAVES ? s.round_counts[lane] : 0u;
+            static_assert(ATLAS_ROUNDS * PW <= 64, "one (round, wave) count per lane");
+            const u32 c_ = lane < ATLAS_ROUNDS * PW ? s.round_counts[lane] : 0u;
             u32 incl = c_;
 #pragma unroll
             for (int off = 1; off < 64; off <<= 1) {
@@ -1430,17 +1465,18 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
             const u32 wave_u = __builtin_amdgcn_readfirstlane(wave);
 #pragma unroll
             for (u32 r = 0; r < ATLAS_ROUNDS; ++r) {
-                const u32 mine = __builtin_amdgcn_readlane(excl, r * ATLAS_WAVES + wave_u);
+                if (replica != 0) break;
+                const u32 mine = __builtin_amdgcn_readlane(excl, r * PW + wave_u);
                 if ((masks[r] >> lane) & 1ull) {
                     const u32 kk = mine + (u32)__popcll(masks[r] & ((1ull << lane) - 1ull));
-                    const u32 word = ring_word(stamp, base + r * ATLAS_WG + threadIdx.x);
+                    const u32 word = ring_word(stamp, base + r * LANES + neuron_lane);
                     ring_store_u32(&ids[kk], word);
                     if (kk < ATLAS_REC_IDS) ring_store_u32(&rec[1 + kk], word);
                 }
-                if (recording && lane < 2 && r * ATLAS_WG + wave * 64 + lane * 32 < n) {
+                if (recording && lane < 2 && r * LANES + wave * 64 + lane * 32 < n) {
                     u32* bits = buf<u32>(tab, Pop::REC) + (u64)(tick - Pop::WIN0) * Pop::REC_WORDS;
                     __builtin_nontemporal_store((u32)(masks[r] >> (32 * lane)),
-                                                bits + (base + r * ATLAS_WG + wave * 64) / 32 + lane);
+                                                bits + (base + r * LANES + wave * 64) / 32 + lane);
                 }
             }
             // the words the slot's previous tick wrote past this tick's count (a block that fired
@@ -1478,20 +1514,26 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
         // 5. each neuron's counts applied to its updated states, then cleared
 #pragma unroll
         for (u32 r = 0; r < ATLAS_ROUNDS; ++r) {
-            const u32 j = r * ATLAS_WG + threadIdx.x;
+            const u32 j = r * LANES + neuron_lane;
             if (j < n) {
                 Fused::apply(tab, base + j, j, st[r], s, t, tick, fault);
+                if constexpr (ATLAS_REPL == 1) {
 #pragma unroll
-                for (u32 p = 0; p < NP; ++p) s.hist[HB + p * ATLAS_BLOCK + j] = 0;
+                    for (u32 p = 0; p < NP; ++p) s.hist[HB + p * ATLAS_BLOCK + j] = 0;
+                }
             }
+        }
+        if constexpr (ATLAS_REPL > 1) {   // cleared once every replica has read them
+            lds_barrier();
+            for (u32 j = threadIdx.x; j < NP * ATLAS_BLOCK; j += ATLAS_WG) s.hist[HB + j] = 0;
         }
         report(tab, Pop::FAULT, fault);
     }
     // end of launch: states and delivered counters back to memory
 #pragma unroll
     for (u32 r = 0; r < ATLAS_ROUNDS; ++r) {
-        const u32 j = r * ATLAS_WG + threadIdx.x;
-        if (j < n) Pop::store(tab, base + j, j, st[r], s.post);
+        const u32 j = r * LANES + neuron_lane;
+        if (j < n && replica == 0) Pop::store(tab, base + j, j, st[r], s.post);
     }
     // the launch's delivered events per pathway: wave sums through LDS (the list area is free once
     // the last tick is done), then one work-item per pathway
@@ -2287,7 +2329,7 @@ __device__ void take_counts(const u64* __restrict__ tab, i64 tick, u32 blk, u32 
     constexpr u32 HB = Group::HIST_BASE;
     constexpr u32 ROW = Group::NP * ATLAS_BLOCK;
     constexpr u32 PER = ROW / ATLAS_WG;
-    static_assert(ATLAS_BLOCK % ATLAS_WG == 0, "a block is whole rounds of work-items");
+    static_assert(ATLAS_BLOCK * ATLAS_REPL % ATLAS_WG == 0, "a block is whole rounds of work-items");
     if (threadIdx.x < Group::NP) s.delivered[threadIdx.x] = 0;
     gptr<u32> row = buf<u32>(tab, Group::ARR) + ((u64)(tick % Group::AR) * Group::TB + blk) * ROW;
     u32 c[PER];
@@ -2303,7 +2345,7 @@ __device__ void take_counts(const u64* __restrict__ tab, i64 tick, u32 blk, u32 
         const u32 k = q * ATLAS_WG + threadIdx.x;
         s.hist[HB + k] = c[q];
         if (c[q]) row[k] = 0u;
-        per_path[q / (ATLAS_BLOCK / ATLAS_WG)] += c[q];
+        per_path[q / ATLAS_ROUNDS] += c[q];
     }
 #pragma unroll
     for (u32 p = 0; p < Group::NP; ++p) {
@@ -2462,7 +2504,7 @@ template <class Group>
 __device__ void take_events(const u64* __restrict__ tab, i64 tick, double t, u32 blk, u32 wg_index, u32 wg_count,
                             Lds& s) {
     constexpr u32 PERE = ATLAS_CAP / ATLAS_WG;
-    constexpr u32 PER = ATLAS_BLOCK / ATLAS_WG;
+    constexpr u32 PER = ATLAS_ROUNDS;
     u32 fault = 0;
     const u64 q = (u64)(tick % Group::AR) * Group::TB + blk;
     gptr<u32> qcnt = buf<u32>(tab, Group::QCNT);

@@ -280,3 +280,18 @@ def test_split_loop_of_several_groups_and_populations_equals_the_oracle(monkeypa
     monkeypatch.setattr(engine, "PERSISTENT_TICKS", 37)
     dump, events, _ = run(doc, "persistent", monkeypatch, lift_recording_budget=True)
     assert dump == expected.results and events == expected.events
+
+
+@pytest.mark.parametrize("n,p,delay", [(64, 0.3, 0), (65, 0.3, 0), (1000, 0.05, 1), (2500, 0.03, 0)])
+def test_sliced_update_equals_the_oracle(monkeypatch, n, p, delay):
+    """COBAHH in blocks of 64 neurons whose update four replicas share: one block, a last block of one
+    neuron, both orders of a tick; equal to the oracle in one launch and in launches of 37 ticks."""
+    print(f"case: sliced COBAHH {n}, p {p}, delay {delay}", flush=True)
+    doc = models.cobahh_network(n, p=p, steps=600, delay_ticks=delay)
+    expected = oracle.run(doc)
+    assert expected.spike_count > 30
+    dump, events, result = run(doc, "persistent", monkeypatch)
+    assert dump == expected.results and events == expected.events
+    monkeypatch.setattr(engine, "PERSISTENT_TICKS", 37)
+    dump, events, _ = run(doc, "persistent", monkeypatch)
+    assert dump == expected.results and events == expected.events

@@ -811,7 +811,8 @@ def test_fit_shape_takes_the_smallest_block_the_network_fits(n, block):
 
 
 def test_fit_shape_keeps_other_plans():
-    for doc, fitted in ((models.cobahh_network(600, steps=5), True), (models.cuba_network(1100, p=0.02, steps=5), True), (models.cobahh_network(600, steps=5, delay_ticks=1), True),
+    for doc, fitted in ((models.cuba_network(1100, p=0.02, steps=5), True),
+                        (models.cobahh_network(64 * 256 + 1, p=0.0005, steps=5), True),   # too many small blocks
                         (models.cuba_network(600, p=0.02, steps=5, delay_ticks=40), False),
                         (models.generator_network(50, 200, spikes=100, indegree=10, steps=20), False),
                         (models.plastic_network(500, indegree=20, steps=5), False)):
@@ -842,3 +843,40 @@ def test_fitted_plans_of_several_groups_run_the_split_loop(doc, rings, readers):
     assert run.count("persistent_run_split<") == len(plan.populations)
     assert [name for name in ("Reader0", "Reader1") if name in run] == readers
     assert len(rtc.compile_source(plan.source, engine.COMPILE_OPTIONS)) > 1000
+
+
+@pytest.mark.parametrize("delay", [0, 1])
+def test_heavy_update_is_sliced(delay):
+    """COBAHH's update is split into four parts, {m}, {h}, {n} and {v, ge, gi}, each with the statements
+    its states need, in blocks of 64 neurons with four work-items per neuron; every statement is in
+    one part, and both modules compile."""
+    plan = engine.lower(models.cobahh_network(300, steps=5, delay_ticks=delay))
+    assert engine.fit_shape(plan)
+    assert sorted(sorted(names) for _, names in plan.slices) == [["ge", "gi", "v"], ["h"], ["m"], ["n"]]
+    vector = plan.populations[0].update["vector"]
+    assert sorted(vector.index(s) for part, _ in plan.slices for s in part) == list(range(len(vector)))
+    engine.allocate(plan)
+    engine.generate(plan, native.device_header_text())
+    assert plan.persistent is not None and plan.persistent[1:3] == (8, 256) and plan.total_blocks == 5
+    assert len(rtc.compile_source(plan.source, engine.COMPILE_OPTIONS + [engine.RUN_ONLY])) > 1000
+    assert len(rtc.compile_source(plan.source, engine.COMPILE_OPTIONS)) > 1000
+
+
+def test_update_slices_keep_reads_conditions_and_dead_statements():
+    """A part holds every statement its states read through, conditional ones with the earlier
+    assignments they may keep; statements no state reads are checked in some part; one state, or one
+    part above half of the operations, is not sliced."""
+    from types import SimpleNamespace
+    load = lambda name: {"op": "load", "name": name}  # noqa: E731
+    exp = lambda name: {"op": "exp", "arg": load(name)}  # noqa: E731
+    stmt = lambda target, value, condition=None: {"target": target, "dtype": "f64", "value": value, "condition": condition}  # noqa: E731
+    vector = [stmt("_a", exp("a")), stmt("_b", exp("b")), stmt("_c", exp("c")), stmt("_d", exp("d")),
+              stmt("_a", exp("b"), "flag"), stmt("dead", exp("c")), stmt("a", load("_a")), stmt("b", load("_b")),
+              stmt("c", load("_c")), stmt("d", load("_d"))]
+    pop = SimpleNamespace(regular=[], update={"vector": vector, "effects": {"writes": ["a", "b", "c", "d"]}})
+    parts = {tuple(names): [vector.index(s) for s in part] for part, names in engine.update_slices(pop)}
+    assert parts[("a",)] == [0, 4, 6]
+    assert all(k in {i for part in parts.values() for i in part} for k in range(len(vector)))
+    assert engine.update_slices(SimpleNamespace(regular=[], update={
+        "vector": vector[:1] + vector[6:7], "effects": {"writes": ["a"]}})) is None
+    assert engine.update_slices(SimpleNamespace(regular=[({}, "pre")], update=pop.update)) is None
