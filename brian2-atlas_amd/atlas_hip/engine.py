@@ -2715,9 +2715,10 @@ def update_slices(pop: PopulationPlan) -> list | None:
     statements = pop.update["vector"]
     cost = [_value_ops(statement) for statement in statements]
 
-    def needed(names) -> set:
+    def needed(names, before: int = len(statements)) -> set:
+        # the statements ahead of `before` that the names' values there come from
         live, keep = set(names), set()
-        for k in range(len(statements) - 1, -1, -1):
+        for k in range(before - 1, -1, -1):
             if statements[k]["target"] in live:
                 keep.add(k)
                 if statements[k].get("condition") is None:
@@ -2732,8 +2733,9 @@ def update_slices(pop: PopulationPlan) -> list | None:
         part[0] |= needed([name])
         part[1].append(name)
     rest = set(range(len(statements))) - set().union(*(p[0] for p in parts))
-    if rest:   # read by no state: checked all the same, with what they read
-        parts[-1][0] |= needed([statements[k]["target"] for k in rest]) | rest
+    for k in sorted(rest):   # read by no state: checked all the same, with what they read
+        with_reads = needed(_statement_reads(statements[k]), k) | {k}
+        min(parts, key=lambda p: weigh(p[0] | with_reads))[0].update(with_reads)
     if 2 * max(weigh(p[0]) for p in parts) > sum(cost) or not all(names for _, names in parts):
         return None
     return [([statements[k] for k in sorted(keep)], names) for keep, names in parts]
