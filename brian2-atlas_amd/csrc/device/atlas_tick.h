@@ -128,6 +128,13 @@ struct Lds {
     alignas(16) byte_t exch[ATLAS_EXCH_BYTES > 0 ? ATLAS_EXCH_BYTES : 16];   // sliced updates' states
 };
 
+// Orders a wave's LDS stores before its lanes' later LDS loads of other lanes' entries.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // Workgroup barrier ordering LDS only.  Inside the tick every thread touches global
 // memory of its own neurons, targets and edges only (the same thread-to-neuron map
 // in every phase), so the phases' barriers exchange LDS data alone; a full
@@ -229,7 +236,9 @@ __device__ __forceinline__ void report(const u64* __restrict__ tab, int fault_bu
 // A reader of tick e, past the barrier of e, sees each word either as the publication of e
 // left it or as that of e - R did (whose stores every producer waited for before arriving at
 // barrier e - R + 1 <= e): stamp(e), stamp(e - R) or zero, and stamp(e - R) != stamp(e) for
-// any ring of 1 <= R < 4095 ticks.  So a word carrying stamp(e) is the one tick e wrote.
+// any ring of 1 <= R < 4095 ticks.  So a word carrying stamp(e) is the one tick e wrote.  Where no
+// barrier runs (delay 0, persistent_run's DIRECT) the reader has instead read every block's record of
+// tick e - 1, published after that block's waits for the stores of e - R, R >= 3.
 #define ATLAS_FAULT_STALL 32u          // a ring wait ran out of polls (the launch went on)
 #define ATLAS_SPIN_LIMIT (1u << 20)    // polls of one ring word, at least 0.1 s, before giving up
 #define ATLAS_RING_VALUE 0xFFFFFu      // value bits of a stamped ring word
@@ -1213,6 +1222,17 @@ __device__ void deliver(const u64* __restrict__ tab, i64 tick, double t, u32 blk
 // publishes tick t + 1 while the slowest may still read tick t (2 ring slots needed), and it
 // can arrive at tick t + 1 before the slowest has seen the barrier of tick t complete, but not
 // at tick t + 2 (2 barrier slots).
+//
+// The barrier would stand on that chain (an atomic, then its poll, then the records' round trip), and
+// the records validate themselves, so workgroups of one wave per SIMD, at most one to a CU, go
+// without it at delay 0 (DIRECT): each polls the records of its own tick.  A block publishes t only
+// after it has read every block's record of t - 1, published after that block's last read of t - 2: a
+// ring of 3 is never overwritten while read.  us per tick, with the barrier and without: CUBA of
+// 2000 neurons 3.8 / 3.1, 4000 3.6 / 3.15, 8000 3.85 / 3.25, 40,000 5.2 / 4.7; COBAHH of 1500 5.8 / 5.3,
+// 4000 6.1 / 5.6.  Where polling waves share a SIMD with publishing ones it loses: 100,000 neurons in
+// 391 blocks 8.7 / 9.0, 400,000 in blocks of 4096 (16 waves) 10.3 / 11.1.  Records polled by another wave
+// than the publishing one (3.4 at 4000 neurons) or by every wave, without the exchange's two
+// workgroup barriers (3.8), measured slower: first polls that come too early cost a round trip each.
 template <class Pop, class Group, class Fused>
 __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks, u32 blk, u32 nwg,
                                i64 start_tick, double dt_clock, int bar_buf, Lds& s) {
@@ -1232,6 +1252,7 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
     constexpr u32 BAR_SLOTS = 2 * Group::gval_max + 2;   // more than the 2 d barriers a wait and an arrival span
     // delay 0: each tick's deliveries follow its own publication and barrier
     constexpr bool SAME_TICK = Group::gval_max == 0;
+    constexpr bool DIRECT = SAME_TICK && Pop::R >= 3 && ATLAS_WG <= 256 && Group::SRC_NB <= 256;   // no grid barrier
     static_assert(Group::SRC_NB <= ATLAS_PASS, "block starts fit s.dense");
     static_assert(Pop::R == Group::SRC_R && Pop::R >= 2 * Group::gval_max + 2 && Pop::R < 4095u &&
                   Pop::R <= ATLAS_RING_PREV, "ring of 2 d + 2 ticks");
@@ -1286,7 +1307,7 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
         if (emitted >= start_tick) {
             // every block has issued its words of tick - delay (those of an earlier launch are
             // ordered by the launch boundary)
-            if (emitted >= tick0) grid_wait<BAR_SLOTS>(bar, (u32)(emitted - tick0 + 1), nwg, gave_up, fault);
+            if (!DIRECT && emitted >= tick0) grid_wait<BAR_SLOTS>(bar, (u32)(emitted - tick0 + 1), nwg, gave_up, fault);
             const u32 stamp = ring_stamp(emitted);
             uint4 rc[PERB][ATLAS_REC_WORDS / 4];
             u32 local = 0;
@@ -1491,13 +1512,14 @@ __device__ void persistent_run(const u64* __restrict__ tab, i64 tick0, i64 ticks
                 ring_store_u32(&rec[0], ring_word(stamp, before));
                 buf<u32>(tab, Pop::CNT)[(u64)slot * Pop::NB + blk] = before;   // for the host
             }
-            grid_arrive<BAR_SLOTS>(bar, (u32)(k + 1), blk, nwg);
-            // every work-item has read the slot's previous count (before grid_arrive's barrier)
+            if constexpr (!DIRECT) grid_arrive<BAR_SLOTS>(bar, (u32)(k + 1), blk, nwg);
+            // delay 0: the tick's own spikes, once every block has published them
+            if constexpr (SAME_TICK) exchange();
+            // every work-item has read the slot's previous count (before grid_arrive's or the exchange's
+            // barrier)
             if (threadIdx.x == 0) s.ring_prev[slot] = before;
         }
         if constexpr (SAME_TICK) {
-            // delay 0: the tick's own spikes, once every block has published them
-            exchange();
             issue(0);
             __builtin_amdgcn_s_setprio(0);
         }
@@ -1708,13 +1730,6 @@ __device__ __forceinline__ u32 edge_scan(u32* cnt, u32& largest) {
         run += c;
     }
     return total;
-}
-
-// Orders a wave's LDS stores before its lanes' later LDS loads of other lanes' entries.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
 // The counts of tick `tick` (LDS counters of tick & 1) applied to an update work-item's neurons
