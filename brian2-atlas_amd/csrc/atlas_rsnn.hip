@@ -19,9 +19,9 @@
 //     else fp32), with rows ordered (tick, sample);
 //   * the tick-sequential recurrence s_{t-1} W_rec (and g_{t+1} W_rec^T on the
 //     way back) runs in one persistent launch per pass, fused with the LIF
-//     update or its adjoint: at H = 256 one sample per workgroup with fp32 FMAs
-//     (a GEMV per tick), otherwise four samples per workgroup on fp32 MFMA;
-//     beyond H = 256, one launch of tiled 16x16 MFMA kernels per tick;
+//     update or its adjoint: up to H = 256 one sample per workgroup, three
+//     ticks per exchange on fp32 MFMA; beyond, one launch of tiled 16x16 MFMA
+//     kernels per tick;
 //   * the readout recurrence, loss and Adam are element-wise kernels.
 // Everything stays resident between steps: weights, Adam moments, the current
 // batch and the tapes.
@@ -153,249 +153,12 @@ __global__ void __launch_bounds__(256) backward_tick(u64 t, u64 T, u64 B, u64 H,
     }
 }
 
-// ------------------------------------------------- persistent recurrent pass
-// The recurrence couples the hidden units of one sample only, so a workgroup can own four
-// samples for every tick of a pass with nothing but workgroup barriers between ticks.  Wave w
-// owns columns [64w, 64w + 64): lane l holds column h = 64w + l of all four samples (state in
-// registers) and the matching slab of W_rec, the B operand of v_mfma_f32_4x4x1f32 (16 blocks of
-// 4x4; lane 4b+j gives A_b[j] and B_b[j] and receives D_b[i][j] in acc[i]).  The A operand is
-// broadcast (CBSZ = 4: every block takes block ABID's A), so lane 4b+i can hold x_i[16r + b]
-// in register r: the instruction with ABID = b then adds x_i[k] W[k][64w + l], k = 16r + b, for
-// the four samples i, and a tick is KMAX instructions per wave fed by KMAX / 16 A registers.
-// The four samples' vectors of the tick are exchanged through a double-buffered LDS array laid
-// out for that: row 4b + i holds x_i[16r + b] at column r (rows padded to a 16-byte multiple
-// plus 16 bytes, so that the row-per-lane float4 reads do not conflict), one barrier per tick.
-// The slab's first KREG rows live in registers, the remaining KMAX - KREG rows in LDS as float4
-// groups of four rows per column (conflict-free 16-byte reads), which leaves registers free for
-// the next tick's prefetch.  Columns and rows >= H hold zero weights and zero exchanged values,
-// so the product runs over all KMAX rows unbranched.
-template <int KMAX>
-struct Exchange {
-    static constexpr int R = KMAX / 16;   // A registers per lane
-    static constexpr int ROW = R + 4;     // floats per padded row
-    static constexpr int SIZE = 64 * ROW;
-
-    // column h of sample i
-    __device__ static __forceinline__ void put(float* x, u64 h, int i, float v) {
-        x[((h % 16) * 4 + i) * ROW + h / 16] = v;
-    }
-};
-
-template <int KMAX, int KREG>
-struct Slab {
-    static constexpr int KLDS = KMAX - KREG;
-    float w[KREG];
-    float4_t* tail;  // LDS: KLDS / 4 groups x KMAX columns
-
-    // FORWARD: B operand W[k][h]; otherwise W^T, i.e. W[h][k]
-    template <bool FORWARD>
-    __device__ __forceinline__ void load(const float* __restrict__ w_rec, u64 H, u64 h) {
-        const bool live = h < H;
-#pragma unroll
-        for (int k = 0; k < KREG; ++k)
-            w[k] = (live && (u64)k < H) ? (FORWARD ? w_rec[(u64)k * H + h] : w_rec[h * H + k]) : 0.0f;
-#pragma unroll
-        for (int g = 0; g < KLDS / 4; ++g) {
-            float4_t v;
-            for (int j = 0; j < 4; ++j) {
-                const u64 k = (u64)(KREG + 4 * g + j);
-                v[j] = (live && k < H) ? (FORWARD ? w_rec[k * H + h] : w_rec[h * H + k]) : 0.0f;
-            }
-            tail[g * KMAX + h] = v;
-        }
-    }
-
-    __device__ __forceinline__ float4_t product(const float* __restrict__ x, unsigned lane, u64 h) const {
-        typedef Exchange<KMAX> X;
-        float a[X::R];
-        const float4_t* row = reinterpret_cast<const float4_t*>(x + lane * X::ROW);
-#pragma unroll
-        for (int q = 0; q < X::R / 4; ++q) {
-            const float4_t v = row[q];
-            a[4 * q] = v[0];
-            a[4 * q + 1] = v[1];
-            a[4 * q + 2] = v[2];
-            a[4 * q + 3] = v[3];
-        }
-        float4_t acc[4] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f},
-                           {0.0f, 0.0f, 0.0f, 0.0f}};
-        chain<0>(a, h, acc);
-        return (acc[0] + acc[1]) + (acc[2] + acc[3]);
-    }
-
-    // rows K .. K + 3 (K + j = 16 r + id: A register r, broadcast block id), then the rest
-    template <int K>
-    __device__ __forceinline__ void chain(const float* a, u64 h, float4_t* acc) const {
-        if constexpr (K < KMAX) {
-            float4_t b;
-            if constexpr (K < KREG) {
-                b[0] = w[K];
-                b[1] = w[K + 1];
-                b[2] = w[K + 2];
-                b[3] = w[K + 3];
-            } else {
-                b = tail[((K - KREG) / 4) * KMAX + h];
-            }
-            // row K + j accumulates into acc[j]: consecutive MFMAs are independent, so none waits for
-            // the one before it
-            constexpr int r = K / 16, id = K % 16;
-            acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r], b[0], acc[0], 4, id, 0);
-            acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r], b[1], acc[1], 4, id + 1, 0);
-            acc[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r], b[2], acc[2], 4, id + 2, 0);
-            acc[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r], b[3], acc[3], 4, id + 3, 0);
-            chain<K + 4>(a, h, acc);
-        }
-    }
-};
-
 // Workgroup barrier ordering LDS only: the tick's global stores and prefetches stay in flight
 // (a full __syncthreads() would wait for every outstanding global access each tick).
 __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// Forward pass over every tick.  Tick t: P_t = s_t W_rec (used by tick t + 1) and the update
-// with h1_t = Hin_t + P_{t-1}; then s_{t+1} from the new membrane, published to LDS and taped
-// (tick 0's before the loop).  The update and the next tick's threshold, exchange and tapes do
-// not depend on P_t, so they share one block with its MFMA chain (with every work-item live,
-// FULL, the block has no branch) and the compiler schedules them together.  Grid: batch / 4
-// workgroups of KMAX work-items, H <= KMAX.
-template <int KMAX, int KREG, bool FULL>
-__global__ void __launch_bounds__(KMAX) forward_pass(u64 T, u64 B, u64 H, float alpha, float beta, float theta,
-                                                     const float* __restrict__ w_rec, const float* __restrict__ hin,
-                                                     float* __restrict__ mem_tape, float* __restrict__ spikes,
-                                                     bf16_t* __restrict__ spikes16) {
-    __shared__ __attribute__((aligned(16))) float xs[2][Exchange<KMAX>::SIZE];
-    __shared__ float4_t tail[(KMAX - KREG) / 4 * KMAX + 1];
-    const unsigned lane = threadIdx.x % 64;
-    const u64 h = threadIdx.x, b0 = (u64)blockIdx.x * 4;
-    const bool live = FULL || h < H;
-    Slab<KMAX, KREG> slab;
-    slab.tail = tail;
-    slab.template load<true>(w_rec, H, h);
-    float syn[4] = {0.0f, 0.0f, 0.0f, 0.0f}, mem[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    float s[4], in[4], next[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    float4_t rec = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int i = 0; i < 4; ++i) in[i] = live ? hin[(b0 + i) * H + h] : 0.0f;
-    // s_t from the membrane entering tick t, published and taped; tick t + 1's input prefetched
-    // (the index is clamped inside the run; the value is unused after the last tick)
-    auto emit = [&](u64 t) {
-        float* x = xs[t & 1];
-        const u64 tn = t + 1 < T ? t + 1 : t;
-        for (int i = 0; i < 4; ++i) {
-            s[i] = mem[i] > theta ? 1.0f : 0.0f;
-            Exchange<KMAX>::put(x, h, i, s[i]);
-            if (live) {
-                const u64 at = (t * B + b0 + i) * H + h;
-                mem_tape[at] = mem[i];
-                spikes[at] = s[i];
-                spikes16[at] = s[i] != 0.0f ? (bf16_t)0x3F80 : (bf16_t)0;
-                next[i] = hin[(tn * B + b0 + i) * H + h];
-            }
-        }
-    };
-    auto update = [&]() {
-        for (int i = 0; i < 4; ++i) {
-            const float h1 = in[i] + rec[i];
-            const float sy = syn[i];
-            syn[i] = alpha * sy + h1;
-            mem[i] = (beta * mem[i] + sy) * (1.0f - s[i]);
-            in[i] = next[i];
-        }
-    };
-    emit(0);
-    for (u64 t = 0; t < T; ++t) {
-        lds_barrier();
-        float4_t product = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (t + 1 < T) {
-            product = slab.product(xs[t & 1], lane, h);
-            update();
-            emit(t + 1);
-        } else {
-            update();
-        }
-        rec = product;
-    }
-}
-
-// Backward pass over every tick, descending.  Tick t: Q_t = g1_t W_rec^T (used by tick t - 1),
-// then the adjoints of (mem_t, syn_t) with gs_t = gs_read_t + Q_{t+1}; then g1_{t-1} (the new
-// adjoint of syn) written and published, and tick t - 2's tape values prefetched.  As in the
-// forward pass, everything but Q_t shares one block with its MFMA chain.  Lane l holds row h of
-// W_rec (the B operand of W_rec^T).
-template <int KMAX, int KREG, bool FULL>
-__global__ void __launch_bounds__(KMAX) backward_pass(u64 T, u64 B, u64 H, float alpha, float beta, float theta,
-                                                      float slope, const float* __restrict__ w_rec,
-                                                      const float* __restrict__ gs_read,
-                                                      const float* __restrict__ mem_tape,
-                                                      const float* __restrict__ spikes, float* __restrict__ g1,
-                                                      bf16_t* __restrict__ g3) {
-    __shared__ __attribute__((aligned(16))) float xs[2][Exchange<KMAX>::SIZE];
-    __shared__ float4_t tail[(KMAX - KREG) / 4 * KMAX + 1];
-    const unsigned lane = threadIdx.x % 64;
-    const u64 h = threadIdx.x, b0 = (u64)blockIdx.x * 4;
-    const bool live = FULL || h < H;
-    Slab<KMAX, KREG> slab;
-    slab.tail = tail;
-    slab.template load<false>(w_rec, H, h);
-    float gmem[4] = {0.0f, 0.0f, 0.0f, 0.0f}, gsyn[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    float4_t rec = {0.0f, 0.0f, 0.0f, 0.0f};
-    float gr[4] = {0.0f, 0.0f, 0.0f, 0.0f}, sp[4] = {0.0f, 0.0f, 0.0f, 0.0f}, mt[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    float ngr[4] = {0.0f, 0.0f, 0.0f, 0.0f}, nsp[4] = {0.0f, 0.0f, 0.0f, 0.0f}, nmt[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (live)
-        for (int i = 0; i < 4; ++i) {
-            const u64 at = ((T - 1) * B + b0 + i) * H + h;
-            gr[i] = gs_read[at];
-            sp[i] = spikes[at];
-            mt[i] = mem_tape[at];
-        }
-    // g1_t (the adjoint of syn_{t+1}) published and written; tick t - 1's tape values prefetched
-    // (clamped inside the run; unused before tick 0)
-    auto emit = [&](u64 t) {
-        float* x = xs[t & 1];
-        const u64 tp = t > 0 ? t - 1 : t;
-        for (int i = 0; i < 4; ++i) {
-            Exchange<KMAX>::put(x, h, i, gsyn[i]);
-            if (live) {
-                const u64 at = (t * B + b0 + i) * H + h;
-                g1[at] = gsyn[i];
-                bf16_t* piece = g3 + (t * B + b0 + i) * 3 * H + h;
-                split3(gsyn[i], piece[0], piece[H], piece[2 * H]);
-                const u64 prev = (tp * B + b0 + i) * H + h;
-                ngr[i] = gs_read[prev];
-                nsp[i] = spikes[prev];
-                nmt[i] = mem_tape[prev];
-            }
-        }
-    };
-    auto update = [&]() {
-        for (int i = 0; i < 4; ++i) {
-            const float q = slope * fabsf(mt[i] - theta) + 1.0f;
-            const float sigma = 1.0f / (q * q);
-            const float gs = gr[i] + rec[i];
-            const float gm_next = gmem[i], gs_next = gsyn[i];
-            gmem[i] = beta * (1.0f - sp[i]) * gm_next + gs * sigma;
-            gsyn[i] = (1.0f - sp[i]) * gm_next + alpha * gs_next;
-            gr[i] = ngr[i];
-            sp[i] = nsp[i];
-            mt[i] = nmt[i];
-        }
-    };
-    emit(T - 1);
-    for (u64 t = T; t-- > 0;) {
-        lds_barrier();
-        float4_t product = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (t > 0) {
-            product = slab.product(xs[t & 1], lane, h);
-            update();
-            emit(t - 1);
-        } else {
-            update();
-        }
-        rec = product;
-    }
 }
 
 // ------------------------------------------------ one sample per workgroup (H = 256)
@@ -542,7 +305,7 @@ __global__ void __launch_bounds__(1024) backward_vec(u64 T, u64 B, float alpha, 
     }
 }
 
-// ------------------------------------- three ticks per exchange (H = 256, one sample per workgroup)
+// ------------------------------------- three ticks per exchange (H <= 256, one sample per workgroup)
 // The recurrent product of tick t enters the membrane three ticks later at the earliest: P_t =
 // s_t W_rec enters h1_{t+1}, hence syn_{t+2}, hence mem_{t+3} and s_{t+3} (the membrane update
 // reads the synaptic current of the tick before).  So once s_t0, s_t0+1 and s_t0+2 are known the
@@ -551,50 +314,55 @@ __global__ void __launch_bounds__(1024) backward_vec(u64 T, u64 B, float alpha, 
 // pass has the same three-tick latency (Q_t = g_t W_rec^T enters gmem_{t-1}, hence gsyn_{t-2}).
 //
 // The 3-row product runs on v_mfma_f32_4x4x1f32 (16 blocks of 4 x 4, K = 1; row 3 is zero):
-// wave w takes the 64 columns 64 (w % 4) .. + 63 (lane l: column 64 (w % 4) + l) over the
-// quarter of the rows 64 (w / 4) .. + 63, whose weights it keeps in 64 registers as B operands.
-// The A operand is broadcast from one block (CBSZ = 4, ABID = b): lane 4b + i holds row i's value
-// x_i[64 (w / 4) + 16 r + b] in register r, one 16-byte LDS read per lane per exchange.  Each
+// with NC = ceil(H / 64) groups of 64 columns, wave w of 4 NC takes columns 64 (w % NC) .. + 63 (lane
+// l: column 64 (w % NC) + l) over the quarter of the rows 16 NC (w / NC) .. + 16 NC - 1, whose weights
+// it keeps in 16 NC registers as B operands (zeros past H).  The A operand is broadcast from one
+// block (CBSZ = 4, ABID = b): lane 4b + i holds row i's value x_i[16 NC (w / NC) + 16 r + b] in
+// register r < NC, one 16-byte LDS read per lane per exchange.  Each
 // wave accumulates row k into accumulator k % 4 in ascending k and sums them as
 // (a0 + a1) + (a2 + a3); the four quarters' partial products meet in LDS and are summed as
-// (q0 + q1) + (q2 + q3): the order of the one-tick passes above (quarter_dot, quad_sum), so with
-// the MFMA's fused multiply-add per element both give the same bits.  The four waves of a column
+// (q0 + q1) + (q2 + q3): at H = 256 the order of the one-tick passes above (quarter_dot, quad_sum), so
+// with the MFMA's fused multiply-add per element both give the same bits.  The four waves of a column
 // update its state redundantly (identical bits); the first quarter's writes the tapes and the
 // exchanged values.
 constexpr int TRI_ROWS = 3;
 
-// x_i[k] of the exchanged 4 x 256 operand (i = tick row, k = hidden unit) in the A-register layout
+// x_i[k] of the exchanged 4 x 64 NC operand (i = tick row, k = hidden unit) in the A-register layout
+template <int NC>
 __device__ __forceinline__ int tri_at(int k, int i) {
-    const int m = k & 63;
-    return (k >> 6) * 256 + ((m & 15) * 4 + i) * 4 + (m >> 4);
+    const int m = k % (16 * NC);
+    return (k / (16 * NC)) * 256 + ((m & 15) * 4 + i) * 4 + (m >> 4);
 }
 
-// Rows M .. M + 3 of the wave's quarter (row 64 kq + m: A register m / 16, broadcast block m % 16,
+// Rows M .. M + 3 of the wave's quarter (row 16 NC kq + m: A register m / 16, broadcast block m % 16,
 // accumulator m % 4), then the rest.
-template <int M>
+template <int NC, int M>
 __device__ __forceinline__ void tri_chain(const float4_t& a, const float* w, float4_t* acc) {
-    if constexpr (M < 64) {
+    if constexpr (M < 16 * NC) {
         acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[M / 16], w[M], acc[0], 4, M % 16, 0);
         acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[M / 16], w[M + 1], acc[1], 4, M % 16 + 1, 0);
         acc[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[M / 16], w[M + 2], acc[2], 4, M % 16 + 2, 0);
         acc[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[M / 16], w[M + 3], acc[3], 4, M % 16 + 3, 0);
-        tri_chain<M + 4>(a, w, acc);
+        tri_chain<NC, M + 4>(a, w, acc);
     }
 }
 
-// The wave's quarter (rows 64 kq .. 64 kq + 63) of the 4-row product for its lane's column.
+// The wave's quarter (rows 16 NC kq .. 16 NC kq + 16 NC - 1) of the 4-row product for its lane's column.
+template <int NC>
 __device__ __forceinline__ float4_t tri_quarter(const float* __restrict__ x, const float* w, unsigned lane,
                                                 unsigned kq) {
     const float4_t a = *reinterpret_cast<const float4_t*>(x + kq * 256 + lane * 4);
     float4_t acc[4] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f},
                        {0.0f, 0.0f, 0.0f, 0.0f}};
-    tri_chain<0>(a, w, acc);
+    tri_chain<NC, 0>(a, w, acc);
     return (acc[0] + acc[1]) + (acc[2] + acc[3]);
 }
 
 // The lane's column of the 4-row product from the four quarters' partial products in LDS.
+template <int NC>
 __device__ __forceinline__ float4_t tri_sum(const float4_t* part, unsigned h) {
-    return (part[h] + part[VEC_H + h]) + (part[2 * VEC_H + h] + part[3 * VEC_H + h]);
+    constexpr unsigned W = 64 * NC;
+    return (part[h] + part[W + h]) + (part[2 * W + h] + part[3 * W + h]);
 }
 
 // Forward pass, three ticks per exchange.  Before block t0 (t0 = 0, 3, ...) the exchange holds
@@ -605,38 +373,47 @@ __device__ __forceinline__ float4_t tri_sum(const float4_t* part, unsigned h) {
 // operations of forward_vec's tick loop, in the same order per value.  The second quarter's waves
 // load the block's inputs and stage them in LDS, so that the updating lanes never wait for a load
 // (a wait for a load also waits for every store issued before it).
-__global__ void __launch_bounds__(1024) forward_tri(u64 T, u64 B, float alpha, float beta, float theta,
+template <int NC, bool FULL>
+__global__ void __launch_bounds__(256 * NC) forward_tri(u64 T, u64 B, u64 hidden, float alpha, float beta, float theta,
                                                     const float* __restrict__ w_rec, const float* __restrict__ hin,
                                                     float* __restrict__ mem_tape, float* __restrict__ spikes,
                                                     bf16_t* __restrict__ spikes16) {
-    constexpr u64 H = VEC_H;
+    const u64 H = FULL ? 64 * NC : hidden;
+    constexpr unsigned W = 64 * NC, ROWS = 16 * NC;   // columns with padding, rows of a quarter
     __shared__ __attribute__((aligned(16))) float xs[2][4 * 256];
-    __shared__ float4_t part[4 * H];
-    __shared__ float ins[TRI_ROWS][H];   // the block's inputs Hin_t0+1 .. Hin_t0+3
-    const unsigned lane = threadIdx.x % 64, wave = threadIdx.x / 64, kq = wave >> 2;
-    const unsigned h = (wave & 3u) * 64u + lane;
+    __shared__ float4_t part[4 * W];
+    __shared__ float ins[TRI_ROWS][W];   // the block's inputs Hin_t0+1 .. Hin_t0+3
+    const unsigned lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), kq = wave / NC;
+    const unsigned h = (wave % NC) * 64u + lane;
+    // a padded column repeats the last one (the same loads, values and stores); its row of the product
+    // has zero weights
+    const unsigned col = FULL || h < H ? h : (unsigned)H - 1u;
     const u64 b = blockIdx.x;
     const bool first = kq == 0, loader = kq == 1;
-    float w[64];
+    float w[ROWS];
 #pragma unroll
-    for (int m = 0; m < 64; ++m) w[m] = w_rec[(64 * kq + m) * H + h];
+    for (unsigned m = 0; m < ROWS; ++m) {
+        const unsigned k = ROWS * kq + m;   // uniform; past the last row: a load in bounds, a zero weight
+        const float v = (w_rec + (FULL || k < H ? k : H - 1) * H)[col];
+        w[m] = FULL || k < H ? v : 0.0f;
+    }
     // the weights are waited for here: otherwise the compiler's wait counting assumes they may
     // still be pending in every block and waits in the middle of the product for the block's
     // other memory accesses
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-    for (unsigned j = threadIdx.x; j < 2 * 4 * 256; j += 1024) (&xs[0][0])[j] = 0.0f;   // row 3 stays zero
+    for (unsigned j = threadIdx.x; j < 2 * 4 * 256; j += 256 * NC) (&xs[0][0])[j] = 0.0f;   // row 3 stays zero
     lds_barrier();
-    auto input = [&](u64 t) { return hin[(uint32_t)(((t < T ? t : T - 1) * B + b) * H + h)]; };
+    auto input = [&](u64 t) { return (hin + ((t < T ? t : T - 1) * B + b) * H)[col]; };
     // s_t of the membrane entering tick t, taped and exchanged in row `row` of buffer `x` (`full`:
     // t is known to lie inside the run)
     auto emit = [&](u64 t, float mem, float* x, int row, bool full) {
         const float s = mem > theta ? 1.0f : 0.0f;
-        x[tri_at((int)h, row)] = s;
+        x[tri_at<NC>((int)h, row)] = s;
         if (full || t < T) {
-            const uint32_t at = (uint32_t)((t * B + b) * H + h);
-            mem_tape[at] = mem;
-            spikes[at] = s;
-            spikes16[at] = s != 0.0f ? (bf16_t)0x3F80 : (bf16_t)0;
+            const u64 at = (t * B + b) * H;   // uniform: a scalar base, the column as the lane's offset
+            (mem_tape + at)[col] = mem;
+            (spikes + at)[col] = s;
+            (spikes16 + at)[col] = s != 0.0f ? (bf16_t)0x3F80 : (bf16_t)0;
         }
         return s;
     };
@@ -660,7 +437,7 @@ __global__ void __launch_bounds__(1024) forward_tri(u64 T, u64 B, float alpha, f
 #pragma unroll
             for (int j = 0; j < TRI_ROWS; ++j) in[j] = input(t0 + 1 + j);
         lds_barrier();
-        part[kq * VEC_H + h] = tri_quarter(xs[k & 1], w, lane, kq);
+        part[kq * W + h] = tri_quarter<NC>(xs[k & 1], w, lane, kq);
         // every wave's global accesses complete here, under the other waves' products: the
         // loading waves' inputs, and the updating lanes' tape stores of the block before (their
         // registers are then free for the update without a wait on its chain)
@@ -670,7 +447,7 @@ __global__ void __launch_bounds__(1024) forward_tri(u64 T, u64 B, float alpha, f
             for (int j = 0; j < TRI_ROWS; ++j) ins[j][h] = in[j];
         lds_barrier();
         if (first) {
-            const float4_t p = tri_sum(part, h);
+            const float4_t p = tri_sum<NC>(part, h);
             float* next = xs[(k + 1) & 1];
 #pragma unroll
             for (int j = 0; j < TRI_ROWS; ++j) {
@@ -699,34 +476,45 @@ __global__ void __launch_bounds__(1024) forward_tri(u64 T, u64 B, float alpha, f
 // lanes leave g in LDS (double-buffered by block parity) and the third quarter's waves write it,
 // and its split pieces, in the next block while its update runs (measured faster for this pass
 // than the updating lanes' own stores, which the forward pass keeps).
-__global__ void __launch_bounds__(1024) backward_tri(u64 T, u64 B, float alpha, float beta, float theta, float slope,
+template <int NC, bool FULL>
+__global__ void __launch_bounds__(256 * NC) backward_tri(u64 T, u64 B, u64 hidden, float alpha, float beta, float theta,
+                                                     float slope,
                                                      const float* __restrict__ w_rec,
                                                      const float* __restrict__ gs_read,
                                                      const float* __restrict__ mem_tape,
                                                      const float* __restrict__ spikes, float* __restrict__ g1,
                                                      bf16_t* __restrict__ g3) {
-    constexpr u64 H = VEC_H;
+    const u64 H = FULL ? 64 * NC : hidden;
+    constexpr unsigned W = 64 * NC, ROWS = 16 * NC;   // columns with padding, rows of a quarter
     __shared__ __attribute__((aligned(16))) float xs[2][4 * 256];
-    __shared__ float4_t part[4 * H];
+    __shared__ float4_t part[4 * W];
     // the block's gs_read, beta (1 - s) and sigma of ticks t0 - 1 - j, 1 - s of ticks t0 - 2 - j
-    __shared__ float tin[4][TRI_ROWS][H];
-    __shared__ float tout[2][TRI_ROWS][H];   // g_t0-3-j of the block, by parity
-    const unsigned lane = threadIdx.x % 64, wave = threadIdx.x / 64, kq = wave >> 2;
-    const unsigned h = (wave & 3u) * 64u + lane;
+    __shared__ float tin[4][TRI_ROWS][W];
+    __shared__ float tout[2][TRI_ROWS][W];   // g_t0-3-j of the block, by parity
+    const unsigned lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), kq = wave / NC;
+    const unsigned h = (wave % NC) * 64u + lane;
+    // a padded column repeats the last one (the same loads, values and stores); its row of the product
+    // has zero weights
+    const unsigned col = FULL || h < H ? h : (unsigned)H - 1u;
     const u64 b = blockIdx.x;
     const bool first = kq == 0, loader = kq == 1, storer = kq == 2;
-    float w[64];
+    float w[ROWS];
 #pragma unroll
-    for (int m = 0; m < 64; ++m) w[m] = w_rec[(u64)h * H + 64 * kq + m];   // row h of W_rec: column h of W_rec^T
+    for (unsigned m = 0; m < ROWS; ++m) {
+        const unsigned k = ROWS * kq + m;
+        const float v = (w_rec + (FULL || k < H ? k : H - 1))[col * (unsigned)H];
+        w[m] = FULL || k < H ? v : 0.0f;
+    }
+    // row h of W_rec: column h of W_rec^T
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): as in the forward pass
-    for (unsigned j = threadIdx.x; j < 2 * 4 * 256; j += 1024) (&xs[0][0])[j] = 0.0f;
+    for (unsigned j = threadIdx.x; j < 2 * 4 * 256; j += 256 * NC) (&xs[0][0])[j] = 0.0f;
     lds_barrier();
-    auto at = [&](i64 t) { return (uint32_t)(((u64)(t > 0 ? t : 0) * B + b) * H + h); };
+    auto row = [&](i64 t) { return ((u64)(t > 0 ? t : 0) * B + b) * H; };   // uniform
     auto write = [&](i64 t, float g) {
         if (t >= 0) {
-            g1[at(t)] = g;
-            const u64 pc = ((u64)t * B + b) * 3 * H + h;
-            split3(g, g3[pc], g3[pc + H], g3[pc + 2 * H]);
+            (g1 + row(t))[col] = g;
+            bf16_t* pieces = g3 + 3 * row(t);
+            split3(g, pieces[col], (pieces + H)[col], (pieces + 2 * H)[col]);
         }
     };
     auto sigma_of = [&](float mt) {
@@ -737,18 +525,18 @@ __global__ void __launch_bounds__(1024) backward_tri(u64 T, u64 B, float alpha, 
     float gmem = 0.0f, gsyn = 0.0f;
     if (first) {
         // g_T-1 = gsyn_T = 0; g_T-2 and g_T-3 need no product (Q_T = 0)
-        xs[0][tri_at((int)h, 0)] = gsyn;
+        xs[0][tri_at<NC>((int)h, 0)] = gsyn;
         write(last, gsyn);
-        const float gr = gs_read[at(last)], sp = spikes[at(last)], sigma = sigma_of(mem_tape[at(last)]);
-        const float sp1 = spikes[at(last - 1)];
+        const float gr = (gs_read + row(last))[col], sp = (spikes + row(last))[col], sigma = sigma_of((mem_tape + row(last))[col]);
+        const float sp1 = (spikes + row(last - 1))[col];
         const float gs = gr + 0.0f;
         const float gm_next = gmem, gs_next = gsyn;
         gmem = beta * (1.0f - sp) * gm_next + gs * sigma;   // gmem_T-1
         gsyn = (1.0f - sp) * gm_next + alpha * gs_next;     // gsyn_T-1 = g_T-2
-        xs[0][tri_at((int)h, 1)] = gsyn;
+        xs[0][tri_at<NC>((int)h, 1)] = gsyn;
         write(last - 1, gsyn);
         gsyn = (1.0f - sp1) * gmem + alpha * gsyn;          // gsyn_T-2 = g_T-3
-        xs[0][tri_at((int)h, 2)] = gsyn;
+        xs[0][tri_at<NC>((int)h, 2)] = gsyn;
         write(last - 2, gsyn);
         // the compiler's wait counting then knows these stores complete before the loop
         __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
@@ -763,13 +551,13 @@ __global__ void __launch_bounds__(1024) backward_tri(u64 T, u64 B, float alpha, 
         if (loader)
 #pragma unroll
             for (int j = 0; j < TRI_ROWS; ++j) {
-                v[0][j] = gs_read[at(t0 - 1 - j)];
-                v[1][j] = spikes[at(t0 - 1 - j)];
-                v[2][j] = mem_tape[at(t0 - 1 - j)];
-                v[3][j] = spikes[at(t0 - 2 - j)];
+                v[0][j] = (gs_read + row(t0 - 1 - j))[col];
+                v[1][j] = (spikes + row(t0 - 1 - j))[col];
+                v[2][j] = (mem_tape + row(t0 - 1 - j))[col];
+                v[3][j] = (spikes + row(t0 - 2 - j))[col];
             }
         lds_barrier();
-        part[kq * VEC_H + h] = tri_quarter(xs[k & 1], w, lane, kq);
+        part[kq * W + h] = tri_quarter<NC>(xs[k & 1], w, lane, kq);
         if (loader)
 #pragma unroll
             for (int j = 0; j < TRI_ROWS; ++j) {
@@ -781,14 +569,14 @@ __global__ void __launch_bounds__(1024) backward_tri(u64 T, u64 B, float alpha, 
             }
         lds_barrier();
         if (first) {
-            const float4_t q = tri_sum(part, h);
+            const float4_t q = tri_sum<NC>(part, h);
             float* next = xs[(k + 1) & 1];
 #pragma unroll
             for (int j = 0; j < TRI_ROWS; ++j) {
                 const float gs = tin[0][j][h] + q[j];
                 gmem = tin[1][j][h] * gmem + gs * tin[2][j][h];   // gmem_t0-1-j
                 gsyn = tin[3][j][h] * gmem + alpha * gsyn;        // gsyn_t0-2-j = g_t0-3-j
-                next[tri_at((int)h, j)] = gsyn;
+                next[tri_at<NC>((int)h, j)] = gsyn;
                 tout[k & 1][j][h] = gsyn;
             }
         }
@@ -988,37 +776,37 @@ bool gemm(AtlasRsnn* r, bool ta, bool tb, u64 M, u64 N, u64 K, const float* A, u
 // beyond it every tick is a launch of the tiled kernels.
 constexpr u64 PERSISTENT_MAX_HIDDEN = 256;
 
-template <int KMAX, int KREG, bool FULL>
-void launch_passes(AtlasRsnn* r, bool forward) {
+template <int NC, bool FULL>
+void launch_tri(AtlasRsnn* r, bool forward) {
     const AtlasRsnnSpec& s = r->spec;
-    const dim3 grid((unsigned)(s.batch / 4)), block(KMAX);
+    const dim3 grid((unsigned)s.batch), block(256 * NC);
     if (forward)
-        hipLaunchKernelGGL((forward_pass<KMAX, KREG, FULL>), grid, block, 0, r->stream, s.time, s.batch, s.hidden,
-                           s.alpha, s.beta, s.threshold, r->w[1], r->hin, r->mem_tape, r->spikes, r->spikes16);
+        hipLaunchKernelGGL((forward_tri<NC, FULL>), grid, block, 0, r->stream, s.time, s.batch, s.hidden, s.alpha,
+                           s.beta, s.threshold, r->w[1], r->hin, r->mem_tape, r->spikes, r->spikes16);
     else
-        hipLaunchKernelGGL((backward_pass<KMAX, KREG, FULL>), grid, block, 0, r->stream, s.time, s.batch, s.hidden,
-                           s.alpha, s.beta, s.threshold, s.slope, r->w[1], r->gs_read, r->mem_tape, r->spikes, r->g1,
-                           r->g3);
+        hipLaunchKernelGGL((backward_tri<NC, FULL>), grid, block, 0, r->stream, s.time, s.batch, s.hidden, s.alpha,
+                           s.beta, s.threshold, s.slope, r->w[1], r->gs_read, r->mem_tape, r->spikes, r->g1, r->g3);
 }
 
-// H = 256 (configuration 4): one sample per workgroup; otherwise four samples per workgroup with
-// the slab's rows in registers, all of them up to 128, between 129 and 255 192 in registers and
-// 64 in LDS.
 void persistent_pass(AtlasRsnn* r, bool forward) {
-    const u64 H = r->spec.hidden;
-    if (H == 256) {
-        const AtlasRsnnSpec& s = r->spec;
+    const AtlasRsnnSpec& s = r->spec;
+    if (s.hidden == 256 && r->one_tick) {
         if (forward)
-            hipLaunchKernelGGL(r->one_tick ? forward_vec : forward_tri, dim3((unsigned)s.batch), dim3(1024), 0,
-                               r->stream, s.time, s.batch, s.alpha, s.beta, s.threshold, r->w[1], r->hin, r->mem_tape,
-                               r->spikes, r->spikes16);
+            hipLaunchKernelGGL(forward_vec, dim3((unsigned)s.batch), dim3(1024), 0, r->stream, s.time, s.batch, s.alpha,
+                               s.beta, s.threshold, r->w[1], r->hin, r->mem_tape, r->spikes, r->spikes16);
         else
-            hipLaunchKernelGGL(r->one_tick ? backward_vec : backward_tri, dim3((unsigned)s.batch), dim3(1024), 0,
-                               r->stream, s.time, s.batch, s.alpha, s.beta, s.threshold, s.slope, r->w[1], r->gs_read,
-                               r->mem_tape, r->spikes, r->g1, r->g3);
-    } else if (H <= 64) launch_passes<64, 64, false>(r, forward);
-    else if (H <= 128) launch_passes<128, 128, false>(r, forward);
-    else launch_passes<256, 192, false>(r, forward);
+            hipLaunchKernelGGL(backward_vec, dim3((unsigned)s.batch), dim3(1024), 0, r->stream, s.time, s.batch,
+                               s.alpha, s.beta, s.threshold, s.slope, r->w[1], r->gs_read, r->mem_tape, r->spikes,
+                               r->g1, r->g3);
+        return;
+    }
+    const bool full = s.hidden % 64 == 0;
+    switch ((s.hidden + 63) / 64) {
+    case 1: full ? launch_tri<1, true>(r, forward) : launch_tri<1, false>(r, forward); break;
+    case 2: full ? launch_tri<2, true>(r, forward) : launch_tri<2, false>(r, forward); break;
+    case 3: full ? launch_tri<3, true>(r, forward) : launch_tri<3, false>(r, forward); break;
+    default: full ? launch_tri<4, true>(r, forward) : launch_tri<4, false>(r, forward);
+    }
 }
 
 // Phase boundaries of one step, recorded only by atlas_rsnn_profile.

@@ -177,3 +177,20 @@ def test_three_tick_passes_equal_one_tick_passes(T, monkeypatch):
         assert np.array_equal(vec[key], tri[key]), key
     for a, b in zip(vec["weights"], tri["weights"]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("H", [16, 64, 80, 128, 144, 192, 240])
+def test_three_tick_passes_at_every_width(H):
+    """Hidden sizes of one to four column groups, whole and with padded columns, at run lengths around
+    the block of three ticks, against the oracle at its bar."""
+    for T in (1, 2, 4, 31):
+        print(f"case: rsnn widths B=16 T={T} H={H}", flush=True)
+        plan, x, labels, weights = setup(16, T, 50, H, 5, seed=H + T)
+        with rsnn.NativeRecurrentTrainer(plan, weights=weights) as trainer:
+            out = trainer.step(x, labels)
+            spikes, ref = check_pass(plan, trainer, x, labels, weights, out)
+            assert T < 31 or spikes.mean() > 0.005
+            want = ro.backward(plan, *weights, x, ref)
+            for key, got in trainer.gradients().items():
+                err = np.abs(got - want[key]).max()
+                assert err <= 1e-5 * np.abs(want[key]).max() + 1e-12, (key, T, err)
