@@ -697,16 +697,29 @@ __global__ void split_rows(u64 n, const float* __restrict__ w, bf16_t* __restric
 
 __global__ void fill_int(int* __restrict__ p, int value) { *p = value; }
 
-__global__ void adam(u64 n, float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
-                     const float* __restrict__ g, float lr, float beta1, float beta2, float eps, float bc1, float bc2) {
-    const u64 x = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= n) return;
-    const float grad = g[x];
+// The Adam update of all three weight matrices and the split of the new W_in, in one launch: four
+// launches of a few us of work each cost 12 us of a step, this one 6 (H = 128, I = 200).
+struct AdamArrays {
+    u64 n[3];
+    float *w[3], *m[3], *v[3];
+    const float* g[3];
+};
+
+__global__ void adam(AdamArrays a, bf16_t* __restrict__ w3_in, float lr, float beta1, float beta2, float eps, float bc1,
+                     float bc2) {
+    u64 x = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    int k = 0;
+    for (; k < 3 && x >= a.n[k]; ++k) x -= a.n[k];
+    if (k == 3) return;
+    float *m = a.m[k], *v = a.v[k], *w = a.w[k];
+    const float grad = a.g[k][x];
     const float m1 = beta1 * m[x] + (1.0f - beta1) * grad;
     const float v1 = beta2 * v[x] + (1.0f - beta2) * grad * grad;
     m[x] = m1;
     v[x] = v1;
-    w[x] -= lr * (m1 / bc1) / (sqrtf(v1 / bc2) + eps);
+    const float updated = w[x] - lr * (m1 / bc1) / (sqrtf(v1 / bc2) + eps);
+    w[x] = updated;
+    if (k == 0) split3(updated, w3_in[x], w3_in[a.n[0] + x], w3_in[2 * a.n[0] + x]);
 }
 
 }  // namespace
@@ -776,6 +789,11 @@ bool gemm(AtlasRsnn* r, bool ta, bool tb, u64 M, u64 N, u64 K, const float* A, u
 // beyond it every tick is a launch of the tiled kernels.
 constexpr u64 PERSISTENT_MAX_HIDDEN = 256;
 
+// The three-tick passes at every hidden size up to 256: what bounds them is the chain of exchanges (an
+// MFMA chain of 16 NC rows and two workgroup barriers per three ticks), so each sample has a workgroup
+// of its own.  Against four samples per workgroup and one tick per exchange (forward / backward, us): 48
+// samples, 150 ticks, H = 128 178 / 212 -> 41 / 52; 256 samples, 100 ticks, H = 64 94 / 113 -> 23 / 29, H = 192
+// 193 / 229 -> 45 / 60, H = 240 201 / 244 -> 63 / 108; 2048 samples, 60 ticks, H = 128 113 / 154 -> 80 / 115.
 template <int NC, bool FULL>
 void launch_tri(AtlasRsnn* r, bool forward) {
     const AtlasRsnnSpec& s = r->spec;
@@ -944,12 +962,17 @@ int run_step(AtlasRsnn* r, bool train, char* err, size_t cap) {
         r->step_count += 1;
         const float bc1 = (float)(1.0 - std::pow((double)s.beta1, (double)r->step_count));
         const float bc2 = (float)(1.0 - std::pow((double)s.beta2, (double)r->step_count));
-        if (s.learning_rate != 0.0f)
-            for (int k = 0; k < 3; ++k)
-                hipLaunchKernelGGL(adam, dim3(blocks(r->size[k])), dim3(256), 0, st, r->size[k], r->w[k], r->m[k],
-                                   r->v[k], r->g[k], s.learning_rate, s.beta1, s.beta2, s.epsilon, bc1, bc2);
-        if (s.learning_rate != 0.0f)
-            hipLaunchKernelGGL(split_rows, dim3(blocks(I * H)), dim3(256), 0, st, I * H, r->w[0], r->w3_in);
+        if (s.learning_rate != 0.0f) {
+            AdamArrays a{};
+            u64 total = 0;
+            for (int k = 0; k < 3; ++k) {
+                a.n[k] = r->size[k];
+                a.w[k] = r->w[k], a.m[k] = r->m[k], a.v[k] = r->v[k], a.g[k] = r->g[k];
+                total += r->size[k];
+            }
+            hipLaunchKernelGGL(adam, dim3(blocks(total)), dim3(256), 0, st, a, r->w3_in, s.learning_rate, s.beta1,
+                               s.beta2, s.epsilon, bc1, bc2);
+        }
         mark(r, 7);
     }
     if (hipGetLastError() != hipSuccess) return fail(err, cap, 4, "kernel launch failed");
