@@ -2631,15 +2631,30 @@ FITTED = (Shape(256, 256, 4, 10), Shape(512, 512, 2, 10), Shape(1024, 1024, 1, 1
           Shape(3072, 1024, 2, 11), Shape(4096, 1024, 2, 11))
 
 
+def _split_pathways(plan: Plan, groups: list) -> int:
+    """The most pathways into one population, at least 1 (atlas_tick.h ATLAS_SUM_NP)."""
+    return max([1] + [sum(len(g) for g in groups if g[0].target == pop.index) for pop in plan.populations])
+
+
+def _split_lds(shape: Shape, xwaves: int, pathways: int) -> int:
+    """Bytes of the split loop's LDS (atlas_tick.h LdsSplit) where every group counts: two ticks' counters
+    of every pathway into a population, the fired masks and sums, and each exchange wave's lists."""
+    head = 4 * RING_SLOTS + 24 + 8 * 64 + 8 * (shape.wg // 64) * pathways
+    size = -(-head // 16) * 16 + 2 * 4 * pathways * shape.block + 4 * xwaves * (ATLAS_XLIST + 64)
+    return -(-size // 16) * 16
+
+
 def _fits_split(plan: Plan, groups: list, shape: Shape) -> bool:
     """Whether the split loop takes the plan in this shape: two halves of waves, every workgroup on a
     CU of its own, at most 64 source blocks per exchange wave (the first one only publishes), one fired
-    mask per lane of that wave."""
+    mask per lane of that wave, and LDS for the counters (edge buckets take what is left of it)."""
     xwaves = SPLIT_XWAVES or shape.wg // 128
     blocks = [-(-pop.count // shape.block) for pop in plan.populations]
     return (1 <= xwaves < shape.wg // 64 and sum(blocks) <= CUS
             and all(blocks[g[0].source] <= 64 * max(1, xwaves - 1) for g in groups)
-            and -(-shape.block // (shape.wg - 64 * xwaves)) * (shape.wg // 64 - xwaves) <= 64)
+            and -(-shape.block // (shape.wg - 64 * xwaves)) * (shape.wg // 64 - xwaves) <= 64
+            and (not all(counting_group(g) for g in groups)
+                 or _split_lds(shape, xwaves, _split_pathways(plan, groups)) <= LDS_BYTES))
 
 
 def _split_lag(groups: list) -> int:
@@ -4396,11 +4411,13 @@ def generate(plan: Plan, header_text: str) -> None:
             and all("slot" in path.buffers and path.index not in plan.slot_fallback for g in groups for path in g))
     split_loop = wide or (PERSISTENT_SPLIT and not plan.split and len(groups) == 1 and _fits_split(plan, groups, plan.shape))
     if split_loop:
-        pathways_into = [sum(len(g) for g in groups if g[0].target == pop.index) for pop in plan.populations]
+        pathways = _split_pathways(plan, groups)
         parts.insert(parts.index(header_text), f"#define ATLAS_XWAVES {xwaves}u")
-        parts.insert(parts.index(header_text), f"#define ATLAS_SUM_NP {max(1, *pathways_into)}u")
+        parts.insert(parts.index(header_text), f"#define ATLAS_SUM_NP {pathways}u")
     eligible = wide or persistent_eligible(plan, groups, counting, split_loop)
     if eligible and split_loop:
+        if all(counting):
+            parts.append(f"static_assert(sizeof(atlas::LdsSplit) == {_split_lds(plan.shape, xwaves, pathways)}u, \"LDS of a shape\");")
         lag = _split_lag(groups)
         for q in sorted({q for pop in plan.populations for q in readers_of(pop)}):
             reader = plan.populations[q]

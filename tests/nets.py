@@ -708,6 +708,30 @@ def multiclock_network(n: int = 3000, *, steps: int = 600, seed: int = 11, indeg
                      delay_ticks=rng.integers(delays[0], delays[1] + 1, src.size))
     return b.document()
 
+
+def population_graph(counts, paths, *, steps: int = 5, seed: int = 3, late: tuple = ()) -> dict:
+    """Driven LIF populations of ``counts`` neurons; ``paths`` = (source, target, delay, in-degree, weight in
+    V): on_pre ``ge += w``, or ``v += w`` into the populations in ``late``, whose reset (it writes v too) then
+    follows the deliveries.  Every pathway is a delivery group of its own (all write one state)."""
+    c = models.CUBA
+    rng = np.random.default_rng(seed)
+    b = NetworkBuilder(dt=1e-4, steps=steps, seed=seed)
+    scalar = lambda value, dims: ("f64", dims, value)  # noqa: E731
+    params = {"taum": scalar(c["taum"], SECOND), "taue": scalar(c["taue"], SECOND), "taui": scalar(c["taui"], SECOND),
+              "El": scalar(-49e-3, VOLT), "Vt": scalar(c["Vt"], VOLT), "Vr": scalar(c["Vr"], VOLT)}
+    pops = [b.population(
+        f"group{k}", n, states={"v": ("f32", VOLT, c["Vr"] + rng.random(n) * (c["Vt"] - c["Vr"])),
+                                "ge": ("f32", VOLT, np.zeros(n)), "gi": ("f32", VOLT, np.zeros(n))},
+        parameters=params, update=models.cuba_update("f32"), threshold=op("gt", wide(ld("v")), ld("Vt")),
+        reset=[stmt("v", "f32", narrow(ld("Vr")), VOLT)], refractory=c["refractory"]) for k, n in enumerate(counts)]
+    for k, (source, target, delay, indegree, weight) in enumerate(paths):
+        state = "v" if target in late else "ge"
+        b.projection(f"path{k:02d}", pops[source], pops[target], fixed_indegree=indegree, delay_ticks=delay,
+                     on_pre=[stmt(state, "f32", narrow(add(wide(ld(state)), ld("w"))), VOLT)],
+                     post_aliases={state: state}, parameters={"w": ("f64", VOLT, weight)})
+    return b.document()
+
+
 def clock_arrival_network(source_clock: int, delay: int, ticks, indices) -> dict:
     """A two-neuron spike generator on one of two clocks (0: dt = 0.1 ms, 60 ticks; 1: dt =
     0.15 ms, 40 ticks) driving one accumulator (v += w, w = 1 and 16 by source) on the other

@@ -845,6 +845,24 @@ def test_fitted_plans_of_several_groups_run_the_split_loop(doc, rings, readers):
     assert len(rtc.compile_source(plan.source, engine.COMPILE_OPTIONS)) > 1000
 
 
+@pytest.mark.parametrize("n,pathways,late,block", [
+    (900_000, 4, False, 4096), (900_000, 5, True, None), (800_000, 5, False, None), (600_000, 5, True, 3072),
+    (600_000, 6, False, None), (400_000, 8, False, 2048)])
+def test_split_loop_leaves_plans_whose_counters_pass_the_lds(n, pathways, late, block):
+    """Two ticks' counters of every pathway into a population share a workgroup's LDS: a plan with more
+    than a shape holds keeps one launch per tick.  Both sides of the line compile."""
+    doc = nets.population_graph([n], [(0, 0, 1 + k % 2, 2, 1e-5) for k in range(pathways)], late=(0,) if late else ())
+    plan = engine.lower(doc, verify_envelope=False)
+    before = plan.shape
+    engine.fit_shape(plan)
+    engine.allocate(plan)
+    engine.generate(plan, native.device_header_text())
+    assert len(plan.groups) == pathways and plan.fitted == (plan.persistent is not None) == (block is not None)
+    assert plan.shape.block == (block or before.block)
+    options = [engine.RUN_ONLY] if plan.persistent else []
+    assert len(rtc.compile_source(plan.source, engine.COMPILE_OPTIONS + options)) > 1000
+
+
 @pytest.mark.parametrize("delay", [0, 1])
 def test_heavy_update_is_sliced(delay):
     """COBAHH's update is split into four parts, {m}, {h}, {n} and {v, ge, gi}, each with the statements
