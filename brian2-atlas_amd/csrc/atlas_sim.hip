@@ -44,7 +44,10 @@ struct AtlasSim {
     void* work = nullptr;
     u64 work_bytes = 0;
     unsigned char* staging = nullptr;
-    u64 spikes_total = 0, spikes_rows = 0;   // atlas_sim_spikes_count's, for atlas_sim_spikes_read
+    // atlas_sim_spikes_count's, for the atlas_sim_spikes_read after it; not valid once the workspace (their
+    // row starts) is another call's or a call may have written the bitmap
+    bool spikes_counted = false;
+    u64 spikes_total = 0, spikes_rows = 0, spikes_words = 0;
     uint32_t spikes_buffer = 0;
     std::vector<double> kernel_ms;
     std::vector<u64> kernel_launches;
@@ -389,8 +392,10 @@ __global__ void gather_field(const unsigned char* __restrict__ records, u64 stri
         out[order ? order[r] : r] = *reinterpret_cast<const T*>(records + r * stride + offset);
 }
 
-// The handle's device workspace of at least `bytes` (its contents are lost when it grows).
+// The handle's device workspace of at least `bytes` (its contents are lost when it grows), taken from
+// whoever had it.
 int workspace(AtlasSim* sim, u64 bytes, char* err, size_t cap) {
+    sim->spikes_counted = false;
     if (bytes <= sim->work_bytes) return ATLAS_OK;
     if (sim->work) {
         HIP_TRY(hipStreamSynchronize(sim->stream), ATLAS_E_KERNEL);
@@ -494,6 +499,7 @@ int atlas_sim_upload(AtlasSim* sim, uint32_t buffer, uint64_t offset, const void
                      char* err, size_t cap) {
     if (!sim || buffer >= sim->buffers.size() || offset + bytes > sim->sizes[buffer])
         return fail(err, cap, ATLAS_E_HOST, "upload outside buffer %u", buffer);
+    sim->spikes_counted = false;
     HIP_TRY(hipMemcpyAsync(static_cast<char*>(sim->buffers[buffer]) + offset, host, bytes,
                            hipMemcpyHostToDevice, sim->stream), ATLAS_E_UPLOAD);
     HIP_TRY(hipStreamSynchronize(sim->stream), ATLAS_E_UPLOAD);
@@ -516,6 +522,7 @@ int atlas_sim_copy(AtlasSim* sim, uint32_t dst, uint64_t dst_offset, uint32_t sr
         src_offset + bytes > sim->sizes[src])
         return fail(err, cap, ATLAS_E_HOST, "copy outside buffers %u <- %u", dst, src);
     if (!bytes) return ATLAS_OK;
+    sim->spikes_counted = false;
     HIP_TRY(hipMemcpyAsync(static_cast<char*>(sim->buffers[dst]) + dst_offset,
                            static_cast<const char*>(sim->buffers[src]) + src_offset, bytes,
                            hipMemcpyDeviceToDevice, sim->stream), ATLAS_E_KERNEL);
@@ -525,6 +532,7 @@ int atlas_sim_copy(AtlasSim* sim, uint32_t dst, uint64_t dst_offset, uint32_t sr
 int atlas_sim_zero(AtlasSim* sim, uint32_t buffer, uint64_t offset, uint64_t bytes, char* err, size_t cap) {
     if (!sim || buffer >= sim->buffers.size() || offset + bytes > sim->sizes[buffer])
         return fail(err, cap, ATLAS_E_HOST, "zero outside buffer %u", buffer);
+    sim->spikes_counted = false;
     return zero_range(sim, static_cast<char*>(sim->buffers[buffer]) + offset, bytes, err, cap);
 }
 
@@ -690,6 +698,7 @@ int atlas_sim_run(AtlasSim* sim, int64_t start_tick, int64_t ticks, AtlasRunStat
                   size_t cap) {
     if (!sim || ticks < 0) return fail(err, cap, ATLAS_E_HOST, "invalid run arguments");
     HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
+    sim->spikes_counted = false;
     int rc = upload_table(sim, err, cap);
     if (rc) return rc;
     if (sim->persistent_ticks > 0) {
@@ -789,6 +798,7 @@ int atlas_sim_fixed_indegree(AtlasSim* sim, const AtlasFixedIndegree* spec, char
         return fail(err, cap, ATLAS_E_HOST, "fixed-indegree output buffers too small");
     if (spec->block == 0 || spec->blocks * spec->block < spec->target_start + n_tgt)
         return fail(err, cap, ATLAS_E_HOST, "target blocks do not cover the projection");
+    sim->spikes_counted = false;
     HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
     u32 log2cap = 7;
     while ((1ull << log2cap) < 2 * k_in) ++log2cap;
@@ -865,6 +875,7 @@ int atlas_sim_build_slots(AtlasSim* sim, const AtlasSlotTable* spec, uint32_t* m
         sim->sizes[spec->segment_buffer] < groups * (blocks + 1) * 4 ||
         sim->sizes[spec->slot_buffer] < spec->xcds * groups * per_xcd * 32)
         return fail(err, cap, ATLAS_E_HOST, "slot table does not match the segment table");
+    sim->spikes_counted = false;
     HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
     u32* flags = nullptr;
     HIP_TRY(hipMalloc(&flags, 8), ATLAS_E_ALLOC);
@@ -914,7 +925,6 @@ int atlas_sim_extract_spikes(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t row
         return fail(err, cap, ATLAS_E_HOST, "invalid spike bitmap arguments");
     HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
     *count = 0;
-    sim->spikes_total = sim->spikes_rows = 0;   // the workspace is this call's
     if (!rows) return ATLAS_OK;
     const u32* bits = static_cast<const u32*>(sim->buffers[bitmap_buffer]);
     if (int rc = count_rows(sim, bits, rows, words, count, err, cap)) return rc;
@@ -944,22 +954,24 @@ int atlas_sim_spikes_count(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t rows,
         return fail(err, cap, ATLAS_E_HOST, "invalid spike bitmap arguments");
     HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
     *count = 0;
+    sim->spikes_counted = false;
+    if (rows)
+        if (int rc = count_rows(sim, static_cast<const u32*>(sim->buffers[bitmap_buffer]), rows, words, count, err, cap))
+            return rc;
     sim->spikes_buffer = bitmap_buffer;
     sim->spikes_rows = rows;
-    sim->spikes_total = 0;
-    if (!rows) return ATLAS_OK;
-    if (int rc = count_rows(sim, static_cast<const u32*>(sim->buffers[bitmap_buffer]), rows, words, count, err, cap))
-        return rc;
+    sim->spikes_words = words;
     sim->spikes_total = *count;
+    sim->spikes_counted = true;
     return ATLAS_OK;
 }
 
 int atlas_sim_spikes_read(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t rows, uint64_t words, uint64_t neurons,
                           int64_t first_tick, int64_t* ticks, int64_t* indices, int64_t* counts, uint64_t total,
                           char* err, size_t cap) {
-    if (!sim || !counts || (total && (!ticks || !indices)) || bitmap_buffer != sim->spikes_buffer ||
-        rows != sim->spikes_rows || total != sim->spikes_total || bitmap_buffer >= sim->buffers.size() ||
-        sim->sizes[bitmap_buffer] < rows * words * 4)
+    if (!sim || !counts || (total && (!ticks || !indices)) || !sim->spikes_counted ||
+        bitmap_buffer != sim->spikes_buffer || rows != sim->spikes_rows || words != sim->spikes_words ||
+        total != sim->spikes_total)
         return fail(err, cap, ATLAS_E_HOST, "the spikes of this bitmap have not been counted");
     HIP_TRY(hipSetDevice(sim->device), ATLAS_E_DEVICE);
     if (!total) {
@@ -974,6 +986,7 @@ int atlas_sim_spikes_read(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t rows, 
         if (int rc = workspace(sim, bytes, err, cap)) return rc;
         if (int rc = count_rows(sim, bits, rows, words, &again, err, cap)) return rc;
         if (again != total) return fail(err, cap, ATLAS_E_HOST, "the spike bitmap changed between count and read");
+        sim->spikes_counted = true;
     }
     unsigned char* work = static_cast<unsigned char*>(sim->work);
     if (int rc = zero_range(sim, work + at_counts, neurons * 8, err, cap)) return rc;

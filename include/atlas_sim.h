@@ -167,9 +167,10 @@ int atlas_sim_extract_spikes(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t row
                              uint64_t neurons, int64_t* pairs_host, uint64_t capacity,
                              uint64_t* count, char* err, size_t cap);
 
-/* The same as one array per column, in two calls: the spikes counted (into *count), then read by the
- * next call on the handle, of the same bitmap and `total`: ticks (row + first_tick) and neurons of
- * every spike, and the spikes of each of the `neurons` neurons. */
+/* The same as one array per column, in two calls: the spikes counted (into *count), then read for the same
+ * bitmap, rows, words and `total`: ticks (row + first_tick) and neurons of every spike, and the spikes of
+ * each of the `neurons` neurons.  Another count, a run, an upload, a copy, a clear, atlas_sim_extract_spikes
+ * or atlas_sim_read_field on the handle in between ends the count's validity: the read then fails. */
 int atlas_sim_spikes_count(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t rows, uint64_t words, uint64_t* count,
                            char* err, size_t cap);
 int atlas_sim_spikes_read(AtlasSim* sim, uint32_t bitmap_buffer, uint64_t rows, uint64_t words, uint64_t neurons,

@@ -5,6 +5,7 @@ Bar: spike rasters, counts, last-spike lists, refractory state and synaptic even
 counts bit-exact; states bit-exact (both paths evaluate f64 registers with f32
 storage rounding per statement, so the results are identical, not merely close).
 """
+import ctypes
 import struct
 
 import numpy as np
@@ -1016,6 +1017,45 @@ def test_spike_bitmap_decoding(rows, words, neurons, density):
             assert np.array_equal(sim.extract_spikes(buffer, rows, words, neurons), want)
         with pytest.raises(native.NativeError):   # another total than counted
             sim._call("atlas_sim_spikes_read", buffer, rows, words, neurons, 0, None, None, counts.ctypes.data, 1)
+    finally:
+        sim.close()
+
+
+def test_spikes_are_read_only_after_their_own_count():
+    """The row starts of counted spikes live in the handle's workspace: a read after anything that may have
+    taken it or written the bitmap, or of other rows or words, is an error; a repeated read is not."""
+    bits = np.full((6, 4), 0x11, np.uint32)   # two spikes a word
+    sim = native.Sim(0)
+    try:
+        buffer, other = sim.alloc(bits.nbytes, bits), sim.alloc(4096, np.zeros(4096, np.uint8))
+        ticks, indices, counts = np.empty(48, np.int64), np.empty(48, np.int64), np.empty(128, np.int64)
+
+        def read(rows=6, words=4):
+            sim._call("atlas_sim_spikes_read", buffer, rows, words, 128, 0, ticks.ctypes.data, indices.ctypes.data,
+                      counts.ctypes.data, 48)
+
+        def count(buffer=buffer, rows=6, words=4):
+            total = ctypes.c_uint64()
+            sim._call("atlas_sim_spikes_count", buffer, rows, words, ctypes.byref(total))
+            return total.value
+
+        with pytest.raises(native.NativeError):
+            read()
+        for between in (lambda: sim.read_field(other, 8, 0, np.float64, 512, None), lambda: count(other, 1, 1),
+                        lambda: sim.extract_spikes(buffer, 6, 4, 128), lambda: sim.upload(buffer, bits),
+                        lambda: sim.copy(other, buffer, 16), lambda: sim.zero(other)):
+            assert count() == 48
+            between()
+            with pytest.raises(native.NativeError):
+                read()
+        assert count() == 48
+        for shape in ((4, 6), (5, 4), (6, 3)):
+            with pytest.raises(native.NativeError):
+                read(*shape)
+        for _ in range(2):
+            read()
+            assert np.array_equal(ticks, np.repeat(np.arange(6), 8)) and counts.sum() == 48
+            assert np.array_equal(indices[:8], [0, 4, 32, 36, 64, 68, 96, 100])
     finally:
         sim.close()
 
