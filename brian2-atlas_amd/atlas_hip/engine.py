@@ -4441,10 +4441,13 @@ def generate(plan: Plan, header_text: str) -> None:
         # workgroups per CU for 489 blocks of 2048: 4, at most 128 VGPRs; one 1024-wide for 245 of 4096:
         # 4; one 256-wide for configs 1 and 2: 1, so config 2's HH update keeps its values in registers)
         waves = max(1, -(-plan.total_blocks // CUS) * (run_wg // 64) // 4)
+        # left out of the module that launches the per-tick kernels alone (TICK_ONLY)
+        parts.append("#ifndef ATLAS_TICK_ONLY")
         parts.append(f'extern "C" __global__ void __launch_bounds__(ATLAS_WG) __attribute__((amdgpu_waves_per_eu({waves}))) '
                      "atlas_run(const u64* __restrict__ tab, i64 tick0, i64 ticks) {")
         parts.extend(persistent_body())
         parts.append("}")
+        parts.append("#endif")
         plan.persistent = (len(kernels), padded, run_wg, 0)
         kernels.append(("atlas_run", []))
     # synapse state updates and summed variables, each its own launch before the tick kernel,
@@ -4464,6 +4467,7 @@ def generate(plan: Plan, header_text: str) -> None:
         plan.launches.append((1, padded, WG, 0))
 
 
-RUN_ONLY = "-DATLAS_RUN_ONLY"   # compile option: the persistent launch's kernel alone
+RUN_ONLY = "-DATLAS_RUN_ONLY"     # compile option: the persistent launch's kernel alone
+TICK_ONLY = "-DATLAS_TICK_ONLY"   # the per-tick kernels alone
 COMPILE_OPTIONS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off", "-fno-fast-math",
                    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

@@ -129,7 +129,7 @@ class HipExecutor:
                     raise
                 self.persistent = False   # the grid cannot be resident at once: one launch per tick
         self.kernels = [name for name in self.plan.kernels if name != "atlas_run"]
-        self.sim.compile(self.plan.source, self.kernels, engine.COMPILE_OPTIONS)
+        self.sim.compile(self.plan.source, self.kernels, engine.COMPILE_OPTIONS + [engine.TICK_ONLY])
         # the launches name plan.kernels
         at = {k: self.kernels.index(name) for k, name in enumerate(self.plan.kernels) if name in self.kernels}
         self.sim.set_schedule([(at[k], *shape) for k, *shape in self.plan.launches])

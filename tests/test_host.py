@@ -880,6 +880,21 @@ def test_heavy_update_is_sliced(delay):
     assert len(rtc.compile_source(plan.source, engine.COMPILE_OPTIONS)) > 1000
 
 
+@pytest.mark.parametrize("doc", [models.cuba_network(600, p=0.02, steps=5), models.cobahh_network(300, steps=5),
+                                 models.delta_lif_network(3000, indegree=40, steps=5)], ids=["cuba", "cobahh", "delta_lif"])
+def test_modules_hold_only_the_kernels_they_launch(doc):
+    """A persistent plan's two modules: its run kernel alone, and the per-tick kernels a run falls back to
+    without it."""
+    plan = engine.lower(doc, verify_envelope=False)
+    engine.fit_shape(plan)
+    engine.allocate(plan)
+    engine.generate(plan, native.device_header_text())
+    run = rtc.compile_source(plan.source, engine.COMPILE_OPTIONS + [engine.RUN_ONLY])
+    tick = rtc.compile_source(plan.source, engine.COMPILE_OPTIONS + [engine.TICK_ONLY])
+    assert b"atlas_run" in run and b"atlas_tick" not in run
+    assert b"atlas_run" not in tick and b"atlas_tick" in tick
+
+
 def test_update_slices_keep_reads_conditions_and_dead_statements():
     """A part holds every statement its states read through, conditional ones with the earlier
     assignments they may keep; statements no state reads are checked in some part; one state, or one
