@@ -20,8 +20,9 @@
 //   * the tick-sequential recurrence s_{t-1} W_rec (and g_{t+1} W_rec^T on the
 //     way back) runs in one persistent launch per pass, fused with the LIF
 //     update or its adjoint: up to H = 256 one sample per workgroup, three
-//     ticks per exchange on fp32 MFMA; beyond, one launch of tiled 16x16 MFMA
-//     kernels per tick;
+//     ticks per exchange on fp32 MFMA (large batches below H = 256: four samples
+//     per workgroup, one tick per exchange); beyond, one launch of tiled 16x16
+//     MFMA kernels per tick;
 //   * the readout recurrence, loss and Adam are element-wise kernels.
 // Everything stays resident between steps: weights, Adam moments, the current
 // batch and the tapes.
@@ -153,12 +154,249 @@ __global__ void __launch_bounds__(256) backward_tick(u64 t, u64 T, u64 B, u64 H,
     }
 }
 
+// ------------------------------------------- four samples per workgroup (H < 256, large batches)
+// The recurrence couples the hidden units of one sample only, so a workgroup can own four
+// samples for every tick of a pass with nothing but workgroup barriers between ticks.  Wave w
+// owns columns [64w, 64w + 64): lane l holds column h = 64w + l of all four samples (state in
+// registers) and the matching slab of W_rec, the B operand of v_mfma_f32_4x4x1f32 (16 blocks of
+// 4x4; lane 4b+j gives A_b[j] and B_b[j] and receives D_b[i][j] in acc[i]).  The A operand is
+// broadcast (CBSZ = 4: every block takes block ABID's A), so lane 4b+i can hold x_i[16r + b]
+// in register r: the instruction with ABID = b then adds x_i[k] W[k][64w + l], k = 16r + b, for
+// the four samples i, and a tick is KMAX instructions per wave fed by KMAX / 16 A registers.
+// The four samples' vectors of the tick are exchanged through a double-buffered LDS array laid
+// out for that: row 4b + i holds x_i[16r + b] at column r (rows padded to a 16-byte multiple
+// plus 16 bytes, so that the row-per-lane float4 reads do not conflict), one barrier per tick.
+// The slab's first KREG rows live in registers, the remaining KMAX - KREG rows in LDS as float4
+// groups of four rows per column (conflict-free 16-byte reads), which leaves registers free for
+// the next tick's prefetch.  Columns and rows >= H hold zero weights and zero exchanged values,
+// so the product runs over all KMAX rows unbranched.
+template <int KMAX>
+struct Exchange {
+    static constexpr int R = KMAX / 16;   // A registers per lane
+    static constexpr int ROW = R + 4;     // floats per padded row
+    static constexpr int SIZE = 64 * ROW;
+
+    // column h of sample i
+    __device__ static __forceinline__ void put(float* x, u64 h, int i, float v) {
+        x[((h % 16) * 4 + i) * ROW + h / 16] = v;
+    }
+};
+
+template <int KMAX, int KREG>
+struct Slab {
+    static constexpr int KLDS = KMAX - KREG;
+    float w[KREG];
+    float4_t* tail;  // LDS: KLDS / 4 groups x KMAX columns
+
+    // FORWARD: B operand W[k][h]; otherwise W^T, i.e. W[h][k]
+    template <bool FORWARD>
+    __device__ __forceinline__ void load(const float* __restrict__ w_rec, u64 H, u64 h) {
+        const bool live = h < H;
+#pragma unroll
+        for (int k = 0; k < KREG; ++k)
+            w[k] = (live && (u64)k < H) ? (FORWARD ? w_rec[(u64)k * H + h] : w_rec[h * H + k]) : 0.0f;
+#pragma unroll
+        for (int g = 0; g < KLDS / 4; ++g) {
+            float4_t v;
+            for (int j = 0; j < 4; ++j) {
+                const u64 k = (u64)(KREG + 4 * g + j);
+                v[j] = (live && k < H) ? (FORWARD ? w_rec[k * H + h] : w_rec[h * H + k]) : 0.0f;
+            }
+            tail[g * KMAX + h] = v;
+        }
+    }
+
+    __device__ __forceinline__ float4_t product(const float* __restrict__ x, unsigned lane, u64 h) const {
+        typedef Exchange<KMAX> X;
+        float a[X::R];
+        const float4_t* row = reinterpret_cast<const float4_t*>(x + lane * X::ROW);
+#pragma unroll
+        for (int q = 0; q < X::R / 4; ++q) {
+            const float4_t v = row[q];
+            a[4 * q] = v[0];
+            a[4 * q + 1] = v[1];
+            a[4 * q + 2] = v[2];
+            a[4 * q + 3] = v[3];
+        }
+        float4_t acc[4] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f},
+                           {0.0f, 0.0f, 0.0f, 0.0f}};
+        chain<0>(a, h, acc);
+        return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    }
+
+    // rows K .. K + 3 (K + j = 16 r + id: A register r, broadcast block id), then the rest
+    template <int K>
+    __device__ __forceinline__ void chain(const float* a, u64 h, float4_t* acc) const {
+        if constexpr (K < KMAX) {
+            float4_t b;
+            if constexpr (K < KREG) {
+                b[0] = w[K];
+                b[1] = w[K + 1];
+                b[2] = w[K + 2];
+                b[3] = w[K + 3];
+            } else {
+                b = tail[((K - KREG) / 4) * KMAX + h];
+            }
+            // row K + j accumulates into acc[j]: consecutive MFMAs are independent, so none waits for
+            // the one before it
+            constexpr int r = K / 16, id = K % 16;
+            acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r], b[0], acc[0], 4, id, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r], b[1], acc[1], 4, id + 1, 0);
+            acc[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r], b[2], acc[2], 4, id + 2, 0);
+            acc[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r], b[3], acc[3], 4, id + 3, 0);
+            chain<K + 4>(a, h, acc);
+        }
+    }
+};
+
 // Workgroup barrier ordering LDS only: the tick's global stores and prefetches stay in flight
 // (a full __syncthreads() would wait for every outstanding global access each tick).
 __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Forward pass over every tick.  Tick t: P_t = s_t W_rec (used by tick t + 1) and the update
+// with h1_t = Hin_t + P_{t-1}; then s_{t+1} from the new membrane, published to LDS and taped
+// (tick 0's before the loop).  The update and the next tick's threshold, exchange and tapes do
+// not depend on P_t, so they share one block with its MFMA chain and the compiler schedules them
+// together.  Grid: batch / 4
+// workgroups of KMAX work-items, H <= KMAX.
+template <int KMAX, int KREG>
+__global__ void __launch_bounds__(KMAX) forward_pass(u64 T, u64 B, u64 H, float alpha, float beta, float theta,
+                                                     const float* __restrict__ w_rec, const float* __restrict__ hin,
+                                                     float* __restrict__ mem_tape, float* __restrict__ spikes,
+                                                     bf16_t* __restrict__ spikes16) {
+    __shared__ __attribute__((aligned(16))) float xs[2][Exchange<KMAX>::SIZE];
+    __shared__ float4_t tail[(KMAX - KREG) / 4 * KMAX + 1];
+    const unsigned lane = threadIdx.x % 64;
+    const u64 h = threadIdx.x, b0 = (u64)blockIdx.x * 4;
+    const bool live = h < H;
+    Slab<KMAX, KREG> slab;
+    slab.tail = tail;
+    slab.template load<true>(w_rec, H, h);
+    float syn[4] = {0.0f, 0.0f, 0.0f, 0.0f}, mem[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float s[4], in[4], next[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float4_t rec = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < 4; ++i) in[i] = live ? hin[(b0 + i) * H + h] : 0.0f;
+    // s_t from the membrane entering tick t, published and taped; tick t + 1's input prefetched
+    // (the index is clamped inside the run; the value is unused after the last tick)
+    auto emit = [&](u64 t) {
+        float* x = xs[t & 1];
+        const u64 tn = t + 1 < T ? t + 1 : t;
+        for (int i = 0; i < 4; ++i) {
+            s[i] = mem[i] > theta ? 1.0f : 0.0f;
+            Exchange<KMAX>::put(x, h, i, s[i]);
+            if (live) {
+                const u64 at = (t * B + b0 + i) * H + h;
+                mem_tape[at] = mem[i];
+                spikes[at] = s[i];
+                spikes16[at] = s[i] != 0.0f ? (bf16_t)0x3F80 : (bf16_t)0;
+                next[i] = hin[(tn * B + b0 + i) * H + h];
+            }
+        }
+    };
+    auto update = [&]() {
+        for (int i = 0; i < 4; ++i) {
+            const float h1 = in[i] + rec[i];
+            const float sy = syn[i];
+            syn[i] = alpha * sy + h1;
+            mem[i] = (beta * mem[i] + sy) * (1.0f - s[i]);
+            in[i] = next[i];
+        }
+    };
+    emit(0);
+    for (u64 t = 0; t < T; ++t) {
+        lds_barrier();
+        float4_t product = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (t + 1 < T) {
+            product = slab.product(xs[t & 1], lane, h);
+            update();
+            emit(t + 1);
+        } else {
+            update();
+        }
+        rec = product;
+    }
+}
+
+// Backward pass over every tick, descending.  Tick t: Q_t = g1_t W_rec^T (used by tick t - 1),
+// then the adjoints of (mem_t, syn_t) with gs_t = gs_read_t + Q_{t+1}; then g1_{t-1} (the new
+// adjoint of syn) written and published, and tick t - 2's tape values prefetched.  As in the
+// forward pass, everything but Q_t shares one block with its MFMA chain.  Lane l holds row h of
+// W_rec (the B operand of W_rec^T).
+template <int KMAX, int KREG>
+__global__ void __launch_bounds__(KMAX) backward_pass(u64 T, u64 B, u64 H, float alpha, float beta, float theta,
+                                                      float slope, const float* __restrict__ w_rec,
+                                                      const float* __restrict__ gs_read,
+                                                      const float* __restrict__ mem_tape,
+                                                      const float* __restrict__ spikes, float* __restrict__ g1,
+                                                      bf16_t* __restrict__ g3) {
+    __shared__ __attribute__((aligned(16))) float xs[2][Exchange<KMAX>::SIZE];
+    __shared__ float4_t tail[(KMAX - KREG) / 4 * KMAX + 1];
+    const unsigned lane = threadIdx.x % 64;
+    const u64 h = threadIdx.x, b0 = (u64)blockIdx.x * 4;
+    const bool live = h < H;
+    Slab<KMAX, KREG> slab;
+    slab.tail = tail;
+    slab.template load<false>(w_rec, H, h);
+    float gmem[4] = {0.0f, 0.0f, 0.0f, 0.0f}, gsyn[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float4_t rec = {0.0f, 0.0f, 0.0f, 0.0f};
+    float gr[4] = {0.0f, 0.0f, 0.0f, 0.0f}, sp[4] = {0.0f, 0.0f, 0.0f, 0.0f}, mt[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float ngr[4] = {0.0f, 0.0f, 0.0f, 0.0f}, nsp[4] = {0.0f, 0.0f, 0.0f, 0.0f}, nmt[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (live)
+        for (int i = 0; i < 4; ++i) {
+            const u64 at = ((T - 1) * B + b0 + i) * H + h;
+            gr[i] = gs_read[at];
+            sp[i] = spikes[at];
+            mt[i] = mem_tape[at];
+        }
+    // g1_t (the adjoint of syn_{t+1}) published and written; tick t - 1's tape values prefetched
+    // (clamped inside the run; unused before tick 0)
+    auto emit = [&](u64 t) {
+        float* x = xs[t & 1];
+        const u64 tp = t > 0 ? t - 1 : t;
+        for (int i = 0; i < 4; ++i) {
+            Exchange<KMAX>::put(x, h, i, gsyn[i]);
+            if (live) {
+                const u64 at = (t * B + b0 + i) * H + h;
+                g1[at] = gsyn[i];
+                bf16_t* piece = g3 + (t * B + b0 + i) * 3 * H + h;
+                split3(gsyn[i], piece[0], piece[H], piece[2 * H]);
+                const u64 prev = (tp * B + b0 + i) * H + h;
+                ngr[i] = gs_read[prev];
+                nsp[i] = spikes[prev];
+                nmt[i] = mem_tape[prev];
+            }
+        }
+    };
+    auto update = [&]() {
+        for (int i = 0; i < 4; ++i) {
+            const float q = slope * fabsf(mt[i] - theta) + 1.0f;
+            const float sigma = 1.0f / (q * q);
+            const float gs = gr[i] + rec[i];
+            const float gm_next = gmem[i], gs_next = gsyn[i];
+            gmem[i] = beta * (1.0f - sp[i]) * gm_next + gs * sigma;
+            gsyn[i] = (1.0f - sp[i]) * gm_next + alpha * gs_next;
+            gr[i] = ngr[i];
+            sp[i] = nsp[i];
+            mt[i] = nmt[i];
+        }
+    };
+    emit(T - 1);
+    for (u64 t = T; t-- > 0;) {
+        lds_barrier();
+        float4_t product = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (t > 0) {
+            product = slab.product(xs[t & 1], lane, h);
+            update();
+            emit(t - 1);
+        } else {
+            update();
+        }
+        rec = product;
+    }
 }
 
 // ------------------------------------------------ one sample per workgroup (H = 256)
@@ -789,11 +1027,11 @@ bool gemm(AtlasRsnn* r, bool ta, bool tb, u64 M, u64 N, u64 K, const float* A, u
 // beyond it every tick is a launch of the tiled kernels.
 constexpr u64 PERSISTENT_MAX_HIDDEN = 256;
 
-// The three-tick passes at every hidden size up to 256: what bounds them is the chain of exchanges (an
-// MFMA chain of 16 NC rows and two workgroup barriers per three ticks), so each sample has a workgroup
-// of its own.  Against four samples per workgroup and one tick per exchange (forward / backward, us): 48
-// samples, 150 ticks, H = 128 178 / 212 -> 41 / 52; 256 samples, 100 ticks, H = 64 94 / 113 -> 23 / 29, H = 192
-// 193 / 229 -> 45 / 60, H = 240 201 / 244 -> 63 / 108; 2048 samples, 60 ticks, H = 128 113 / 154 -> 80 / 115.
+// The three-tick passes give each sample a workgroup of its own: what bounds them is the chain of
+// exchanges (an MFMA chain of 16 NC rows and two workgroup barriers per three ticks).  Against four
+// samples per workgroup and one tick per exchange (forward / backward, us): 48 samples, 150 ticks, H =
+// 128 178 / 212 -> 41 / 52; 256 samples, 100 ticks, H = 64 94 / 113 -> 23 / 29, H = 192 193 / 229 ->
+// 45 / 60, H = 240 201 / 244 -> 63 / 108.
 template <int NC, bool FULL>
 void launch_tri(AtlasRsnn* r, bool forward) {
     const AtlasRsnnSpec& s = r->spec;
@@ -806,6 +1044,42 @@ void launch_tri(AtlasRsnn* r, bool forward) {
                            s.beta, s.threshold, s.slope, r->w[1], r->gs_read, r->mem_tape, r->spikes, r->g1, r->g3);
 }
 
+template <int KMAX, int KREG>
+void launch_four(AtlasRsnn* r, bool forward) {
+    const AtlasRsnnSpec& s = r->spec;
+    const dim3 grid((unsigned)(s.batch / 4)), block(KMAX);
+    if (forward)
+        hipLaunchKernelGGL((forward_pass<KMAX, KREG>), grid, block, 0, r->stream, s.time, s.batch, s.hidden, s.alpha,
+                           s.beta, s.threshold, r->w[1], r->hin, r->mem_tape, r->spikes, r->spikes16);
+    else
+        hipLaunchKernelGGL((backward_pass<KMAX, KREG>), grid, block, 0, r->stream, s.time, s.batch, s.hidden, s.alpha,
+                           s.beta, s.threshold, s.slope, r->w[1], r->gs_read, r->mem_tape, r->spikes, r->g1, r->g3);
+}
+
+// Whether a pass runs four samples per workgroup.  Once a batch fills the CUs several times over, the
+// chain of exchanges is hidden and the work counts: four samples use all four rows of the MFMA, three
+// ticks three of them, and a hidden size that is no multiple of 64 costs the three-tick backward pass
+// more.  Above H = 128 a CU holds one workgroup of the three-tick passes (256 samples a round) and
+// the four-sample passes run 1024 samples a round, which takes as long as 3.6 (forward, H > 192), 3.2
+// (backward, H <= 192) and 2.4 (backward, H > 192) rounds of 256; at H = 192 the three-tick passes always
+// win, and forward up to there.  Up to H = 128 many workgroups share a CU and the line is a batch.
+// 60 ticks, us, three ticks / four samples, forward and backward:
+//   H = 240: 512 samples 81 / 132, 167 / 161; 768 116 / 136, 242 / 181; 1024 152 / 142, 316 / 202; 1536
+//     226 / 263, 475 / 392; 4096 573 / 594, 1211 / 822.  H = 208, 1024 samples: 153 / 136, 265 / 180.
+//   H = 176, backward: 768 145 / 147; 1024 199 / 159; 1536 320 / 337; 4096 837 / 711.
+//   H = 128: 2048 89 / 116, 121 / 153; 3072 129 / 132, 178 / 176; 4096 172 / 149, 226 / 199; 8192
+//     338 / 395, 438 / 453.  H = 112: 2048 96 / 113, 159 / 145; 8192 360 / 389, 622 / 443.
+//   H = 48: 4096 72 / 81, 113 / 107; 8192 139 / 114, 220 / 151.
+bool four_samples(const AtlasRsnnSpec& s, bool forward) {
+    const u64 H = s.hidden, B = s.batch;
+    const bool padded = H % 64 != 0;
+    if (H <= 64) return B > 4096;
+    if (H <= 128) return padded ? (forward ? B > 2048 : B >= 2048) : B > 2048 && B <= 4096;
+    if (!padded || (forward && H <= 192)) return false;
+    const u64 round_tenths = forward ? 36 : H <= 192 ? 32 : 24;
+    return (B + 255) / 256 * 10 > (B + 1023) / 1024 * round_tenths;
+}
+
 void persistent_pass(AtlasRsnn* r, bool forward) {
     const AtlasRsnnSpec& s = r->spec;
     if (s.hidden == 256 && r->one_tick) {
@@ -816,6 +1090,13 @@ void persistent_pass(AtlasRsnn* r, bool forward) {
             hipLaunchKernelGGL(backward_vec, dim3((unsigned)s.batch), dim3(1024), 0, r->stream, s.time, s.batch,
                                s.alpha, s.beta, s.threshold, s.slope, r->w[1], r->gs_read, r->mem_tape, r->spikes,
                                r->g1, r->g3);
+        return;
+    }
+    if (four_samples(s, forward)) {
+        // the slab's rows in registers, all of them up to 128, above 192 in registers and 64 in LDS
+        if (s.hidden <= 64) launch_four<64, 64>(r, forward);
+        else if (s.hidden <= 128) launch_four<128, 128>(r, forward);
+        else launch_four<256, 192>(r, forward);
         return;
     }
     const bool full = s.hidden % 64 == 0;

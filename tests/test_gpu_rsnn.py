@@ -194,3 +194,20 @@ def test_three_tick_passes_at_every_width(H):
             for key, got in trainer.gradients().items():
                 err = np.abs(got - want[key]).max()
                 assert err <= 1e-5 * np.abs(want[key]).max() + 1e-12, (key, T, err)
+
+
+@pytest.mark.parametrize("B,H", [(4112, 48), (4096, 128), (2048, 112), (1024, 176), (528, 240), (1024, 208), (2048, 240)])
+def test_four_sample_passes_of_large_batches(B, H):
+    """Batches from which one or both passes run four samples per workgroup, in the slab shapes of 64, 128 and
+    256 rows, against the oracle at its bar."""
+    for T in (1, 2, 7, 16):
+        print(f"case: rsnn large batches B={B} T={T} H={H}", flush=True)
+        plan, x, labels, weights = setup(B, T, 16, H, 5, seed=H + T, scale=6.0, rate=0.2)
+        with rsnn.NativeRecurrentTrainer(plan, weights=weights) as trainer:
+            out = trainer.step(x, labels)
+            spikes, ref = check_pass(plan, trainer, x, labels, weights, out)
+            assert T < 16 or spikes.mean() > 0.005
+            want = ro.backward(plan, *weights, x, ref)
+            for key, got in trainer.gradients().items():
+                err = np.abs(got - want[key]).max()
+                assert err <= 1e-5 * np.abs(want[key]).max() + 1e-12, (key, T, err)
