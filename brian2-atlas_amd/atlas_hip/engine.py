@@ -2647,11 +2647,19 @@ def _split_lds(shape: Shape, xwaves: int, pathways: int) -> int:
 def _fits_split(plan: Plan, groups: list, shape: Shape) -> bool:
     """Whether the split loop takes the plan in this shape: two halves of waves, every workgroup on a
     CU of its own, at most 64 source blocks per exchange wave (the first one only publishes), one fired
-    mask per lane of that wave, and LDS for the counters (edge buckets take what is left of it)."""
+    mask per lane of that wave, and LDS for the counters (edge buckets take what is left of it).
+
+    Where a single wave reads (256 work-items) and the plan has several groups or populations, it takes
+    at most 32 source blocks: at high rates that wave lists every spike and bounds the tick.  us per tick
+    in blocks of 256, of 512 and with one launch per tick: 16,000 neurons firing at 120 Hz in four groups
+    16.1 / 10.1 / 13.6, in two 8.5 / 5.2 / 8.1, at 20 Hz 3.4 / 3.7 / 7.7; 16,000 Poisson inputs of 300 Hz 10.1 /
+    5.1 / 8.3, of 30 Hz 1.9 / 2.0 / 5.3; 8192 neurons at 120 Hz in four groups 10.2 / 7.6 / 12.9, at 20 Hz in two
+    3.0 / 3.4 / 7.4."""
     xwaves = SPLIT_XWAVES or shape.wg // 128
     blocks = [-(-pop.count // shape.block) for pop in plan.populations]
+    records = 32 if xwaves <= 2 and max(len(groups), len(plan.populations)) > 1 else 64
     return (1 <= xwaves < shape.wg // 64 and sum(blocks) <= CUS
-            and all(blocks[g[0].source] <= 64 * max(1, xwaves - 1) for g in groups)
+            and all(blocks[g[0].source] <= records * max(1, xwaves - 1) for g in groups)
             and -(-shape.block // (shape.wg - 64 * xwaves)) * (shape.wg // 64 - xwaves) <= 64
             and (not all(counting_group(g) for g in groups)
                  or _split_lds(shape, xwaves, _split_pathways(plan, groups)) <= LDS_BYTES))

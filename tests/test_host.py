@@ -845,6 +845,17 @@ def test_fitted_plans_of_several_groups_run_the_split_loop(doc, rings, readers):
     assert len(rtc.compile_source(plan.source, engine.COMPILE_OPTIONS)) > 1000
 
 
+@pytest.mark.parametrize("counts,paths,block", [
+    ([8192], [(0, 0, 1), (0, 0, 2)], 256), ([8193], [(0, 0, 1), (0, 0, 2)], 512), ([16_384], [(0, 0, 1)], 256),
+    ([8193, 300], [(0, 1, 1)], 512), ([300, 8193], [(0, 1, 1)], 256), ([49_153], [(0, 0, 1), (0, 0, 2)], 512)])
+def test_several_groups_give_a_single_reading_wave_32_blocks(counts, paths, block):
+    """With several groups or populations, the one exchange wave of 256-neuron blocks reads at most 32 source
+    blocks (64 with one group of one population); larger blocks have several."""
+    plan = engine.lower(nets.population_graph(counts, [(*path, 2, 1e-5) for path in paths]), verify_envelope=False)
+    engine.fit_shape(plan)
+    assert plan.fitted and plan.shape.block == block
+
+
 @pytest.mark.parametrize("n,pathways,late,block", [
     (900_000, 4, False, 4096), (900_000, 5, True, None), (800_000, 5, False, None), (600_000, 5, True, 3072),
     (600_000, 6, False, None), (400_000, 8, False, 2048)])
