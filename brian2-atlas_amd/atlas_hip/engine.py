@@ -2644,6 +2644,15 @@ def _split_lds(shape: Shape, xwaves: int, pathways: int) -> int:
     return -(-size // 16) * 16
 
 
+# Groups up to which a plan runs the split loop: its kernel holds every population's code over all of its
+# groups, and compiles in more time than the per-tick kernels'.  Seconds of compilation, split loop /
+# per tick, and us per tick: two groups 0.47 / 0.36, 3.1 / 7.4; one Poisson group into a population 0.38 /
+# 0.27, 2.2 / 6.2; four 0.75 / 0.58, 5.9 / 12.3; twelve 2.0 / 1.25, 17.3 / 34.6; four populations in 16
+# groups 2.9 / 1.7, 5.6 / 14.6, five in 25 4.7 / 2.6, 6.8 / 17.0, six in 36 7.1 / 3.6, 8.1 / 19.4: 25,000 ticks make
+# up for it with two groups, 130,000 with 16, 310,000 with 36.
+SPLIT_GROUPS = 16
+
+
 def _fits_split(plan: Plan, groups: list, shape: Shape) -> bool:
     """Whether the split loop takes the plan in this shape: two halves of waves, every workgroup on a
     CU of its own, at most 64 source blocks per exchange wave (the first one only publishes), one fired
@@ -2678,9 +2687,12 @@ def _split_model(plan: Plan, groups: list) -> bool:
     ordered one that edge buckets take), under updates light enough for its few update waves."""
     if not PERSISTENT_SPLIT or plan.multi_clock or plan.post_paths or plan.synapse_codes or not groups:
         return False
+    if len(groups) > SPLIT_GROUPS:
+        return False
     # a population driving itself without delay has one chain, update to apply, and more of its waves
-    # on each part of it in persistent_run, from a few blocks on (us per tick, split loop against
-    # persistent_run: CUBA of 500 neurons 2.8 / 3.2, 4000 3.9 / 3.5, 8000 4.1 / 3.7)
+    # on each part of it in persistent_run (us per tick, split loop / persistent_run: CUBA of 64 neurons
+    # 2.0 / 2.2, 300 2.4 / 2.4, 500 2.7 / 2.5, 1000 3.3 / 2.8, 1500 3.3 / 2.9, 2000 3.5 / 3.0).  Up to 1024
+    # neurons the split loop is kept: it also takes several groups, which persistent_run does not
     if plan.split and len(plan.populations) == 1 and plan.populations[0].count > 1024:
         return False
     for pop in plan.populations:

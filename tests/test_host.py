@@ -856,6 +856,19 @@ def test_several_groups_give_a_single_reading_wave_32_blocks(counts, paths, bloc
     assert plan.fitted and plan.shape.block == block
 
 
+@pytest.mark.parametrize("populations,fitted", [(4, True), (5, False)])
+def test_plans_of_many_groups_keep_one_launch_per_tick(populations, fitted):
+    """Fully coupled populations: 16 groups run the split loop, 25 do not (its compilation grows with them)."""
+    every = range(populations)
+    plan = engine.lower(nets.population_graph([200] * populations, [(i, j, 1, 2, 1e-5) for i in every for j in every]))
+    shape = plan.shape
+    engine.fit_shape(plan)
+    engine.allocate(plan)
+    engine.generate(plan, native.device_header_text())
+    assert len(plan.groups) == populations ** 2 and plan.fitted == (plan.persistent is not None) == fitted
+    assert plan.shape == shape
+
+
 @pytest.mark.parametrize("n,pathways,late,block", [
     (900_000, 4, False, 4096), (900_000, 5, True, None), (800_000, 5, False, None), (600_000, 5, True, 3072),
     (600_000, 6, False, None), (400_000, 8, False, 2048)])
