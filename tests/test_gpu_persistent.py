@@ -4,6 +4,7 @@ the CPU oracle and against one launch per tick: identical dumps, bit for bit."""
 import numpy as np
 import pytest
 
+import nets
 from atlas_hip import engine, models, protocol
 from atlas_hip.executor import HipExecutor
 from atlas_hip.models import hex_array
@@ -71,17 +72,21 @@ def test_persistent_synchronous_burst(monkeypatch):
 
 
 def test_large_blocks_with_long_segments_equal_oracle_and_per_tick(monkeypatch):
-    """280,000 neurons (one population of at least 64 x 4096) take 4096-neuron blocks of 1024
-    work-items, one workgroup per CU; at in-degree 1000 a (source, block) segment holds 14.6
-    targets on average, so about 40% exceed a slot's 15 inline targets and are read from the
-    row table.  100 ticks: the persistent launch equals the oracle and one launch per tick."""
+    """280,000 neurons forced into 4096-neuron blocks of 1024 work-items, one workgroup per CU (the
+    executor would take 2048); at in-degree 1000 a (source, block) segment holds 14.6 targets on
+    average, so about 40% exceed a slot's 15 inline targets and are read from the row table.  100
+    ticks: the persistent launch equals the oracle and one launch per tick."""
     print("case: persistent 280k x 1000 in 4096-neuron blocks, 100 ticks", flush=True)
     doc = models.cuba_network(280_000, indegree=1000, delay_ticks=1, steps=100, weight_scale=0.0116)
     expected = oracle.run(doc, lift_recording_budget=True)
     assert expected.synaptic_events > 1_000_000
-    plan = engine.lower(doc)
-    assert plan.shape.block == 4096 and plan.shape.wg == 1024 and plan.total_blocks == 69
-    dump, events, result = run(doc, "persistent", monkeypatch, lift_recording_budget=True)
+    shape = engine.Shape(4096, 1024, 2, 11)
+    monkeypatch.setenv("ATLAS_HIP_PERSISTENT", "1")
+    with HipExecutor(doc, device=0, shape=shape, lift_recording_budget=True) as ex:
+        assert ex.plan.shape == shape and ex.plan.total_blocks == 69
+        result = ex.run()
+        assert result["hip_runtime"]["launch_mode"] == "persistent"
+        dump, events = write_results(ex.document, result), write_events(ex.document, result)
     assert dump == expected.results and events == expected.events
     tick_dump, tick_events, _ = run(doc, "per-tick", monkeypatch, lift_recording_budget=True)
     assert tick_dump == dump and tick_events == events
@@ -280,6 +285,52 @@ def test_split_loop_of_several_groups_and_populations_equals_the_oracle(monkeypa
     monkeypatch.setattr(engine, "PERSISTENT_TICKS", 37)
     dump, events, _ = run(doc, "persistent", monkeypatch, lift_recording_budget=True)
     assert dump == expected.results and events == expected.events
+
+
+W = 0.1e-3   # V per event
+SPLIT_GRAPHS = {   # population sizes, (source, target, delay, in-degree, weight), populations reset after the deliveries
+    "three groups": ([700], [(0, 0, 1, 20, W), (0, 0, 5, 20, -W), (0, 0, 2, 20, W)], ()),
+    "three groups, late reset": ([700], [(0, 0, 5, 20, W), (0, 0, 1, 20, -W), (0, 0, 2, 20, W)], (0,)),
+    "five groups of 512-neuron blocks": ([9001], [(0, 0, d, 10, W * s) for d, s in zip((3, 1, 2, 1, 7), (1, -1, 1, 1, -1))], ()),
+    "two populations reading each other": ([600, 900], [(0, 1, 2, 20, W), (1, 0, 5, 20, -W), (0, 0, 1, 20, W)], ()),
+    "chain of three": ([300, 700, 513], [(0, 1, 1, 20, W), (1, 2, 4, 20, W)], ()),
+    "cycle of three": ([300, 700, 513], [(0, 1, 1, 20, W), (1, 2, 4, 20, W), (2, 0, 6, 20, -W)], ()),
+    "delay 0 beside others": ([300, 700], [(0, 1, 0, 20, W), (1, 0, 3, 20, -W), (1, 1, 0, 20, W)], ()),
+    "delay 0 into a chain": ([300, 700, 513], [(0, 1, 0, 20, W), (1, 2, 0, 20, W), (0, 2, 7, 20, -W)], ()),
+    "late reset of a population that others read": ([300, 700, 513], [(0, 1, 2, 20, W), (1, 1, 1, 20, -W), (1, 2, 3, 20, W)],
+                                                    (1,)),
+    "four coupled populations": ([300] * 4, [(i, j, 1 + (i + 2 * j) % 5, 10, W) for i in range(4) for j in range(4)], (2,))}
+
+
+@pytest.mark.parametrize("name", SPLIT_GRAPHS)
+def test_split_loop_over_population_graphs_equals_the_oracle(monkeypatch, name):
+    """Populations that read each other, chains, cycles, three and more groups, delay 0 beside longer ones
+    and resets after the deliveries in read populations, 700 ticks: the split loop equals the oracle in one
+    launch and in launches of 37 ticks."""
+    counts, paths, late = SPLIT_GRAPHS[name]
+    print(f"case: split loop, {name}", flush=True)
+    doc = nets.population_graph(counts, paths, steps=700, late=late)
+    expected = oracle.run(doc, lift_recording_budget=True)
+    assert expected.spike_count > sum(counts) // 2
+    for ticks in (engine.PERSISTENT_TICKS, 37):
+        monkeypatch.setattr(engine, "PERSISTENT_TICKS", ticks)
+        dump, events, result = run(doc, "persistent", monkeypatch, lift_recording_budget=True)
+        assert result["hip_runtime"]["launches"] == -(-700 // min(700, ticks))
+        assert dump == expected.results and events == expected.events
+
+
+def test_counters_past_the_lds_keep_one_launch_per_tick(monkeypatch):
+    """600,000 neurons in six groups, whose counters pass the split loop's LDS: accepted, one launch per
+    tick, equal to the oracle."""
+    print("case: 600k neurons in six groups, 40 ticks", flush=True)
+    doc = nets.population_graph([600_000], [(0, 0, 1 + k % 2, 2, W) for k in range(6)], steps=40)
+    expected = oracle.run(doc, lift_recording_budget=True)
+    assert expected.spike_count > 1000
+    monkeypatch.setenv("ATLAS_HIP_PERSISTENT", "1")
+    with HipExecutor(doc, device=0, lift_recording_budget=True) as ex:
+        result = ex.run()
+        assert result["hip_runtime"]["launch_mode"] == "per-tick"
+        assert write_results(ex.document, result) == expected.results
 
 
 @pytest.mark.parametrize("n,p,delay", [(64, 0.3, 0), (65, 0.3, 0), (1000, 0.05, 1), (2500, 0.03, 0)])
