@@ -2646,27 +2646,30 @@ def _split_lds(shape: Shape, xwaves: int, pathways: int) -> int:
 
 # Groups up to which a plan runs the split loop: its kernel holds every population's code over all of its
 # groups, and compiles in more time than the per-tick kernels'.  Seconds of compilation, split loop /
-# per tick, and us per tick: two groups 0.47 / 0.36, 3.1 / 7.4; one Poisson group into a population 0.38 /
-# 0.27, 2.2 / 6.2; four 0.75 / 0.58, 5.9 / 12.3; twelve 2.0 / 1.25, 17.3 / 34.6; four populations in 16
-# groups 2.9 / 1.7, 5.6 / 14.6, five in 25 4.7 / 2.6, 6.8 / 17.0, six in 36 7.1 / 3.6, 8.1 / 19.4: 25,000 ticks make
-# up for it with two groups, 130,000 with 16, 310,000 with 36.
+# per tick, and us per tick: two groups 0.45 / 0.36, 3.0 / 7.4; one Poisson group into a population 0.37 /
+# 0.27, 2.2 / 6.2; four 0.73 / 0.56, 5.9 / 12.3; twelve 2.0 / 1.25, 16.9 / 34.7; four populations in 16
+# groups 2.8 / 1.7, 5.6 / 14.4, five in 25 4.7 / 2.5, 6.8 / 17.0, six in 36 7.1 / 3.5, 8.1 / 19.4: 20,000 ticks make
+# up for it with two groups, 130,000 with 16, 320,000 with 36.
 SPLIT_GROUPS = 16
+
+
+# Source blocks a single reading wave (256 work-items) takes where the plan has several groups or
+# populations: at high rates that wave lists every spike and bounds the tick, and past this line the
+# slowest networks found ran behind one launch per tick.  us per tick in blocks of 256, of 512 and with
+# one launch per tick: four groups at 120 Hz, 11,000 neurons 12.8 / 7.9 / 13.3, 12,288 13.4 / 8.0 / 13.3, 16,000
+# 16.0 / 10.0 / 13.6; Poisson inputs of 300 Hz, 11,000 7.3 / 4.4 / 8.0, 12,288 8.1 / 4.5 / 7.9, 16,000 10.0 / 5.2 /
+# 8.4.  At ordinary rates the larger blocks cost a little: voltage jumps of 11,000 neurons 3.2 / 3.5 / 8.8,
+# two groups of 16,000 at 20 Hz 3.3 / 3.5 / 7.7.
+SINGLE_WAVE_BLOCKS = 46
 
 
 def _fits_split(plan: Plan, groups: list, shape: Shape) -> bool:
     """Whether the split loop takes the plan in this shape: two halves of waves, every workgroup on a
     CU of its own, at most 64 source blocks per exchange wave (the first one only publishes), one fired
-    mask per lane of that wave, and LDS for the counters (edge buckets take what is left of it).
-
-    Where a single wave reads (256 work-items) and the plan has several groups or populations, it takes
-    at most 32 source blocks: at high rates that wave lists every spike and bounds the tick.  us per tick
-    in blocks of 256, of 512 and with one launch per tick: 16,000 neurons firing at 120 Hz in four groups
-    16.1 / 10.1 / 13.6, in two 8.5 / 5.2 / 8.1, at 20 Hz 3.4 / 3.7 / 7.7; 16,000 Poisson inputs of 300 Hz 10.1 /
-    5.1 / 8.3, of 30 Hz 1.9 / 2.0 / 5.3; 8192 neurons at 120 Hz in four groups 10.2 / 7.6 / 12.9, at 20 Hz in two
-    3.0 / 3.4 / 7.4."""
+    mask per lane of that wave, and LDS for the counters (edge buckets take what is left of it)."""
     xwaves = SPLIT_XWAVES or shape.wg // 128
     blocks = [-(-pop.count // shape.block) for pop in plan.populations]
-    records = 32 if xwaves <= 2 and max(len(groups), len(plan.populations)) > 1 else 64
+    records = SINGLE_WAVE_BLOCKS if xwaves <= 2 and max(len(groups), len(plan.populations)) > 1 else 64
     return (1 <= xwaves < shape.wg // 64 and sum(blocks) <= CUS
             and all(blocks[g[0].source] <= records * max(1, xwaves - 1) for g in groups)
             and -(-shape.block // (shape.wg - 64 * xwaves)) * (shape.wg // 64 - xwaves) <= 64

@@ -846,11 +846,11 @@ def test_fitted_plans_of_several_groups_run_the_split_loop(doc, rings, readers):
 
 
 @pytest.mark.parametrize("counts,paths,block", [
-    ([8192], [(0, 0, 1), (0, 0, 2)], 256), ([8193], [(0, 0, 1), (0, 0, 2)], 512), ([16_384], [(0, 0, 1)], 256),
-    ([8193, 300], [(0, 1, 1)], 512), ([300, 8193], [(0, 1, 1)], 256), ([49_153], [(0, 0, 1), (0, 0, 2)], 512)])
-def test_several_groups_give_a_single_reading_wave_32_blocks(counts, paths, block):
-    """With several groups or populations, the one exchange wave of 256-neuron blocks reads at most 32 source
-    blocks (64 with one group of one population); larger blocks have several."""
+    ([11_776], [(0, 0, 1), (0, 0, 2)], 256), ([11_777], [(0, 0, 1), (0, 0, 2)], 512), ([16_384], [(0, 0, 1)], 256),
+    ([11_777, 300], [(0, 1, 1)], 512), ([300, 11_777], [(0, 1, 1)], 256), ([98_304], [(0, 0, 1), (0, 0, 2)], 512)])
+def test_several_groups_give_a_single_reading_wave_fewer_blocks(counts, paths, block):
+    """With several groups or populations, the one exchange wave of 256-neuron blocks reads at most 46 source
+    blocks (64 with one group of one population); larger blocks have several such waves."""
     plan = engine.lower(nets.population_graph(counts, [(*path, 2, 1e-5) for path in paths]), verify_envelope=False)
     engine.fit_shape(plan)
     assert plan.fitted and plan.shape.block == block
