@@ -2655,7 +2655,7 @@ SPLIT_GROUPS = 16
 
 # Source blocks a single reading wave (256 work-items) takes where the plan has several groups or
 # populations: at high rates that wave lists every spike and bounds the tick, and past this line the
-# slowest networks found ran behind one launch per tick.  us per tick in blocks of 256, of 512 and with
+# fastest-firing networks tried ran behind one launch per tick.  us per tick in blocks of 256, of 512 and with
 # one launch per tick: four groups at 120 Hz, 11,000 neurons 12.8 / 7.9 / 13.3, 12,288 13.4 / 8.0 / 13.3, 16,000
 # 16.0 / 10.0 / 13.6; Poisson inputs of 300 Hz, 11,000 7.3 / 4.4 / 8.0, 12,288 8.1 / 4.5 / 7.9, 16,000 10.0 / 5.2 /
 # 8.4.  At ordinary rates the larger blocks cost a little: voltage jumps of 11,000 neurons 3.2 / 3.5 / 8.8,
